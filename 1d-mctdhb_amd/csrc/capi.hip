@@ -221,7 +221,10 @@ extern "C" int mctdhb_density_dev(mctdhb_space* sp, const void* coef, void* rho1
         set_error("unknown precision mode");
         return kInvalidArgument;
     }
-    if (!sp->dm_work) MCTDHB_HIP_CHECK(hipMalloc(&sp->dm_work, dm_workspace_bytes(sp->S)));
+    if (!sp->dm_work) {
+        const int rc = dm_workspace_create(sp->S, &sp->dm_work);
+        if (rc) return rc;
+    }
     return density_matrices(sp->S, coef, (double2*) rho1, (double2*) rho2, prec,
                             prec == kDmMixed ? (int) kIndexOnTheFly : index, sp->dm_work, (hipStream_t) stream);
 }
@@ -540,7 +543,10 @@ extern "C" int mctdhb_density_sync_dev(mctdhb_space* sp, const void* coef, void*
         set_error("unknown precision mode");
         return kInvalidArgument;
     }
-    if (!sp->dm_work) MCTDHB_HIP_CHECK(hipMalloc(&sp->dm_work, dm_workspace_bytes(sp->S)));
+    if (!sp->dm_work) {
+        const int rc = dm_workspace_create(sp->S, &sp->dm_work);
+        if (rc) return rc;
+    }
     const DmSync sy{(double2*) rinv, (double*) eigvals, reg_factor};
     return density_matrices(sp->S, coef, (double2*) rho1, (double2*) rho2, prec, kIndexOnTheFly, sp->dm_work,
                             (hipStream_t) stream, &sy);
@@ -623,7 +629,10 @@ extern "C" int mctdhb_step_graph_create(mctdhb_space* sp, mctdhb_sil* s, mctdhb_
     }
     // Everything the step allocates or tunes on first use is done here, so
     // the capture below records kernels and device copies only.
-    if (!sp->dm_work) MCTDHB_HIP_CHECK(hipMalloc(&sp->dm_work, dm_workspace_bytes(sp->S)));
+    if (!sp->dm_work) {
+        const int rc = dm_workspace_create(sp->S, &sp->dm_work);
+        if (rc) return rc;
+    }
     if (s->L->prec == kPrecMixed) {
         const int rc = hc_tune_tiling(sp->S, nullptr);
         if (rc) return rc;
@@ -711,8 +720,7 @@ static const char* pack_refusal(const mctdhb_space* sp, const mctdhb_sil* s, con
     if (S->norb < 2 || S->norb > 7 || w->eq.norb != S->norb) return "packed steps cover 2 <= norb <= 7";
     if (L->prec != kPrecFP64 || L->generic || !L->small || !sil_small_fits(S, L->lm))
         return "packed steps take the one-workgroup FP64 SIL step";
-    const DmPlan plan = dm_plan(S, kDmFP64, kIndexOnTheFly);
-    if (plan.wave || plan.nb > kDmFinishBlocks || !dm_family_smem(S, sizeof(double)))
+    if (dm_plan(S).nb > kDmFinishBlocks || !dm_pair_smem(S))
         return "packed steps take the one-block density finish";
     return nullptr;
 }
@@ -758,7 +766,7 @@ static int pack_enqueue(const PackGroup& g, PkFft* fft, PkOm* om, PkNlCoef* nlc,
     if (!rc) rc = pk_hc_coefficients(cf, g.count, g.M, st);
     if (!rc) rc = pk_sil_small(sil, g.count, g.M, g.index, g.stage, g.sil_smem, st);
     if (!rc) rc = pk_density(dm, g.count, g.M, g.dm_grid, g.dm_smem, st);
-    if (!rc) rc = pk_dm_finish(fin, g.count, g.M, sizeof(double2) * 4 * g.M * g.M, st);
+    if (!rc) rc = pk_dm_finish(fin, g.count, g.M, st);
     return rc;
 }
 
@@ -842,7 +850,7 @@ extern "C" int mctdhb_pack_create(int n, mctdhb_space* const* spaces, mctdhb_sil
             const Sil* L = sils[i]->L;
             const OrbWork* w = orbitals[i]->w;
             const OrbEq& q = w->eq;
-            if (!sp->dm_work && hipMalloc(&sp->dm_work, dm_workspace_bytes(S)) != hipSuccess) {
+            if (!sp->dm_work && dm_workspace_create(S, &sp->dm_work)) {
                 set_error("hipMalloc of the density workspace failed");
                 mctdhb_pack_destroy(p);
                 return kOutOfMemory;
@@ -875,15 +883,15 @@ extern "C" int mctdhb_pack_create(int n, mctdhb_space* const* spaces, mctdhb_sil
                                             S->d_strideot, S->d_stridett, S->d_occ8);
             sil[j] = PkSil{ctx, L->cf64, S->d_W, S->ldw, a};
             g.sil_smem = std::max(g.sil_smem, sil_small_smem(S) + (g.stage ? sil_small_stage_bytes(S) : 0));
-            const DmPlan plan = dm_plan(S, kDmFP64, kIndexOnTheFly);
-            const unsigned grid = pk_density_grid(S->norb, plan.nb);
-            double2* part = (double2*) sp->dm_work;
-            dm[j] = PkDm{ctx, c, S->d_W, part, S->ldw, S->npar + 3 <= 2048 ? 1 : 0, plan.nb, grid};
-            g.dm_grid = std::max(g.dm_grid, grid);
-            g.dm_smem = std::max(g.dm_smem, dm_family_smem(S, sizeof(double)));
-            const int E = dm_num_elements(S->norb);
-            fin[j] = PkDmFin{part, part + (size_t) plan.nb * E, (double2*) rho1[i], (double2*) rho2[i],
-                             DmSync{(double2*) rinv[i], nullptr, g_reg_factor}, (int) plan.nb};
+            const unsigned nb = dm_plan(S).nb;
+            double2* part = dm_partials(S, sp->dm_work);
+            dm[j] = PkDm{low_ctx(S), c, S->d_W, part, S->ldw, dm_root_table(S) ? 1 : 0, nb};
+            g.dm_grid = std::max(g.dm_grid, nb);
+            g.dm_smem = std::max(g.dm_smem, dm_pair_smem(S));
+            fin[j] = PkDmFin{part,
+                             DmOut{c, (double2*) rho1[i], (double2*) rho2[i],
+                                   DmSync{(double2*) rinv[i], nullptr, g_reg_factor}},
+                             S->npar, (int) nb};
         }
         // one allocation, each table at a 256-byte boundary
         size_t off = 0;
@@ -2141,7 +2149,7 @@ extern "C" void integration_driver(MCTDHBDataStruct m, uint16_t rec_nsteps, char
         cmatrix_h2d(R.d->d_rinv, psi->inv_ob_denmat, M);
         const int lm = m->coef_workspace->lan_work->iter;
         if (mctdhb_sil_create(R.sp, lm, MCTDHB_FP64, MCTDHB_INDEX_FLY, &R.sil)) fail_stop("Lanczos workspace");
-        if (!R.sp->dm_work && hipMalloc(&R.sp->dm_work, dm_workspace_bytes(R.sp->S)) != hipSuccess)
+        if (!R.sp->dm_work && dm_workspace_create(R.sp->S, &R.sp->dm_work))
             fail_stop("density workspace");
     }
 

@@ -3,11 +3,12 @@
 // Replaces reference src/configurational/density_matrices.c:8-443
 // (set_onebody_dm, set_twobody_dm).  The reference runs one OpenMP
 // reduction over all configurations per unique element (~155 sweeps at
-// M = 5).  Here each element family is a block reduction over a tile of
-// configurations, every gather serves all the elements that share its jump
-// target, and a deterministic second stage sums the per-block partials.
+// M = 5).  For 2 <= M <= 7 both matrices come from one pass over the space of
+// N - 2 particles (density_impl.hpp); a deterministic second stage sums the
+// per-block partials and fills rho1 and rho2.
 //
-// Unique elements (e = layout index, see DmLayout):
+// Other orbital counts take the generic kernel, one element at a time over
+// the jump tables (e = layout index, see DmLayout):
 //   D1[k]    = sum |c|^2 n_k                        -> rho1[k][k]
 //   D2[k]    = sum |c|^2 n_k (n_k - 1)              -> rho2[kkkk]          (Rule 1)
 //   D3[k<s]  = sum |c|^2 n_k n_s                    -> rho2[ksks] & perms  (Rule 2)
@@ -21,20 +22,45 @@
 //   T8 (k<s; q<l) = sum conj(c_i) c[i-e_k-e_s+e_q+e_l] sqrt(n_k n_s (n_q+1)(n_l+1)) (Rule 8)
 // and the reference's symmetric fill assembles rho1 (M x M) and rho2 (M^4,
 // element k + sM + qM^2 + lM^3 = <a+_k a+_s a_q a_l>).
-//
-// The mixed form reads complex64 coefficients, multiplies in FP32 and sums
-// each thread's configurations with Kahan compensation; the block and grid
-// stages run in FP64.
 #include <algorithm>
 #include <vector>
 
 #include "density_impl.hpp"
-#include "mxm_wave.hpp"
-#include "pack.hpp"
+#include "orbital.hpp"
+#include "rowctx.hpp"
 
 namespace mctdhb {
 
-int dm_num_elements(int M) { return DmLayout{M}.total(); }
+constexpr int kDmBlock = 256;
+constexpr int kDmCPT = 16;  // configurations per thread per tile (generic kernel)
+constexpr int kDmTile = kDmBlock * kDmCPT;
+
+// ---------------------------------------------------------------- layout
+__host__ __device__ constexpr int c2(int m) { return m * (m - 1) / 2; }
+struct DmLayout {
+    int M;
+    __host__ __device__ constexpr int d1() const { return 0; }
+    __host__ __device__ constexpr int d2() const { return M; }
+    __host__ __device__ constexpr int d3() const { return 2 * M; }
+    __host__ __device__ constexpr int pair() const { return 2 * M + c2(M); }
+    __host__ __device__ constexpr int o3() const { return pair() + c2(M) * (M + 1); }
+    __host__ __device__ constexpr int o6() const { return o3() + c2(M); }
+    __host__ __device__ constexpr int t8() const { return o6() + M * c2(M - 1); }
+    __host__ __device__ constexpr int total() const { return t8() + c2(M) * c2(M > 2 ? M - 2 : 0); }
+    // lexicographic index of the pair a < b among 0..M-1
+    __host__ __device__ constexpr int pidx(int a, int b) const { return a * M - a * (a + 1) / 2 + (b - a - 1); }
+    // index of the pair q < l among the orbitals other than x (lexicographic)
+    __host__ __device__ constexpr int pidx_excl1(int x, int q, int l) const {
+        const int qq = q - (q > x), ll = l - (l > x);
+        const int m = M - 1;
+        return qq * m - qq * (qq + 1) / 2 + (ll - qq - 1);
+    }
+    __host__ __device__ constexpr int pidx_excl2(int x, int y, int q, int l) const {
+        const int qq = q - (q > x) - (q > y), ll = l - (l > x) - (l > y);
+        const int m = M - 2;
+        return qq * m - qq * (qq + 1) / 2 + (ll - qq - 1);
+    }
+};
 
 // -------------------------------------------------- generic (any M, FP64)
 // One block per (tile, element); the element is described at run time.
@@ -140,10 +166,10 @@ __global__ __launch_bounds__(kDmBlock) void k_density_generic(int M, RowCtx ctx,
     if (threadIdx.x == 0) part[(size_t) blockIdx.x * E + blockIdx.y] = make_double2(v[0], v[1]);
 }
 
-// -------------------------------------------------- second stage + fill
+// ------------------------------------- generic second stage and fill
 
-__global__ __launch_bounds__(256) void k_dm_reduce(const double2* __restrict__ part, int nblocks, int E,
-                                                   double2* __restrict__ tot) {
+__global__ __launch_bounds__(256) void k_generic_reduce(const double2* __restrict__ part, int nblocks, int E,
+                                                        double2* __restrict__ tot) {
     __shared__ double red[2 * 4];
     const int e = blockIdx.x;
     double v[2] = {0, 0};
@@ -242,138 +268,202 @@ __device__ __forceinline__ void dm_assemble_block(int M, const double2* __restri
     }
 }
 
-__global__ __launch_bounds__(256) void k_dm_assemble(int M, const double2* __restrict__ tot,
+__global__ __launch_bounds__(256) void k_generic_assemble(int M, const double2* __restrict__ tot,
                                                      double2* __restrict__ rho1, double2* __restrict__ rho2) {
     dm_assemble_block(M, tot, rho1, rho2);
 }
 
-// With fill set (few configuration blocks): the second-stage sums (each
-// element by one thread, over the blocks in order) and the fill; then, with
-// sy.rinv set, the density synchronisation of rho1, all in one block.
-__device__ __forceinline__ void dm_finish_block(double2* work, int M, const double2* __restrict__ part, int nblocks,
-                                                int E, double2* __restrict__ tot, double2* __restrict__ rho1,
-                                                double2* __restrict__ rho2, const DmSync& sy, int fill) {
-    if (fill) {
-        for (int e = threadIdx.x; e < E; e += blockDim.x) {
-            double2 v = make_double2(0, 0);
-            for (int b = 0; b < nblocks; b++) v = v + part[(size_t) b * E + e];
-            tot[e] = v;
-        }
-        __syncthreads();
-        dm_assemble_block(M, tot, rho1, rho2);
+// ------------------------------------------- second stage of the pair sums
+
+// Up to kDmFinishBlocks = 64 partials per element: one block sums them, a
+// wave per element (one load per lane), and fills.
+constexpr int kDmFinishThreads = 1024;
+constexpr size_t dm_finish_lds(int M) { return sizeof(double2) * (gram_elements(M) + 4 * M * M); }
+
+template <typename Z>
+__device__ __forceinline__ void dm_finish_block(double2* lds, int M, int npar, const double2* __restrict__ part,
+                                                int nb, const DmOut& out) {
+    const int E = gram_elements(M), lane = threadIdx.x & 63;
+    for (int e = threadIdx.x >> 6; e < E; e += blockDim.x >> 6) {
+        const double2 p = lane < nb ? part[(size_t) e * nb + lane] : make_double2(0, 0);
+        const double re = wave_sum(p.x), im = wave_sum(p.y);
+        if (lane == 0) lds[e] = make_double2(re, im);
     }
-    if (sy.rinv) {
-        __syncthreads();
-        density_sync_body(M, rho1, sy.rinv, sy.eig, sy.reg, work);
-    }
+    __syncthreads();
+    dm_fill_block<Z>(M, npar, lds, out, lds + E);
 }
 
-__global__ __launch_bounds__(256) void k_dm_finish(int M, const double2* __restrict__ part, int nblocks, int E,
-                                                   double2* __restrict__ tot, double2* __restrict__ rho1,
-                                                   double2* __restrict__ rho2, DmSync sy, int fill) {
-    extern __shared__ double2 work[];  // 4 M^2 for the synchronisation
-    dm_finish_block(work, M, part, nblocks, E, tot, rho1, rho2, sy, fill);
+template <typename Z>
+__global__ __launch_bounds__(kDmFinishThreads) void k_dm_finish(int M, int npar, const double2* __restrict__ part,
+                                                                int nb, DmOut out) {
+    extern __shared__ double2 lds[];
+    dm_finish_block<Z>(lds, M, npar, part, nb, out);
 }
 
-// Packed form: one block per instance, the fill and (with sy.rinv) the
-// synchronisation.
-__global__ __launch_bounds__(256) void k_dm_finish_pk(const PkDmFin* __restrict__ tab, int M, int E) {
-    extern __shared__ double2 work[];
+// Packed form: one block per instance.
+__global__ __launch_bounds__(kDmFinishThreads) void k_dm_finish_pk(const PkDmFin* __restrict__ tab, int M) {
+    extern __shared__ double2 lds[];
     const PkDmFin& a = tab[blockIdx.x];
-    dm_finish_block(work, M, a.part, a.nblocks, E, a.tot, a.rho1, a.rho2, a.sy, 1);
+    dm_finish_block<double2>(lds, M, a.npar, a.part, a.nb, a.out);
 }
 
-int pk_dm_finish(const PkDmFin* tab, int count, int M, size_t smem, hipStream_t st) {
-    k_dm_finish_pk<<<count, 256, smem, st>>>(tab, M, DmLayout{M}.total());
+// More partials: one block per element sums them, and the last block to
+// arrive fills.  Blocks count themselves in *arrive (a vector atomic); the
+// last one resets it.  Each block writes one element before it counts, so
+// the release it makes is cheap.
+template <typename Z>
+__global__ __launch_bounds__(256) void k_dm_reduce(int M, int npar, const double2* __restrict__ part, int nb,
+                                                   double2* tot, unsigned* arrive, DmOut out) {
+    extern __shared__ double2 lds[];
+    __shared__ double red[2 * 4];
+    __shared__ int last;
+    const int e = blockIdx.x;
+    double v[2] = {0, 0};
+    for (int b = threadIdx.x; b < nb; b += blockDim.x) {
+        const double2 p = part[(size_t) e * nb + b];
+        v[0] += p.x;
+        v[1] += p.y;
+    }
+    block_sum<2>(v, red);
+    if (threadIdx.x == 0) {
+        tot[e] = make_double2(v[0], v[1]);
+        __threadfence();
+        last = atomicAdd(arrive, 1u) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    if (threadIdx.x == 0) *arrive = 0;
+    for (int t = threadIdx.x; t < (int) gridDim.x; t += blockDim.x) lds[t] = tot[t];
+    __syncthreads();
+    dm_fill_block<Z>(M, npar, lds, out, lds + gridDim.x);
+}
+
+int pk_dm_finish(const PkDmFin* tab, int count, int M, hipStream_t st) {
+    k_dm_finish_pk<<<count, kDmFinishThreads, dm_finish_lds(M), st>>>(tab, M);
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
 }
 
-int pk_density(const PkDm* tab, int count, int M, unsigned max_grid, size_t smem, hipStream_t st) {
+// instantiated once each in dm_m<M>.hip
+extern template struct DmPairs<2>;
+extern template struct DmPairs<3>;
+extern template struct DmPairs<4>;
+extern template struct DmPairs<5>;
+extern template struct DmPairs<6>;
+extern template struct DmPairs<7>;
+
+int pk_density(const PkDm* tab, int count, int M, unsigned max_nb, size_t smem, hipStream_t st) {
     switch (M) {
-        case 2: return DmFused<2>::run_pk(tab, count, max_grid, smem, st);
-        case 3: return DmFused<3>::run_pk(tab, count, max_grid, smem, st);
-        case 4: return DmFused<4>::run_pk(tab, count, max_grid, smem, st);
-        case 5: return DmFused<5>::run_pk(tab, count, max_grid, smem, st);
-        case 6: return DmFused<6>::run_pk(tab, count, max_grid, smem, st);
-        case 7: return DmFused<7>::run_pk(tab, count, max_grid, smem, st);
+        case 2: return DmPairs<2>::run_pk(tab, count, max_nb, smem, st);
+        case 3: return DmPairs<3>::run_pk(tab, count, max_nb, smem, st);
+        case 4: return DmPairs<4>::run_pk(tab, count, max_nb, smem, st);
+        case 5: return DmPairs<5>::run_pk(tab, count, max_nb, smem, st);
+        case 6: return DmPairs<6>::run_pk(tab, count, max_nb, smem, st);
+        case 7: return DmPairs<7>::run_pk(tab, count, max_nb, smem, st);
         default: set_error("packed density kernels cover 2 <= norb <= 7"); return kInvalidArgument;
     }
 }
 
-unsigned pk_density_grid(int M, unsigned ntiles) {
-    switch (M) {
-        case 2: return dm_family_grid(ntiles, Passes<2>::count());
-        case 3: return dm_family_grid(ntiles, Passes<3>::count());
-        case 4: return dm_family_grid(ntiles, Passes<4>::count());
-        case 5: return dm_family_grid(ntiles, Passes<5>::count());
-        case 6: return dm_family_grid(ntiles, Passes<6>::count());
-        case 7: return dm_family_grid(ntiles, Passes<7>::count());
-        default: return 0;
-    }
-}
-
-size_t dm_family_smem(const Space* S, size_t rsz) {
-    const int M = S->norb;
-    // block sums (as k_density lays them out), the W table, the sqrt table
-    size_t smem = (size_t) 2 * (2 * M + c2(M) + 8 * 9 + 64) * (kDmBlock / 64) * sizeof(double);
-    smem += ((size_t) (M - 1) * S->ldw * 4 + 15) & ~(size_t) 15;
-    if (S->npar + 3 <= 2048) smem += rsz * (S->npar + 3);
-    return smem > 64 * 1024 ? 0 : smem;
-}
-
-// instantiated once each in dm_m<M>.hip
-extern template struct DmFused<2>;
-extern template struct DmFused<3>;
-extern template struct DmFused<4>;
-extern template struct DmFused<5>;
-extern template struct DmFused<6>;
-extern template struct DmFused<7>;
-
-static int dispatch_dm(const Space* S, const void* c, int prec, int index, double2* part, const DmPlan& plan,
+static int dispatch_dm(const Space* S, const void* c, int prec, double2* part, const DmPlan& plan, const DmOut& out,
                        hipStream_t st) {
     switch (S->norb) {
-        case 2: return DmFused<2>::run(S, c, prec, index, part, plan, st);
-        case 3: return DmFused<3>::run(S, c, prec, index, part, plan, st);
-        case 4: return DmFused<4>::run(S, c, prec, index, part, plan, st);
-        case 5: return DmFused<5>::run(S, c, prec, index, part, plan, st);
-        case 6: return DmFused<6>::run(S, c, prec, index, part, plan, st);
-        case 7: return DmFused<7>::run(S, c, prec, index, part, plan, st);
-        default: set_error("fused density kernels cover 2 <= norb <= 7"); return kInvalidArgument;
+        case 2: return DmPairs<2>::run(S, c, prec, part, plan, out, st);
+        case 3: return DmPairs<3>::run(S, c, prec, part, plan, out, st);
+        case 4: return DmPairs<4>::run(S, c, prec, part, plan, out, st);
+        case 5: return DmPairs<5>::run(S, c, prec, part, plan, out, st);
+        case 6: return DmPairs<6>::run(S, c, prec, part, plan, out, st);
+        case 7: return DmPairs<7>::run(S, c, prec, part, plan, out, st);
+        default: set_error("pair density kernels cover 2 <= norb <= 7"); return kInvalidArgument;
     }
 }
 
-static bool wave_fits(const Space* S, int prec, int index) {
-    switch (S->norb) {
-        case 2: return DmFused<2>::wave_fits(S, prec, index);
-        case 3: return DmFused<3>::wave_fits(S, prec, index);
-        case 4: return DmFused<4>::wave_fits(S, prec, index);
-        case 5: return DmFused<5>::wave_fits(S, prec, index);
-        case 6: return DmFused<6>::wave_fits(S, prec, index);
-        case 7: return DmFused<7>::wave_fits(S, prec, index);
-        default: return false;
-    }
+static bool dm_generic(int M) { return M == 1 || M > 7; }
+
+// Runs of configurations go to waves.  Up to 1024 configurations of N - 2
+// particles one block of 8 waves does it all and the separate finish (a
+// launch) is saved; then 64 per wave, so a middling space still reaches many
+// CUs; from 256 blocks on, one per CU (the LDS buffers of M >= 4 hold a CU
+// each), the runs get longer: 512 blocks took 0.169 ms against 0.161 at N=100,
+// M=5 and 0.187 against 0.176 at N=30, M=7.
+DmPlan dm_plan(const Space* S) {
+    if (dm_generic(S->norb)) return {div_up(S->dim, kDmTile)};
+    return {S->low_dim <= 1024 ? 1u : std::min(256u, div_up(S->low_dim, 64 * kDmWaves))};
 }
 
-DmPlan dm_plan(const Space* S, int prec, int index) {
+// The rank and root tables leave room for what the block sums need; at M = 3
+// this is what bounds N (7027).
+constexpr size_t kDmTableBytes = 64 * 1024 - 9280;
+
+bool dm_root_table(const Space* S) { return S->npar + 3 <= 2048; }
+
+size_t dm_pair_smem(const Space* S) {
     const int M = S->norb;
-    const bool generic = M == 1 || M > 7;
-    if (!generic && S->dim >= kDmWaveMinDim && wave_fits(S, prec, index)) {
-        // at most about 4096 blocks: enough waves to hide the gathers'
-        // latency, and a bounded set of partial sums
-        const int cpt = (int) std::min<uint32_t>(16, div_up(S->dim, (uint32_t) kDmBlock * 4096u));
-        return {true, cpt, (unsigned) div_up(S->dim, (uint32_t) cpt * kDmBlock)};
+    size_t tables = ((size_t) (M - 1) * S->ldw * 4 + 15) & ~(size_t) 15;
+    if (dm_root_table(S)) tables += (sizeof(double) * (S->npar + 3) + 15) & ~(size_t) 15;
+    if (tables > kDmTableBytes) return 0;
+    size_t loop = 0, sums = 0;
+    switch (M) {
+#define CASE(m) \
+    case m:                                                               \
+        loop = gram_loop_lds<m>();                                          \
+        sums = gram_sum_lds<m>() + sizeof(double2) * gram_elements(m);      \
+        break;
+        CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
+#undef CASE
+        default: return 0;
     }
-    return {false, kDmCPT, (unsigned) div_up(S->dim, kDmTile)};
+    return std::max(tables + loop, sums);
 }
 
-size_t dm_workspace_bytes(const Space* S) {
-    const size_t E = (size_t) DmLayout{S->norb}.total();
-    // the largest block count of any form
-    size_t nb = div_up(S->dim, kDmTile);
-    for (int prec = 0; prec < 2; prec++)
-        for (int index = 0; index < 2; index++) nb = std::max<size_t>(nb, dm_plan(S, prec, index).nb);
-    return (nb * E + E) * sizeof(double2) + sizeof(ElemDesc) * E + 256;
+// counter | totals | partials | element list (generic)
+struct DmWork {
+    unsigned* arrive;
+    double2* tot;
+    double2* part;
+    ElemDesc* elems;
+    size_t bytes;
+};
+static DmWork dm_work(const Space* S, void* base) {
+    const int M = S->norb;
+    const size_t nb = dm_plan(S).nb;
+    const size_t E = dm_generic(M) ? (size_t) DmLayout{M}.total() : (size_t) gram_elements(M);
+    char* p = (char*) base;
+    DmWork w;
+    w.arrive = (unsigned*) p;
+    w.tot = (double2*) (p + 256);
+    w.part = w.tot + E;
+    w.elems = (ElemDesc*) (w.part + nb * E);
+    w.bytes = 256 + sizeof(double2) * (nb + 1) * E + sizeof(ElemDesc) * E;
+    return w;
+}
+
+int dm_workspace_create(const Space* S, void** work) {
+    const size_t bytes = dm_work(S, nullptr).bytes;
+    MCTDHB_HIP_CHECK(hipMalloc(work, bytes));
+    MCTDHB_HIP_CHECK(hipMemset(*work, 0, 256));
+    MCTDHB_HIP_CHECK(hipStreamSynchronize(nullptr));  // cleared before any stream counts
+    return kOk;
+}
+
+double2* dm_partials(const Space* S, void* work) { return dm_work(S, work).part; }
+
+static int density_generic(const Space* S, const void* coef, double2* rho1, double2* rho2, const DmWork& w,
+                           const DmSync& sy, hipStream_t st) {
+    const int M = S->norb, E = DmLayout{M}.total();
+    const unsigned nb = dm_plan(S).nb;
+    std::vector<ElemDesc> el = element_list(M);
+    MCTDHB_HIP_CHECK(hipMemcpyAsync(w.elems, el.data(), sizeof(ElemDesc) * E, hipMemcpyHostToDevice, st));
+    RowCtx ctx = make_row_ctx(S->dim, S->npar, S->d_ht, S->d_map, S->d_mapot, S->d_maptt, S->d_strideot,
+                              S->d_stridett);
+    k_density_generic<<<dim3(nb, E), kDmBlock, 0, st>>>(M, ctx, (const double2*) coef, w.elems, E, w.part);
+    MCTDHB_HIP_CHECK(hipGetLastError());
+    // the host vector must outlive the async copy
+    MCTDHB_HIP_CHECK(hipStreamSynchronize(st));
+    k_generic_reduce<<<E, 256, 0, st>>>(w.part, (int) nb, E, w.tot);
+    k_generic_assemble<<<1, 256, 0, st>>>(M, w.tot, rho1, rho2);
+    MCTDHB_HIP_CHECK(hipGetLastError());
+    return sy.rinv ? density_sync_small(M, rho1, sy.rinv, sy.eig, sy.reg, st) : kOk;
 }
 
 int density_matrices(const Space* S, const void* coef, double2* rho1, double2* rho2, int prec, int index,
@@ -383,7 +473,7 @@ int density_matrices(const Space* S, const void* coef, double2* rho1, double2* r
         return kInvalidArgument;
     }
     const int M = S->norb;
-    const bool generic = M == 1 || M > 7;
+    const bool generic = dm_generic(M);
     if (prec == kDmMixed && generic) {
         set_error("mixed precision density matrices cover 2 <= norb <= 8");
         return kInvalidArgument;
@@ -392,40 +482,25 @@ int density_matrices(const Space* S, const void* coef, double2* rho1, double2* r
         set_error("this density-matrix form needs the jump tables; build the space with tables");
         return kNotBuilt;
     }
-    const int E = DmLayout{M}.total();
-    const DmPlan plan = dm_plan(S, prec, index);
-    const unsigned nb = plan.nb;
-    double2* part = (double2*) work;
-    double2* tot = part + (size_t) nb * E;
-    ElemDesc* elems = (ElemDesc*) (tot + E);
-    int rc = kOk;
-    if (generic) {
-        std::vector<ElemDesc> el = element_list(M);
-        MCTDHB_HIP_CHECK(hipMemcpyAsync(elems, el.data(), sizeof(ElemDesc) * E, hipMemcpyHostToDevice, st));
-        RowCtx ctx = make_row_ctx(S->dim, S->npar, S->d_ht, S->d_map, S->d_mapot, S->d_maptt, S->d_strideot,
-                                  S->d_stridett);
-        k_density_generic<<<dim3(nb, E), kDmBlock, 0, st>>>(M, ctx, (const double2*) coef, elems, E, part);
-        MCTDHB_HIP_CHECK(hipGetLastError());
-        // the host vector must outlive the async copy
-        MCTDHB_HIP_CHECK(hipStreamSynchronize(st));
-    } else {
-        rc = dispatch_dm(S, coef, prec, index, part, plan, st);
-    }
-    if (rc) return rc;
     const DmSync sy = sync ? *sync : DmSync{nullptr, nullptr, 0.0};
-    if (nb <= kDmFinishBlocks) {
-        k_dm_finish<<<1, 256, sy.rinv ? sizeof(double2) * 4 * M * M : 0, st>>>(M, part, (int) nb, E, tot, rho1, rho2,
-                                                                               sy, 1);
-        MCTDHB_HIP_CHECK(hipGetLastError());
-        return kOk;
+    const DmWork w = dm_work(S, work);
+    if (generic) return density_generic(S, coef, rho1, rho2, w, sy, st);
+    const DmPlan plan = dm_plan(S);
+    const DmOut out{coef, rho1, rho2, sy};
+    const int rc = dispatch_dm(S, coef, prec, w.part, plan, out, st);
+    if (rc || plan.nb == 1) return rc;
+    const int nb = (int) plan.nb, E = gram_elements(M);
+    const size_t smem = dm_finish_lds(M);
+    if (plan.nb <= kDmFinishBlocks) {
+        if (prec == kDmMixed) k_dm_finish<float2><<<1, kDmFinishThreads, smem, st>>>(M, S->npar, w.part, nb, out);
+        else k_dm_finish<double2><<<1, kDmFinishThreads, smem, st>>>(M, S->npar, w.part, nb, out);
+    } else {
+        if (prec == kDmMixed)
+            k_dm_reduce<float2><<<E, 256, smem, st>>>(M, S->npar, w.part, nb, w.tot, w.arrive, out);
+        else
+            k_dm_reduce<double2><<<E, 256, smem, st>>>(M, S->npar, w.part, nb, w.tot, w.arrive, out);
     }
-    k_dm_reduce<<<E, 256, 0, st>>>(part, (int) nb, E, tot);
-    k_dm_assemble<<<1, 256, 0, st>>>(M, tot, rho1, rho2);
     MCTDHB_HIP_CHECK(hipGetLastError());
-    if (sy.rinv) {
-        k_dm_finish<<<1, 256, sizeof(double2) * 4 * M * M, st>>>(M, nullptr, 0, 0, nullptr, rho1, nullptr, sy, 0);
-        MCTDHB_HIP_CHECK(hipGetLastError());
-    }
     return kOk;
 }
 

@@ -1,60 +1,65 @@
-// density.hpp - rho1 / rho2 block reductions over configurations.
+// density.hpp - rho1 / rho2 as sums over configurations.
 #pragma once
 
+#include "pairs.hpp"
 #include "space.hpp"
 
 namespace mctdhb {
 
 enum : int { kDmFP64 = 0, kDmMixed = 1 };
 
-// Scratch needed by density_matrices (per-block partials and totals).
-size_t dm_workspace_bytes(const Space* S);
-int dm_num_elements(int M);
-
-// rho1 (M x M row-major, rho1[k*M+l] = <a+_k a_l>) and, if rho2 is non-null,
-// rho2 (M^4, index k + sM + qM^2 + lM^3 = <a+_k a+_s a_q a_l>), complex128.
-// coef is complex128 (prec = kDmFP64) or complex64 (kDmMixed); index is
-// kIdxTables or kIdxFly.  work must hold dm_workspace_bytes(S).
-// Launch plan of the fused kernels: the one-pass wave form (tiles of
-// cpt x 256 configurations) for large spaces of M >= 6, else the
-// element-family passes (tiles of 16 x 256, one family per block); nb blocks
-// of partial sums either way.  Measured on MI355X: the wave form takes
-// 1.87 ms at N=30, M=7 against 3.7 for the passes, and the passes 0.66 ms at
-// N=100, M=5 against 1.19 (at M <= 5 the wave sums cost more than they save).
+// Launch plan of the pair kernel (2 <= M <= 7): nb blocks of kDmWaves waves.
 struct DmPlan {
-    bool wave;
-    int cpt;
     unsigned nb;
 };
-DmPlan dm_plan(const Space* S, int prec, int index);
-// Spaces from this many configurations and orbitals take the wave form.
-constexpr uint32_t kDmWaveMinDim = 1u << 16;
-constexpr int kDmWaveMinOrb = 6;
+constexpr int kDmWaves = 8;
+constexpr int kDmThreads = 64 * kDmWaves;
+DmPlan dm_plan(const Space* S);
 
-// Per-orbital-count fused kernels (dm_m<M>.hip): write per-block partials.
-struct PkDm;
-template <int M> struct DmFused {
-    static bool wave_fits(const Space* S, int prec, int index);
-    static int run(const Space* S, const void* c, int prec, int index, double2* part, const DmPlan& plan,
-                   hipStream_t st);
-    // FP64, on-the-fly indices, element-family form, count instances
-    // (pack.hpp); max_grid: the largest per-instance family grid
-    static int run_pk(const PkDm* tab, int count, unsigned max_grid, size_t smem, hipStream_t st);
-};
-// LDS of the element-family kernel (FP64 or mixed by rsz), or 0 where it
-// exceeds the 64 KiB budget.
-size_t dm_family_smem(const Space* S, size_t rsz);
+// Scratch of density_matrices (per-block partials, totals and the arrival
+// counter of the last stage): allocated and cleared by dm_workspace_create.
+int dm_workspace_create(const Space* S, void** work);
+// the partial sums in it
+double2* dm_partials(const Space* S, void* work);
 
-// With sync->rinv set, also the synchronisation of rho1 (eigenvalues into
-// sync->eig when set, regularisation by sync->reg, rinv = rho1^-1), as the
-// standalone density_sync_small does.
+// LDS bytes of the pair kernel, or 0 where its tables exceed the budget.
+size_t dm_pair_smem(const Space* S);
+// Whether square roots come from a table in LDS (N + 3 <= 2048).
+bool dm_root_table(const Space* S);
+inline LowCtx low_ctx(const Space* S) { return LowCtx{S->d_low, S->low_dim, S->dim, S->npar}; }
+
+// With rinv set, also the synchronisation of rho1 (eigenvalues into eig when
+// set, regularisation by reg, rinv = rho1^-1), as the standalone
+// density_sync_small does.
 struct DmSync {
     double2* rinv;
     double* eig;
     double reg;
 };
-// Up to this many configuration blocks, one block finishes the reduction.
-constexpr unsigned kDmFinishBlocks = 64;
+// Where the totals go.  c: the coefficients (N = 1 reads them directly).
+struct DmOut {
+    const void* c;
+    double2* rho1;
+    double2* rho2;  // may be null
+    DmSync sy;
+};
+
+// Per-orbital-count kernels (dm_m<M>.hip): per-block partials of the pair
+// sums, or with one block everything.
+struct PkDm;
+template <int M> struct DmPairs {
+    static int run(const Space* S, const void* c, int prec, double2* part, const DmPlan& plan, const DmOut& out,
+                   hipStream_t st);
+    // FP64 partials of count instances (pack.hpp); max_nb: their largest plan
+    static int run_pk(const PkDm* tab, int count, unsigned max_nb, size_t smem, hipStream_t st);
+};
+
+// rho1 (M x M row-major, rho1[k*M+l] = <a+_k a_l>) and, if rho2 is non-null,
+// rho2 (M^4, index k + sM + qM^2 + lM^3 = <a+_k a+_s a_q a_l>), complex128.
+// coef is complex128 (prec = kDmFP64) or complex64 (kDmMixed).  index is
+// kIdxTables or kIdxFly; it matters for norb = 1 and norb > 7, whose generic
+// kernel reads the jump tables.  work: from dm_workspace_create.
+constexpr unsigned kDmFinishBlocks = 64;  // up to this many partials one block finishes
 int density_matrices(const Space* S, const void* coef, double2* rho1, double2* rho2, int prec, int index,
                      void* work, hipStream_t st, const DmSync* sync = nullptr);
 

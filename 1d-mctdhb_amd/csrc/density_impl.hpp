@@ -1,539 +1,318 @@
-// density_impl.hpp - templates of the fused density-matrix kernel,
+// density_impl.hpp - the pair-sum kernel of the density matrices,
 // instantiated once per orbital count in dm_m<M>.hip.
+//
+// Gamma[a][b] = sum over n' of conj(phi_a(n')) phi_b(n') for the pairs
+// a <= b (pairs.hpp) holds all of rho2, and rho1 is its partial trace over
+// N - 1.  The sum is a product of the P x NC' matrix phi with its adjoint,
+// taken on the FP64 matrix cores: lane (g, c) of a wave holds phi of pair c
+// (and 16 + c for M >= 6) at the g-th of four configurations, which is the
+// operand layout of both factors.
+//
+// Why this form: forming every element from the N space takes a gather and a
+// product per jump (about 80 per configuration at M = 5, one sum per element
+// on the vector ALU); here it is P = 15 gathers, and the sums are matrix
+// work.  Measured on MI355X, whole call: N=100, M=5 in FP64 0.495 ms before,
+// 0.149 ms now; N=30, M=7 from complex64 coefficients 1.81 ms before, 0.155 ms
+// now.  What bounds it is the FP64 unit, which matrix and vector instructions
+// share (run together they add up, they do not overlap): 3 products of
+// 16 x 16 x 4 per four configurations (10 at M >= 6) are 0.083 and 0.087 ms at
+// those sizes, the addressing and scaling about a third of that again.  Hence
+// a lane forms its configuration's addresses once for all pairs; with one
+// pair per lane (every lane ranking for itself, no LDS) the same loop took
+// 0.205 ms at both sizes.
+//
+// Complex64 coefficients are widened when read: products and sums are FP64
+// in both forms.
 #pragma once
 
-#include <type_traits>
-#include <utility>
-
 #include "density.hpp"
+#include "mxm_wave.hpp"
 #include "pack.hpp"
-#include "rowctx.hpp"
 
 namespace mctdhb {
 
-constexpr int kDmBlock = 256;
-constexpr int kDmCPT = 16;  // configurations per thread per tile
-constexpr int kDmTile = kDmBlock * kDmCPT;
-
-// ---------------------------------------------------------------- layout
-__host__ __device__ constexpr int c2(int m) { return m * (m - 1) / 2; }
-struct DmLayout {
-    int M;
-    __host__ __device__ constexpr int d1() const { return 0; }
-    __host__ __device__ constexpr int d2() const { return M; }
-    __host__ __device__ constexpr int d3() const { return 2 * M; }
-    __host__ __device__ constexpr int pair() const { return 2 * M + c2(M); }
-    __host__ __device__ constexpr int o3() const { return pair() + c2(M) * (M + 1); }
-    __host__ __device__ constexpr int o6() const { return o3() + c2(M); }
-    __host__ __device__ constexpr int t8() const { return o6() + M * c2(M - 1); }
-    __host__ __device__ constexpr int total() const { return t8() + c2(M) * c2(M > 2 ? M - 2 : 0); }
-    // lexicographic index of the pair a < b among 0..M-1
-    __host__ __device__ constexpr int pidx(int a, int b) const { return a * M - a * (a + 1) / 2 + (b - a - 1); }
-    // index of the pair q < l among the orbitals other than x (lexicographic)
-    __host__ __device__ constexpr int pidx_excl1(int x, int q, int l) const {
-        const int qq = q - (q > x), ll = l - (l > x);
-        const int m = M - 1;
-        return qq * m - qq * (qq + 1) / 2 + (ll - qq - 1);
-    }
-    __host__ __device__ constexpr int pidx_excl2(int x, int y, int q, int l) const {
-        const int qq = q - (q > x) - (q > y), ll = l - (l > x) - (l > y);
-        const int m = M - 2;
-        return qq * m - qq * (qq + 1) / 2 + (ll - qq - 1);
-    }
-};
-
-// --------------------------------------------------------- accumulators
-template <typename R> struct Acc;
-template <> struct Acc<double> {
-    double2 s;
-    __device__ __forceinline__ void zero() { s = make_double2(0, 0); }
-    __device__ __forceinline__ void add(double2 t) { s = s + t; }
-    __device__ __forceinline__ void add_re(double t) { s.x += t; }
-    __device__ __forceinline__ double2 get() const { return s; }
-};
-// Kahan-compensated complex FP32 sum
-template <> struct Acc<float> {
-    float2 s, c;
-    __device__ __forceinline__ void zero() {
-        s = make_float2(0, 0);
-        c = make_float2(0, 0);
-    }
-    __device__ __forceinline__ static void k1(float& sum, float& comp, float t) {
-        const float y = t - comp;
-        const float u = sum + y;
-        comp = (u - sum) - y;
-        sum = u;
-    }
-    __device__ __forceinline__ void add(float2 t) {
-        k1(s.x, c.x, t.x);
-        k1(s.y, c.y, t.y);
-    }
-    __device__ __forceinline__ void add_re(float t) { k1(s.x, c.x, t); }
-    __device__ __forceinline__ double2 get() const {
-        return make_double2((double) s.x - (double) c.x, (double) s.y - (double) c.y);
-    }
-};
-
-// ------------------------------------------------------------- passes
-// kind 0: diagonal moments; 1: pairs (k, l in [a, b)); 2: same-orbital (k);
-// 3: different-orbital (k, s in [a, b)).
-struct PassDesc {
-    int kind, k, a, b;
-};
-template <int M> struct Passes {
-    static constexpr int kPairChunk = M <= 6 ? 8 : 3;
-    static constexpr bool kTTPerK = (M - 1) * c2(M > 2 ? M - 2 : 0) <= 32;
-    static constexpr int count() {
-        int n = 1;
-        for (int k = 0; k < M - 1; k++) n += (M - 1 - k + kPairChunk - 1) / kPairChunk;
-        n += M;
-        if (M >= 4) {
-            for (int k = 0; k < M - 1; k++) n += kTTPerK ? 1 : (M - 1 - k);
-        }
-        return n;
-    }
-    static constexpr PassDesc get(int p) {
-        if (p == 0) return {0, 0, 0, 0};
-        int n = 1;
-        for (int k = 0; k < M - 1; k++)
-            for (int a = k + 1; a < M; a += kPairChunk) {
-                if (n == p) return {1, k, a, (a + kPairChunk < M ? a + kPairChunk : M)};
-                n++;
-            }
-        for (int k = 0; k < M; k++) {
-            if (n == p) return {2, k, 0, 0};
-            n++;
-        }
-        for (int k = 0; k < M - 1; k++) {
-            if (kTTPerK) {
-                if (n == p) return {3, k, k + 1, M};
-                n++;
-            } else {
-                for (int s = k + 1; s < M; s++) {
-                    if (n == p) return {3, k, s, s + 1};
-                    n++;
-                }
-            }
-        }
-        return {-1, 0, 0, 0};
-    }
-    static constexpr int nacc(int p) {
-        const PassDesc d = get(p);
-        if (d.kind == 0) return 2 * M + c2(M);
-        if (d.kind == 1) return (d.b - d.a) * (M + 1);
-        if (d.kind == 2) return (M - 1 - d.k) + c2(M - 1);
-        if (d.kind == 3) return (d.b - d.a) * c2(M - 2);
-        return 0;
-    }
-};
-
-template <int M, typename R, int IDX, int P>
-__device__ __forceinline__ void run_pass(const RowCtx& ctx, const cplx<R>* __restrict__ c, uint32_t base,
-                                         const uint32_t* Wl, int ldw, const R* sql, double* red,
-                                         double2* __restrict__ part, uint32_t row) {
-    using Z = cplx<R>;
-    constexpr PassDesc d = Passes<M>::get(P);
-    constexpr int NA = Passes<M>::nacc(P) > 0 ? Passes<M>::nacc(P) : 1;
-    constexpr DmLayout L{M};
-    Acc<R> acc[NA];
-#pragma unroll
-    for (int t = 0; t < NA; t++) acc[t].zero();
-
-    for (int r = 0; r < kDmCPT; r++) {
-        const uint32_t i = base + threadIdx.x + r * kDmBlock;
-        if (i >= ctx.dim) break;
-        Cfg<M, R, IDX> x;
-        x.load(i, ctx, Wl, ldw, sql);
-        const int* n = x.n;
-        const Z ci = c[i];
-        if constexpr (d.kind == 0) {
-            const R w = ci.x * ci.x + ci.y * ci.y;
-#pragma unroll
-            for (int k = 0; k < M; k++) {
-                acc[k].add_re(w * (R) n[k]);
-                acc[M + k].add_re(w * (R) (n[k] * (n[k] - 1)));
-#pragma unroll
-                for (int s = k + 1; s < M; s++) acc[2 * M + L.pidx(k, s)].add_re(w * (R) (n[k] * n[s]));
-            }
-        } else if constexpr (d.kind == 1) {
-            constexpr int k = d.k;
-            if (n[k] >= 1) {
-#pragma unroll
-                for (int l = d.a; l < d.b; l++) {
-                    const Z cj = c[x.single(k, l)];
-                    const Z t = cscale(cconjmul(ci, cj), x.s0[k] * x.s1[l]);
-                    const int o = (l - d.a) * (M + 1);
-                    acc[o].add(t);
-#pragma unroll
-                    for (int m = 0; m < M; m++) acc[o + 1 + m].add(cscale(t, (R) n[m]));
-                }
-            }
-        } else if constexpr (d.kind == 2) {
-            constexpr int k = d.k;
-            if (n[k] >= 2) {
-                const R a = x.sm[k] * x.s0[k];
-#pragma unroll
-                for (int q = k + 1; q < M; q++) {
-                    const Z cj = c[x.same(k, q, q)];
-                    acc[q - k - 1].add(cscale(cconjmul(ci, cj), a * x.s1[q] * x.s2[q]));
-                }
-#pragma unroll
-                for (int q = 0; q < M; q++) {
-                    if (q == k) continue;
-#pragma unroll
-                    for (int l = q + 1; l < M; l++) {
-                        if (l == k) continue;
-                        const Z cj = c[x.same(k, q, l)];
-                        acc[(M - 1 - k) + L.pidx_excl1(k, q, l)].add(
-                            cscale(cconjmul(ci, cj), a * x.s1[q] * x.s1[l]));
-                    }
-                }
-            }
-        } else if constexpr (d.kind == 3) {
-            constexpr int k = d.k;
-#pragma unroll
-            for (int s = d.a; s < d.b; s++) {
-                if (n[k] >= 1 && n[s] >= 1) {
-                    const R a = x.s0[k] * x.s0[s];
-#pragma unroll
-                    for (int q = 0; q < M; q++) {
-                        if (q == k || q == s) continue;
-#pragma unroll
-                        for (int l = q + 1; l < M; l++) {
-                            if (l == k || l == s) continue;
-                            const Z cj = c[x.diff(k, s, q, l)];
-                            acc[(s - d.a) * c2(M - 2) + L.pidx_excl2(k, s, q, l)].add(
-                                cscale(cconjmul(ci, cj), a * x.s1[q] * x.s1[l]));
-                        }
-                    }
-                }
-            }
-        }
-    }
-    // block reduction, then one partial per element of this pass
-    double v[2 * NA];
-#pragma unroll
-    for (int t = 0; t < NA; t++) {
-        const double2 g = acc[t].get();
-        v[2 * t] = g.x;
-        v[2 * t + 1] = g.y;
-    }
-    block_sum<2 * NA>(v, red);
-    if (threadIdx.x == 0) {
-        const int E = L.total();
-        double2* out = part + (size_t) row * E;
-#pragma unroll
-        for (int t = 0; t < NA; t++) {
-            int e;
-            if constexpr (d.kind == 0) e = t;  // d1, d2, d3 are contiguous from 0
-            else if constexpr (d.kind == 1) {
-                const int l = d.a + t / (M + 1);
-                e = L.pair() + L.pidx(d.k, l) * (M + 1) + t % (M + 1);
-            } else if constexpr (d.kind == 2) {
-                if (t < M - 1 - d.k) e = L.o3() + L.pidx(d.k, d.k + 1 + t);
-                else e = L.o6() + d.k * c2(M - 1) + (t - (M - 1 - d.k));
-            } else {
-                const int s = d.a + t / c2(M - 2);
-                e = L.t8() + L.pidx(d.k, s) * c2(M - 2) + t % c2(M - 2);
-            }
-            out[e] = make_double2(v[2 * t], v[2 * t + 1]);
-        }
-    }
+// Gamma[a][b], a <= b, of the totals tot (row by row over the upper triangle).
+__device__ __forceinline__ double2 gamma_at(const double2* tot, int P, int a, int b) {
+    const bool up = a <= b;
+    const int i = up ? a : b, j = up ? b : a;
+    const double2 v = tot[i * P - i * (i - 1) / 2 + (j - i)];
+    return up ? v : make_double2(v.x, -v.y);
 }
 
-template <int M, typename R, int IDX, int... P>
-__device__ __forceinline__ void run_one(std::integer_sequence<int, P...>, int pass, const RowCtx& ctx,
-                                        const cplx<R>* __restrict__ c, uint32_t base, const uint32_t* Wl, int ldw,
-                                        const R* sql, double* red, double2* part, uint32_t row) {
-    ((P == pass ? run_pass<M, R, IDX, P>(ctx, c, base, Wl, ldw, sql, red, part, row) : (void) 0), ...);
-}
+__device__ __forceinline__ int pair_of(int M, int a, int b) { return a <= b ? pair_index(M, a, b) : pair_index(M, b, a); }
 
-// Block w of the (padded) grid of 8 R blocks runs (tile, family) pair
-// v = (w mod 8) R + w / 8, tile-major: XCD w mod 8 gets the contiguous range
-// [x R, (x + 1) R), so a tile's families are dispatched one after another on
-// one XCD and read its coefficients and occupation rows through that XCD's
-// L2 (dispatched family after family over the whole space, every family
-// streamed them from memory again: 3.2 GB per FP64 launch at N=100, M=5,
-// 0.35 GB now).  Returns false for the padding blocks.
-__device__ __forceinline__ bool dm_tile_family(uint32_t bid, uint32_t grid, uint32_t ntiles, uint32_t nfam,
-                                               uint32_t& tile, uint32_t& fam) {
-    const uint32_t R = grid / 8;
-    const uint32_t v = (bid % 8) * R + bid / 8;
-    if (v >= ntiles * nfam) return false;
-    tile = v / nfam;
-    fam = v % nfam;
-    return true;
-}
-inline unsigned dm_family_grid(unsigned ntiles, unsigned nfam) { return 8 * div_up((uint64_t) ntiles * nfam, 8); }
-
-template <int M, typename R, int IDX>
-__device__ __forceinline__ void density_block(unsigned char* smem, uint32_t bid, uint32_t grid, const RowCtx& ctx,
-                                              const cplx<R>* __restrict__ c, const uint32_t* __restrict__ Wg,
-                                              int ldw, int use_sq, double2* __restrict__ part, uint32_t ntiles) {
-    uint32_t tile, fam;
-    if (!dm_tile_family(bid, grid, ntiles, Passes<M>::count(), tile, fam)) return;  // before any barrier
-    constexpr int kRed = 2 * (2 * M + c2(M) + 8 * 9 + 64);  // >= 2 * max nacc
-    double* red = (double*) smem;
-    uint32_t* Wl = (uint32_t*) (smem + kRed * (kDmBlock / 64) * sizeof(double));
-    const int wsz = (M - 1) * ldw;
-    R* sql = (R*) ((unsigned char*) Wl + ((wsz * 4 + 15) & ~15));
-    if constexpr (IDX == kIdxFly) {
-        for (int t = threadIdx.x; t < wsz; t += blockDim.x) Wl[t] = Wg[t];
+// rho1 and rho2 from the pair sums (every entry written once), then with
+// sy.rinv set the synchronisation of rho1.  One block; tot is in LDS and
+// visible to it.  Wave 0 forms rho1, one element per lane, and inverts it in
+// its registers while the other waves write rho2; the eigenvalues, or a rho1
+// that may need regularisation, take the whole block (density_sync_body).
+// N = 1 has no pairs: rho1 = conj(c_k) c_l, rho2 = 0.
+template <typename Z>
+__device__ __forceinline__ void dm_fill_block(int M, int npar, const double2* tot, const DmOut& o, double2* work) {
+    const int M2 = M * M, P = M * (M + 1) / 2;
+    __shared__ int done;
+    if (threadIdx.x < 64) {
+        const int k = threadIdx.x >> 3, l = threadIdx.x & 7;
+        const bool in = k < M && l < M;
+        double2 v = make_double2(0, 0);
+        if (in && npar < 2) {
+            const Z* c = (const Z*) o.c;
+            v = cconjmul(to_d2(c[k]), to_d2(c[l]));
+        } else if (in) {
+            for (int s = 0; s < M; s++) v = v + gamma_at(tot, P, pair_of(M, k, s), pair_of(M, s, l));
+            v = cscale(v, 1.0 / (npar - 1));
+        }
+        if (in) o.rho1[k * M + l] = v;
+        bool ok = !o.sy.rinv;
+        if (o.sy.rinv && !o.sy.eig) {
+            if (k == l) v.y = 0;
+            ok = hpd_inverse_wave(M, v, o.sy.reg);
+            if (ok && in) o.sy.rinv[k * M + l] = v;
+        }
+        if (threadIdx.x == 0) done = ok;
+    } else if (o.rho2) {
+        for (int e = threadIdx.x - 64; e < M2 * M2; e += blockDim.x - 64) {
+            const int k = e % M, s = (e / M) % M, q = (e / M2) % M, l = e / (M2 * M);
+            o.rho2[e] = npar < 2 ? make_double2(0, 0) : gamma_at(tot, P, pair_of(M, k, s), pair_of(M, q, l));
+        }
     }
-    if (use_sq)
-        for (int t = threadIdx.x; t < ctx.npar + 3; t += blockDim.x) sql[t] = sqrt((R) t);
     __syncthreads();
-    run_one<M, R, IDX>(std::make_integer_sequence<int, Passes<M>::count()>{}, (int) fam, ctx, c, tile * kDmTile, Wl,
-                       ldw, use_sq ? sql : nullptr, red, part, tile);
+    if (!done) density_sync_body(M, o.rho1, o.sy.rinv, o.sy.eig, o.sy.reg, work);
 }
 
-template <int M, typename R, int IDX>
-__global__ __launch_bounds__(kDmBlock) void k_density(RowCtx ctx, const cplx<R>* __restrict__ c,
-                                                      const uint32_t* __restrict__ Wg, int ldw, int use_sq,
-                                                      double2* __restrict__ part, uint32_t ntiles) {
+// Accumulators of a wave: for M <= 5 one tile of 16 pairs, Re = S and
+// Im = Q - Q^T with Q = Xr Xi^T; for M >= 6 two tiles, Re of (0,0), (0,1),
+// (1,1), Q of (0,0) and (1,1), and Im of (0,1).
+template <int M> struct GramAcc {
+    static constexpr int T = pair_count(M) <= 16 ? 1 : 2;
+    static constexpr int N = T == 1 ? 2 : 6;
+    mat4 a[N];
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int t = 0; t < N; t++) a[t] = mat4{0, 0, 0, 0};
+    }
+    __device__ __forceinline__ void add(const double2 (&x)[T]) {
+        if constexpr (T == 1) {
+            a[0] = mma(x[0].x, x[0].x, a[0]);
+            a[1] = mma(x[0].x, x[0].y, a[1]);
+            a[0] = mma(x[0].y, x[0].y, a[0]);
+        } else {
+            a[0] = mma(x[0].x, x[0].x, a[0]);
+            a[1] = mma(x[0].x, x[1].x, a[1]);
+            a[2] = mma(x[1].x, x[1].x, a[2]);
+            a[3] = mma(x[0].x, x[0].y, a[3]);
+            a[4] = mma(x[1].x, x[1].y, a[4]);
+            a[5] = mma(x[0].x, x[1].y, a[5]);
+            a[0] = mma(x[0].y, x[0].y, a[0]);
+            a[1] = mma(x[0].y, x[1].y, a[1]);
+            a[2] = mma(x[1].y, x[1].y, a[2]);
+            a[5] = mma(-x[0].y, x[1].x, a[5]);
+        }
+    }
+};
+
+// A wave works on 64 configurations at a time for M <= 5 (a lane forms all
+// the pairs of its configuration) and on 32 for M >= 6 (lane i and lane
+// i + 32 share one and take half of the pairs each).  The values go through
+// the wave's own LDS buffer, row p the configurations of pair p, padded by
+// one so that the 16 rows a matrix operand reads start in different banks.
+template <int M> struct GramShape {
+    static constexpr int P = pair_count(M);
+    static constexpr int H = P <= 16 ? 1 : 2;
+    static constexpr int C = 64 / H;         // configurations per pass
+    static constexpr int S = (P + H - 1) / H;  // pairs per lane
+    static constexpr int LD = C + 1;
+    static constexpr size_t wave_bytes = sizeof(double2) * P * LD;
+};
+
+// Passes w0 .. w1, in a pipeline: while pass s is multiplied, the
+// coefficients of s + 1 and the rows of s + 2 are on their way.  Reads past
+// the end repeat the last row and count as zero.
+template <int M, bool LUT, typename Z>
+__device__ __forceinline__ void gram_loop(GramAcc<M>& acc, double2* __restrict__ buf, const LowCtx& low,
+                                          const Z* __restrict__ c, const uint32_t* __restrict__ Wl, int ldw,
+                                          const double* __restrict__ sql, uint32_t w0, uint32_t w1) {
+    using G = GramShape<M>;
+    constexpr int T = GramAcc<M>::T;
+    if (w0 >= w1) return;
+    const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+    const uint32_t mine = lane % G::C;
+    const bool second = G::H == 2 && lane >= G::C;
+    LowRow<M> x;
+    Z v[G::S];
+    uint32_t num[G::S];  // the numbers under the roots, 16 bits each
+    // slot t of this lane is pair t, or S + t in the second half (pair P - 1 again past the end)
+    auto gather = [&](uint64_t row) {
+        x.set(row, Wl, ldw, low.top);
+#pragma unroll
+        for (int t = 0; t < G::S; t++) {
+            constexpr int last = G::P - 1;
+            const int p0 = t, p1 = G::S + t < G::P ? G::S + t : last;
+            const int q0 = kPairTable<M>.q[p0], l0 = kPairTable<M>.l[p0];
+            const int q1 = kPairTable<M>.q[p1], l1 = kPairTable<M>.l[p1];
+            uint32_t j = x.from[q0] + x.to[l0];
+            uint32_t a = (x.n[q0] + 1) | (x.n[l0] + 1 + (q0 == l0)) << 16;
+            if (G::H == 2) {
+                const uint32_t j1 = x.from[q1] + x.to[l1];
+                const uint32_t a1 = (x.n[q1] + 1) | (x.n[l1] + 1 + (q1 == l1)) << 16;
+                j = second ? j1 : j;
+                a = second ? a1 : a;
+            }
+            num[t] = a;
+            v[t] = c[j];
+        }
+    };
+    auto fetch = [&](uint32_t s) { return low.rows[min(s * G::C + mine, low.dim - 1)]; };
+    uint64_t next = fetch(w0 + 1);
+    gather(fetch(w0));
+    for (uint32_t s = w0; s < w1; s++) {
+        const bool in = s * G::C + mine < low.dim;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();  // the previous pass has been read
+#pragma unroll
+        for (int t = 0; t < G::S; t++) {
+            const uint32_t a = num[t] & 0xffffu, b = num[t] >> 16;
+            const double f = LUT ? sql[a] * sql[b] : sqrt((double) a * (double) b);
+            const int p = second ? (G::S + t < G::P ? G::S + t : G::P - 1) : t;
+            buf[p * G::LD + mine] = cscale(to_d2(v[t]), in ? f : 0.0);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const uint64_t row = next;
+        next = fetch(s + 2);
+        gather(row);
+        // the loads stay on this side of the products (moved to where their
+        // values are used, they would be waited for at once)
+        asm volatile("" ::: "memory");
+#pragma unroll 4
+        for (int u = 0; u < G::C / 4; u++) {
+            double2 o[T];
+#pragma unroll
+            for (int t = 0; t < T; t++) o[t] = buf[min(t * 16 + col, G::P - 1) * G::LD + 4 * u + grp];
+            acc.add(o);
+        }
+    }
+}
+
+// Dynamic LDS: the tables and one buffer per wave in the loop; after it the
+// waves' values of one accumulator and the block sums of all of them.
+template <int M> constexpr size_t gram_loop_lds() { return kDmWaves * GramShape<M>::wave_bytes; }
+template <int M> constexpr size_t gram_sum_lds() { return sizeof(double) * 256 * (kDmWaves + GramAcc<M>::N); }
+constexpr int gram_elements(int M) { return pair_count(M) * (pair_count(M) + 1) / 2; }
+
+// Block bid of nb: sums its share of the N - 2 space and leaves
+// Gamma (upper triangle) in part[e * nb + bid].
+template <int M, typename Z>
+__device__ __forceinline__ void gram_block(unsigned char* smem, uint32_t bid, uint32_t nb, const LowCtx& low,
+                                           const Z* __restrict__ c, const uint32_t* __restrict__ Wg, int ldw,
+                                           int use_sq, double2* part) {
+    using G = GramShape<M>;
+    constexpr int P = G::P, T = GramAcc<M>::T;
+    uint32_t* Wl = (uint32_t*) smem;
+    const int wsz = (M - 1) * ldw;
+    double* sql = (double*) (smem + ((wsz * 4 + 15) & ~15));
+    for (int t = threadIdx.x; t < wsz; t += blockDim.x) Wl[t] = Wg[t];
+    if (use_sq)
+        for (int t = threadIdx.x; t < low.npar + 3; t += blockDim.x) sql[t] = sqrt((double) t);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, col = lane & 15, grp = lane >> 4;
+    size_t off = (wsz * 4 + 15) & ~(size_t) 15;
+    if (use_sq) off += (sizeof(double) * (low.npar + 3) + 15) & ~(size_t) 15;
+    double2* buf = (double2*) (smem + off + wid * G::wave_bytes);
+    GramAcc<M> acc;
+    acc.zero();
+    // passes of C configurations, a contiguous run of them per wave
+    const uint32_t nsub = (low.dim + G::C - 1) / G::C, nw = nb * kDmWaves;
+    const uint32_t per = (nsub + nw - 1) / nw, w0 = (bid * kDmWaves + wid) * per;
+    const uint32_t w1 = min(w0 + per, nsub);
+    if (use_sq) gram_loop<M, true>(acc, buf, low, c, Wl, ldw, sql, w0, w1);
+    else gram_loop<M, false>(acc, buf, low, c, Wl, ldw, sql, w0, w1);
+    // block sums in a fixed order
+    double* wave = (double*) smem;           // [kDmWaves][256]
+    double* sum = wave + 256 * kDmWaves;     // [accumulator][256]
+    for (int t = 0; t < GramAcc<M>::N; t++) {
+        __syncthreads();
+        mat4 v = acc.a[0];
+#pragma unroll
+        for (int j = 1; j < GramAcc<M>::N; j++)
+            if (j == t) v = acc.a[j];
+#pragma unroll
+        for (int i = 0; i < 4; i++) wave[wid * 256 + (4 * i + grp) * 16 + col] = v[i];
+        __syncthreads();
+        for (int e = threadIdx.x; e < 256; e += blockDim.x) {
+            double v = wave[e];
+#pragma unroll
+            for (int w = 1; w < kDmWaves; w++) v += wave[w * 256 + e];
+            sum[t * 256 + e] = v;
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < P * P; e += blockDim.x) {
+        const int a = e / P, b = e % P;
+        if (a > b) continue;
+        const int i = a & 15, j = b & 15;
+        double re, im;
+        if (T == 1 || b < 16) {
+            re = sum[i * 16 + j];
+            im = sum[(T == 1 ? 1 : 3) * 256 + i * 16 + j] - sum[(T == 1 ? 1 : 3) * 256 + j * 16 + i];
+        } else if (a < 16) {
+            re = sum[256 + i * 16 + j];
+            im = sum[5 * 256 + i * 16 + j];
+        } else {
+            re = sum[2 * 256 + i * 16 + j];
+            im = sum[4 * 256 + i * 16 + j] - sum[4 * 256 + j * 16 + i];
+        }
+        part[(size_t) (a * P - a * (a - 1) / 2 + (b - a)) * nb + bid] = make_double2(re, im);
+    }
+}
+
+// One block (nb = 1) also fills rho1 and rho2 and synchronises rho1: its sums
+// go to LDS behind those of the waves.
+template <int M, typename Z>
+__global__ __launch_bounds__(kDmThreads) void k_gram(LowCtx low, const Z* __restrict__ c,
+                                                     const uint32_t* __restrict__ Wg, int ldw, int use_sq,
+                                                     double2* part, DmOut out) {
     extern __shared__ __align__(16) unsigned char smem[];
-    density_block<M, R, IDX>(smem, blockIdx.x, gridDim.x, ctx, c, Wg, ldw, use_sq, part, ntiles);
+    double2* tot = (double2*) (smem + gram_sum_lds<M>());
+    const bool one = gridDim.x == 1;
+    gram_block<M, Z>(smem, xcd_block(blockIdx.x, gridDim.x), gridDim.x, low, c, Wg, ldw, use_sq, one ? tot : part);
+    if (one) {
+        __syncthreads();
+        dm_fill_block<Z>(M, low.npar, tot, out, (double2*) smem);
+    }
 }
 
-// Packed form: instance blockIdx.y over its own family grid; blocks past it
-// return.
-template <int M>
-__global__ __launch_bounds__(kDmBlock) void k_density_pk(const PkDm* __restrict__ tab) {
+// Packed form: instance blockIdx.y; blocks past its own count return.
+template <int M> __global__ __launch_bounds__(kDmThreads) void k_gram_pk(const PkDm* __restrict__ tab) {
     extern __shared__ __align__(16) unsigned char smem[];
     const PkDm& p = tab[blockIdx.y];
-    if (blockIdx.x >= p.grid) return;
-    density_block<M, double, kIdxFly>(smem, blockIdx.x, p.grid, p.ctx, (const double2*) p.c, p.W, p.ldw, p.use_sq,
-                                      p.part, p.ntiles);
-}
-
-// ------------------------------------------------ one-pass wave form
-// (M >= 6, where the element families are many: 17 at M = 6, 38 at M = 7.)
-// Every configuration is visited once: its 2M + C(M,2) diagonal moments and
-// its jump-target products are formed once each, and each element's values
-// are summed over the wave's 64 configurations right away (DPP row shifts
-// inside each 16-lane row, the four row totals through readlane, all in
-// FP64) into a per-wave accumulator in LDS.  Nothing per configuration is
-// recomputed per element family, and no per-thread accumulator array is
-// needed.  The mixed form forms the products in complex64 and sums in FP64.
-
-// Sum of v over the 64 lanes of the wave, returned in every lane; every lane
-// of the wave must be active.  The order of the additions is fixed.
-__device__ __forceinline__ double wave_total(double v) { return wave_sum(v); }
-
-// Per-wave accumulators, spread over the lanes: element e lives in lane
-// e % 64 of acc[e / 64], so adding a wave total costs a masked add and no
-// memory round trip.
-template <int E> struct WaveAcc {
-    static constexpr int NR = (E + 63) / 64;
-    double2 acc[NR];
-    int lane;
-    __device__ __forceinline__ void zero(int l) {
-        lane = l;
-#pragma unroll
-        for (int j = 0; j < NR; j++) acc[j] = make_double2(0, 0);
-    }
-    __device__ __forceinline__ void add(int e, double2 v) {
-        const double x = wave_total(v.x), y = wave_total(v.y);
-        if (lane == (e & 63)) acc[e >> 6] = acc[e >> 6] + make_double2(x, y);
-    }
-    __device__ __forceinline__ void add_re(int e, double v) {
-        const double x = wave_total(v);
-        if (lane == (e & 63)) acc[e >> 6].x += x;
-    }
-};
-
-template <int M, typename R, int IDX, typename WA>
-__device__ __forceinline__ void wave_config(const RowCtx& ctx, const cplx<R>* __restrict__ c, uint32_t i,
-                                            const uint32_t* Wl, int ldw, const R* sql, WA& wa) {
-    using Z = cplx<R>;
-    constexpr DmLayout L{M};
-    const bool valid = i < ctx.dim;
-    Cfg<M, R, IDX> x;
-    Z ci = mk<R>(0, 0);
-    if (valid) {
-        x.load(i, ctx, Wl, ldw, sql);
-        ci = c[i];
-    } else {
-#pragma unroll
-        for (int k = 0; k < M; k++) {  // an empty row: every term is zero
-            x.n[k] = 0;
-            x.sm[k] = x.s0[k] = x.s1[k] = x.s2[k] = R(0);
-        }
-    }
-    const int* n = x.n;
-    // diagonal moments (real)
-    {
-        const double w = (double) ci.x * ci.x + (double) ci.y * ci.y;
-#pragma unroll
-        for (int k = 0; k < M; k++) {
-            wa.add_re(L.d1() + k, w * n[k]);
-            wa.add_re(L.d2() + k, w * (double) (n[k] * (n[k] - 1)));
-#pragma unroll
-            for (int s = k + 1; s < M; s++) wa.add_re(L.d3() + L.pidx(k, s), w * (double) (n[k] * n[s]));
-        }
-    }
-    // one particle k -> l (k < l): the pair element and its n_m moments
-#pragma unroll
-    for (int k = 0; k < M - 1; k++) {
-#pragma unroll
-        for (int l = k + 1; l < M; l++) {
-            double2 t = make_double2(0, 0);
-            if (n[k] >= 1) {
-                const Z cj = c[x.single(k, l)];
-                t = to_d2(cscale(cconjmul(ci, cj), x.s0[k] * x.s1[l]));
-            }
-            const int o = L.pair() + L.pidx(k, l) * (M + 1);
-            wa.add(o, t);
-#pragma unroll
-            for (int m = 0; m < M; m++) wa.add(o + 1 + m, cscale(t, (double) n[m]));
-        }
-    }
-    // two particles out of orbital k
-#pragma unroll
-    for (int k = 0; k < M; k++) {
-        const bool ok = n[k] >= 2;
-        const R a = x.sm[k] * x.s0[k];
-#pragma unroll
-        for (int q = k + 1; q < M; q++) {
-            double2 t = make_double2(0, 0);
-            if (ok) t = to_d2(cscale(cconjmul(ci, c[x.same(k, q, q)]), a * x.s1[q] * x.s2[q]));
-            wa.add(L.o3() + L.pidx(k, q), t);
-        }
-#pragma unroll
-        for (int q = 0; q < M; q++) {
-            if (q == k) continue;
-#pragma unroll
-            for (int l = q + 1; l < M; l++) {
-                if (l == k) continue;
-                double2 t = make_double2(0, 0);
-                if (ok) t = to_d2(cscale(cconjmul(ci, c[x.same(k, q, l)]), a * x.s1[q] * x.s1[l]));
-                wa.add(L.o6() + k * c2(M - 1) + L.pidx_excl1(k, q, l), t);
-            }
-        }
-    }
-    // one particle out of each of k < s
-    if constexpr (M >= 4) {
-#pragma unroll
-        for (int k = 0; k < M - 1; k++) {
-#pragma unroll
-            for (int s = k + 1; s < M; s++) {
-                const bool ok = n[k] >= 1 && n[s] >= 1;
-                const R a = x.s0[k] * x.s0[s];
-#pragma unroll
-                for (int q = 0; q < M; q++) {
-                    if (q == k || q == s) continue;
-#pragma unroll
-                    for (int l = q + 1; l < M; l++) {
-                        if (l == k || l == s) continue;
-                        double2 t = make_double2(0, 0);
-                        if (ok) t = to_d2(cscale(cconjmul(ci, c[x.diff(k, s, q, l)]), a * x.s1[q] * x.s1[l]));
-                        wa.add(L.t8() + L.pidx(k, s) * c2(M - 2) + L.pidx_excl2(k, s, q, l), t);
-                    }
-                }
-            }
-        }
-    }
-}
-
-// One block of 256 threads takes tile b of `cpt` x 256 consecutive
-// configurations; its four per-wave accumulator sets are added in a fixed
-// order into part[b * E ...].
-template <int M, typename R, int IDX>
-__global__ __launch_bounds__(kDmBlock) void k_density_wave(RowCtx ctx, const cplx<R>* __restrict__ c,
-                                                           const uint32_t* __restrict__ Wg, int ldw, int cpt,
-                                                           double2* __restrict__ part) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    constexpr int E = DmLayout{M}.total();
-    constexpr int NW = kDmBlock / 64;
-    double2* acc = (double2*) smem;
-    uint32_t* Wl = (uint32_t*) (smem + sizeof(double2) * NW * E);
-    const int wsz = (M - 1) * ldw;
-    R* sql = (R*) ((unsigned char*) Wl + ((wsz * 4 + 15) & ~15));
-    if constexpr (IDX == kIdxFly) {
-        for (int t = threadIdx.x; t < wsz; t += blockDim.x) Wl[t] = Wg[t];
-    }
-    for (int t = threadIdx.x; t < ctx.npar + 3; t += blockDim.x) sql[t] = sqrt((R) t);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    WaveAcc<E> wa;
-    wa.zero(lane);
-    const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
-    const uint32_t base = b * (uint32_t) cpt * kDmBlock + threadIdx.x;
-    for (int r = 0; r < cpt; r++) wave_config<M, R, IDX>(ctx, c, base + r * kDmBlock, Wl, ldw, sql, wa);
-#pragma unroll
-    for (int j = 0; j < WaveAcc<E>::NR; j++)
-        if (j * 64 + lane < E) acc[wid * E + j * 64 + lane] = wa.acc[j];
-    __syncthreads();
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
-        double2 v = acc[e];
-#pragma unroll
-        for (int w = 1; w < NW; w++) v = v + acc[w * E + e];
-        part[(size_t) b * E + e] = v;
-    }
-}
-
-template <int M> static size_t dm_wave_smem(const Space* S, size_t rsz) {
-    return sizeof(double2) * (kDmBlock / 64) * DmLayout{M}.total() +
-           (((size_t) (M - 1) * S->ldw * 4 + 15) & ~(size_t) 15) + rsz * (S->npar + 3);
+    if (blockIdx.x >= p.nb) return;
+    gram_block<M, double2>(smem, xcd_block(blockIdx.x, p.nb), p.nb, p.low, p.c, p.W, p.ldw, p.use_sq, p.part);
 }
 
 template <int M>
-bool DmFused<M>::wave_fits(const Space* S, int prec, int index) {
-    const size_t rsz = prec == kDmMixed ? sizeof(float) : sizeof(double);
-    return M >= kDmWaveMinOrb && dm_wave_smem<M>(S, rsz) <= 64 * 1024;
-}
-
-template <int M>
-int DmFused<M>::run_pk(const PkDm* tab, int count, unsigned max_grid, size_t smem, hipStream_t st) {
-    k_density_pk<M><<<dim3(max_grid, count), kDmBlock, smem, st>>>(tab);
+int DmPairs<M>::run_pk(const PkDm* tab, int count, unsigned max_nb, size_t smem, hipStream_t st) {
+    k_gram_pk<M><<<dim3(max_nb, count), kDmThreads, smem, st>>>(tab);
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
 }
 
 template <int M>
-int DmFused<M>::run(const Space* S, const void* c, int prec, int index, double2* part, const DmPlan& plan,
+int DmPairs<M>::run(const Space* S, const void* c, int prec, double2* part, const DmPlan& plan, const DmOut& out,
                     hipStream_t st) {
-    const bool fly = prec == kDmMixed || index == kIdxFly;
-    const size_t rsz = prec == kDmMixed ? sizeof(float) : sizeof(double);
-    RowCtx ctx = make_row_ctx(S->dim, S->npar, S->d_ht, S->d_map, S->d_mapot, S->d_maptt, S->d_strideot,
-                              S->d_stridett, S->d_occ8);
-    if constexpr (M >= kDmWaveMinOrb) {
-    if (plan.wave) {
-        const size_t smem = dm_wave_smem<M>(S, rsz);
-        if (prec == kDmMixed)
-            k_density_wave<M, float, kIdxFly><<<plan.nb, kDmBlock, smem, st>>>(ctx, (const float2*) c, S->d_W, S->ldw,
-                                                                              plan.cpt, part);
-        else if (fly)
-            k_density_wave<M, double, kIdxFly><<<plan.nb, kDmBlock, smem, st>>>(ctx, (const double2*) c, S->d_W,
-                                                                               S->ldw, plan.cpt, part);
-        else
-            k_density_wave<M, double, kIdxTables><<<plan.nb, kDmBlock, smem, st>>>(ctx, (const double2*) c, S->d_W,
-                                                                                  S->ldw, plan.cpt, part);
-        MCTDHB_HIP_CHECK(hipGetLastError());
-        return kOk;
-    }
-    }
-    const unsigned nb = plan.nb;
-    const bool use_sq = S->npar + 3 <= 2048;
-    const size_t smem = dm_family_smem(S, rsz);
+    const size_t smem = dm_pair_smem(S);
     if (!smem) {
-        set_error("density kernel LDS budget exceeded for this (N, M); use table indexing");
+        set_error("density kernel LDS budget exceeded for this (N, M)");
         return kInvalidArgument;
     }
-    // One element family per block: every block's chain of dependent loads
-    // is one family long, and 14x more blocks (M = 5) are in flight than
-    // with every family in turn in one block; a tile's families run
-    // together on one XCD (dm_tile_family).
-    const unsigned grid = dm_family_grid(nb, Passes<M>::count());
+    const int use_sq = dm_root_table(S) ? 1 : 0;
     if (prec == kDmMixed)
-        k_density<M, float, kIdxFly><<<grid, kDmBlock, smem, st>>>(ctx, (const float2*) c, S->d_W, S->ldw, use_sq,
-                                                                   part, nb);
-    else if (fly)
-        k_density<M, double, kIdxFly><<<grid, kDmBlock, smem, st>>>(ctx, (const double2*) c, S->d_W, S->ldw,
-                                                                    use_sq, part, nb);
+        k_gram<M, float2><<<plan.nb, kDmThreads, smem, st>>>(low_ctx(S), (const float2*) c, S->d_W, S->ldw, use_sq,
+                                                             part, out);
     else
-        k_density<M, double, kIdxTables><<<grid, kDmBlock, smem, st>>>(ctx, (const double2*) c, S->d_W, S->ldw,
-                                                                       use_sq, part, nb);
+        k_gram<M, double2><<<plan.nb, kDmThreads, smem, st>>>(low_ctx(S), (const double2*) c, S->d_W, S->ldw, use_sq,
+                                                              part, out);
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
 }

@@ -1,6 +1,6 @@
-// dm_m2.hip - fused density-matrix kernel instantiated for M = 2 orbitals.
+// dm_m2.hip - pair-sum density kernel instantiated for M = 2 orbitals.
 #include "density_impl.hpp"
 
 namespace mctdhb {
-template struct DmFused<2>;
+template struct DmPairs<2>;
 }  // namespace mctdhb

@@ -1,6 +1,6 @@
-// dm_m3.hip - fused density-matrix kernel instantiated for M = 3 orbitals.
+// dm_m3.hip - pair-sum density kernel instantiated for M = 3 orbitals.
 #include "density_impl.hpp"
 
 namespace mctdhb {
-template struct DmFused<3>;
+template struct DmPairs<3>;
 }  // namespace mctdhb

@@ -1,6 +1,6 @@
-// dm_m4.hip - fused density-matrix kernel instantiated for M = 4 orbitals.
+// dm_m4.hip - pair-sum density kernel instantiated for M = 4 orbitals.
 #include "density_impl.hpp"
 
 namespace mctdhb {
-template struct DmFused<4>;
+template struct DmPairs<4>;
 }  // namespace mctdhb

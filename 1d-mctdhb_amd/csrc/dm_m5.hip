@@ -1,6 +1,6 @@
-// dm_m5.hip - fused density-matrix kernel instantiated for M = 5 orbitals.
+// dm_m5.hip - pair-sum density kernel instantiated for M = 5 orbitals.
 #include "density_impl.hpp"
 
 namespace mctdhb {
-template struct DmFused<5>;
+template struct DmPairs<5>;
 }  // namespace mctdhb

@@ -1,6 +1,6 @@
-// dm_m6.hip - fused density-matrix kernel instantiated for M = 6 orbitals.
+// dm_m6.hip - pair-sum density kernel instantiated for M = 6 orbitals.
 #include "density_impl.hpp"
 
 namespace mctdhb {
-template struct DmFused<6>;
+template struct DmPairs<6>;
 }  // namespace mctdhb

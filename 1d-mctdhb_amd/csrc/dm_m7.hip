@@ -1,6 +1,6 @@
-// dm_m7.hip - fused density-matrix kernel instantiated for M = 7 orbitals.
+// dm_m7.hip - pair-sum density kernel instantiated for M = 7 orbitals.
 #include "density_impl.hpp"
 
 namespace mctdhb {
-template struct DmFused<7>;
+template struct DmPairs<7>;
 }  // namespace mctdhb

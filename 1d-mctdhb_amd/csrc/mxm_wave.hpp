@@ -170,6 +170,37 @@ __device__ inline bool herm_posdef_wave(int n, double2* h) {
     return true;
 }
 
+// Inverse of a Hermitian positive definite M x M matrix (M <= 8) held one
+// element per lane, a[i][j] in lane 8 i + j, by in-place Gauss-Jordan sweeps
+// without pivoting (stable for such matrices; every pivot is a Cholesky
+// pivot).  False, with a spoiled, when a pivot is not positive or when
+// 1 / (|a|_F |a^-1|_F), a lower bound of lambda_min / lambda_max, does not
+// clear reg by more than the rounding of that ratio.  All 64 lanes of one
+// wave call it, with no barrier; the row and column of a pivot come by
+// shuffles.  (The block-wide elimination in LDS above, bound by its barriers
+// and one-lane row loops, with the fill before it cost the whole step of N=10,
+// M=4 6 us and that of N=18, M=6 16 us more.)
+__device__ __forceinline__ bool hpd_inverse_wave(int M, double2& a, double reg) {
+    const int lane = threadIdx.x & 63, i = lane >> 3, j = lane & 7;
+    const bool in = i < M && j < M;
+    if (!in) a = make_double2(i == j ? 1.0 : 0.0, 0.0);
+    const double na = wave_sum(in ? a.x * a.x + a.y * a.y : 0.0);
+    bool pd = true;
+    for (int k = 0; k < M; k++) {
+        const double piv = __shfl(a.x, 9 * k, 64);
+        const double2 aik = make_double2(__shfl(a.x, 8 * i + k, 64), __shfl(a.y, 8 * i + k, 64));
+        const double2 akj = make_double2(__shfl(a.x, 8 * k + j, 64), __shfl(a.y, 8 * k + j, 64));
+        pd = pd && piv > 0;
+        const double p = 1.0 / piv;
+        if (i == k && j == k) a = make_double2(p, 0.0);
+        else if (i == k) a = cscale(a, p);
+        else if (j == k) a = cscale(a, -p);
+        else a = a - cmul(aik, cscale(akj, p));
+    }
+    const double ni = wave_sum(in ? a.x * a.x + a.y * a.y : 0.0);
+    return pd && 1.0 / sqrt(na * ni) > reg + 1e-13;
+}
+
 // rho1 eigenvalues (synchronize.c:49), regularisation when the smallest
 // natural occupation is below reg_factor times the largest
 // (lapack_interface.c:126-163, synchronize.c:50-54), then the inverse from

@@ -87,25 +87,21 @@ struct PkSil {
     SmallSilArgs a;
 };
 
-// rho1/rho2 partial sums, one element family per block (grid: the
-// instance's own padded family grid).
+// Pair sums of the density matrices: nb blocks.
 struct PkDm {
-    RowCtx ctx;
+    LowCtx low;
     const double2* c;
     const uint32_t* W;
     double2* part;
     int ldw, use_sq;
-    uint32_t ntiles, grid;
+    uint32_t nb;
 };
 
 // Second-stage sums, fill and density synchronisation: one block.
 struct PkDmFin {
     const double2* part;
-    double2* tot;
-    double2* rho1;
-    double2* rho2;
-    DmSync sy;
-    int nblocks;
+    DmOut out;
+    int npar, nb;
 };
 
 // Stage launchers over count table entries (device pointers).  They check
@@ -120,11 +116,9 @@ bool pk_nl_folds(int M, int ns);
 int pk_gram_schmidt(const PkGs* tab, int count, int M, size_t smem, hipStream_t st);
 int pk_hc_coefficients(const PkCf* tab, int count, int M, hipStream_t st);
 int pk_sil_small(const PkSil* tab, int count, int M, int index, bool stage, size_t smem, hipStream_t st);
-int pk_density(const PkDm* tab, int count, int M, unsigned max_grid, size_t smem, hipStream_t st);
-// The family grid of an instance with ntiles configuration tiles (0: M not covered).
-unsigned pk_density_grid(int M, unsigned ntiles);
+int pk_density(const PkDm* tab, int count, int M, unsigned max_nb, size_t smem, hipStream_t st);
 // LDS of the Gram-Schmidt block: the staged orbitals, or 0 (not staged).
 size_t pk_gs_smem(int M, int n);
-int pk_dm_finish(const PkDmFin* tab, int count, int M, size_t smem, hipStream_t st);
+int pk_dm_finish(const PkDmFin* tab, int count, int M, hipStream_t st);
 
 }  // namespace mctdhb

@@ -12,6 +12,7 @@
 //        one chunk per occupied pair k < s in lexicographic order
 // Every entry is computed independently from the closed-form rank (fock.hpp),
 // one configuration per thread; strides come from a device prefix scan.
+#include "pairs.hpp"
 #include "space.hpp"
 
 #include <cstdlib>
@@ -181,6 +182,22 @@ __global__ void k_occ8(int M, uint32_t dim, const uint16_t* __restrict__ ht, uin
     uint32_t w[2] = {0, 0};
     for (int k = 0; k < M; k++) w[k >> 2] |= (uint32_t) ht[(size_t) i * M + k] << (8 * (k & 3));
     occ8[i] = make_uint2(w[0], w[1]);
+}
+
+// Prefix words of the N - 2 space (pairs.hpp), `bits` per field.
+__global__ void k_low_rows(int N2, int M, uint32_t dim, const uint32_t* __restrict__ W, int ldw, int bits,
+                           uint64_t* __restrict__ rows) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= dim) return;
+    uint32_t n[kMaxOrb];
+    unrank_rt(i, N2, M, dim, W, ldw, n);
+    uint64_t w = 0;
+    uint32_t P = 0;
+    for (int m = 0; m < M; m++) {
+        P += n[m];
+        w |= (uint64_t) P << (bits * m);
+    }
+    rows[i] = w;
 }
 
 // Pair slots.  Within a run (fixed P_1 .. P_{M-2}) the rank grows by one as
@@ -376,6 +393,17 @@ int space_create(int npar, int norb, int flags, Space** out) {
         k_occ8<<<div_up(dim, tb), tb, 0, st>>>(norb, dim, S->d_ht, (uint2*) S->d_occ8);
         MCTDHB_HIP_CHECK(hipGetLastError());
     }
+    if (norb >= 2 && norb <= 7 && npar >= 2) {
+        rc = space_dimension_exact(npar - 2, norb, &S->low_dim);
+        if (rc) {
+            space_destroy(S);
+            return rc;
+        }
+        ALLOC(S->d_low, sizeof(uint64_t) * (size_t) S->low_dim);
+        k_low_rows<<<div_up(S->low_dim, tb), tb, 0, st>>>(npar - 2, norb, S->low_dim, S->d_W, S->ldw, low_bits(norb),
+                                                          S->d_low);
+        MCTDHB_HIP_CHECK(hipGetLastError());
+    }
     if (norb >= 2) {
         rc = build_pair_slots(S, st);
         if (rc) {
@@ -403,6 +431,7 @@ void space_destroy(Space* S) {
     hipFree(S->d_slots);
     hipFree(S->d_pad);
     hipFree(S->d_occ8);
+    hipFree(S->d_low);
     delete S;
 }
 

@@ -37,6 +37,10 @@ struct Space {
     // one 8-byte load per configuration in the fused kernels
     uint8_t* d_occ8 = nullptr;
     uint32_t* d_slots = nullptr;
+    // the space of N - 2 particles (2 <= norb <= 7, N >= 2): prefix words
+    // (pairs.hpp) and size
+    uint64_t* d_low = nullptr;
+    uint32_t low_dim = 0;
     uint32_t n_pairs = 0, n_singles = 0;
     // complex64 staging with one zero element on each side (dim + 2), for
     // callers of the paired kernel whose vectors are not padded

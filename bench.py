@@ -868,7 +868,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "c64 H.C/rho (Kahan) + f64 Lanczos",
+        "dtype": "c64 H.C + f64 rho and Lanczos",
         "data": "synthetic (seeded complex-normal C, random Hermitian h scale 1, symmetrised g scale 0.1)",
         "config": {"workload": f"real-time SIL steps N={N} M={M} NC={nc} m={lm} dt={dt}",
                    "npar": N, "norb": M, "dim": nc, "lanczos_iter": lm, "dt": dt},

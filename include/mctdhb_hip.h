@@ -237,7 +237,7 @@ typedef struct mctdhb_sil   mctdhb_sil;   /* Krylov workspace of the SIL step */
 
 /* arithmetic forms */
 #define MCTDHB_FP64 0  /* complex128 throughout (the parity form) */
-#define MCTDHB_MIXED 1 /* complex64 H.C and density sums (Kahan), FP64 Lanczos scalars */
+#define MCTDHB_MIXED 1 /* complex64 coefficients and H.C, FP64 density sums and Lanczos scalars */
 
 /* index schemes */
 #define MCTDHB_INDEX_TABLES 0 /* read the reference jump tables */
