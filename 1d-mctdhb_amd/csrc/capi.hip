@@ -188,9 +188,13 @@ extern "C" int mctdhb_hc_tiling(mctdhb_space* sp, int set, int* tiling) {
         set_error("null space");
         return kInvalidArgument;
     }
-    if (set < -2 || set > 2) {
-        set_error("tiling must be -2 (query), -1 (time again), 0 (one configuration per lane), 1 (pairs) or 2 "
-                  "(coefficient windows)");
+    if (set < -2 || set > 3) {
+        set_error("tiling must be -2 (query), -1 (choose again), 0 (one configuration per lane), 1 (pairs), 2 "
+                  "(coefficient windows) or 3 (two stages)");
+        return kInvalidArgument;
+    }
+    if (set == kTilingTwo && !two_faster(sp->S, kPrecMixed)) {
+        set_error("the two-stage H.C is not the form of this space's size");
         return kInvalidArgument;
     }
     if (set == kTilingPair && !pair_possible(sp->S)) {

@@ -441,6 +441,7 @@ static DmWork dm_work(const Space* S, void* base) {
 int dm_workspace_create(const Space* S, void** work) {
     const size_t bytes = dm_work(S, nullptr).bytes;
     MCTDHB_HIP_CHECK(hipMalloc(work, bytes));
+    if (dm_generic(S->norb) || dm_plan(S).nb <= kDmFinishBlocks) return kOk;  // nothing counts
     MCTDHB_HIP_CHECK(hipMemset(*work, 0, 256));
     MCTDHB_HIP_CHECK(hipStreamSynchronize(nullptr));  // cleared before any stream counts
     return kOk;

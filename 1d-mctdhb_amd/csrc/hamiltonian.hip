@@ -8,6 +8,7 @@
 // deltas of fock.hpp (W table staged in LDS).  See hamiltonian.hpp for the
 // rule grouping.
 #include "hamiltonian_impl.hpp"
+#include "hc_coef.hpp"
 #include "hamiltonian_window.hpp"
 #include "pack.hpp"
 #include "rowctx.hpp"
@@ -49,6 +50,10 @@ bool hc_window_possible(const Space* S) { return window_possible(S); }
 
 int hc_tune_tiling(const Space* S, hipStream_t st) {
     if (S->hc_tiling >= 0) return kOk;
+    if (two_faster(S, kPrecMixed)) {
+        S->hc_tiling = kTilingTwo;
+        return kOk;
+    }
     const bool cand[3] = {true, pair_possible(S), hc_window_possible(S)};
     if (!cand[kTilingPair] && !cand[kTilingWindow]) {
         S->hc_tiling = kTilingLane;
@@ -122,73 +127,15 @@ unsigned hc_lanczos_blocks(const Space* S, int prec) {
 
 // ------------------------------------------------------- coefficient block
 
-// With sum_m n_m = N the last occupation is folded into the single-jump
-// coefficients: A'_kl = A_kl + N B_kl,M-1 and B'_klm = B_klm - B_kl,M-1, so
-// F_kl(n) = A'_kl + sum_{m < M-1} n_m B'_klm.
-__device__ __forceinline__ void hc_coefficients_block(int M, int N, const double2* __restrict__ hob,
-                                                      const double2* __restrict__ hint, double2* __restrict__ cf64,
-                                                      float2* __restrict__ cf32) {
-    const int t = threadIdx.x;
-    const int M2 = M * M, M3 = M2 * M;
-    auto G = [&](int a, int b, int c, int d) { return hint[a + b * M + c * M2 + d * M3]; };
-    double2* d64 = cf32 ? (double2*) (cf32 + cf_f64_off(M)) : nullptr;
-    auto put = [&](int idx, double2 v) {
-        cf64[idx] = v;
-        if (cf32) {
-            cf32[idx] = make_float2((float) v.x, (float) v.y);
-            // the one-body and diagonal sections once more in FP64
-            if (idx < cf_f64_count(M)) d64[idx] = v;
-        }
-    };
-    const int total = cf_size(M);
-    for (int idx = t; idx < total; idx += blockDim.x) {
-        double2 v = make_double2(0, 0);
-        // B_klm = g_kkkl (m = k), g_klll (m = l), 2 g_kmml (otherwise)
-        auto B = [&](int k, int l, int m) {
-            if (m == k) return G(k, k, k, l);
-            if (m == l) return G(k, l, l, l);
-            return cscale(G(k, m, m, l), 2.0);
-        };
-        if (idx < cf_off_B(M)) {  // A'_kl = h_kl - g_kkkl + N B_kl,M-1
-            int k = idx / M, l = idx % M;
-            if (k != l) v = hob[k * M + l] - G(k, k, k, l) + cscale(B(k, l, M - 1), (double) N);
-        } else if (idx < cf_off_d1(M)) {  // B'_klm = B_klm - B_kl,M-1
-            int r = idx - cf_off_B(M);
-            int k = r / M2, l = (r / M) % M, m = r % M;
-            if (k != l && m < M - 1) v = B(k, l, m) - B(k, l, M - 1);
-        } else if (idx < cf_off_d2(M)) {  // d1_k = h_kk - g_kkkk / 2
-            int k = idx - cf_off_d1(M);
-            v = hob[k * M + k] - cscale(G(k, k, k, k), 0.5);
-        } else if (idx < cf_off_d3(M)) {  // d2_k = g_kkkk / 2
-            int k = idx - cf_off_d2(M);
-            v = cscale(G(k, k, k, k), 0.5);
-        } else if (idx < cf_off_ot(M)) {  // d3_ks = 2 g_ksks (k < s)
-            int r = idx - cf_off_d3(M);
-            int k = r / M, s = r % M;
-            if (k < s) v = cscale(G(k, s, k, s), 2.0);
-        } else if (idx < cf_off_tt(M)) {  // Got[k][q][l]
-            int r = idx - cf_off_ot(M);
-            int k = r / M2, q = (r / M) % M, l = r % M;
-            if (q != k && l != k && q <= l) v = (q == l) ? cscale(G(k, k, q, q), 0.5) : G(k, k, q, l);
-        } else {  // Gtt[k][s][q][l]
-            int r = idx - cf_off_tt(M);
-            int k = r / M3, s = (r / M2) % M, q = (r / M) % M, l = r % M;
-            if (k < s && q <= l && q != k && q != s && l != k && l != s)
-                v = (q == l) ? G(k, s, q, q) : cscale(G(k, s, q, l), 2.0);
-        }
-        put(idx, v);
-    }
-}
-
 __global__ void k_hc_coefficients(int M, int N, const double2* __restrict__ hob, const double2* __restrict__ hint,
                                   double2* __restrict__ cf64, float2* __restrict__ cf32) {
-    hc_coefficients_block(M, N, hob, hint, cf64, cf32);
+    hc_coefficients_part(blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, M, N, hob, hint, cf64, cf32);
 }
 
 // Packed form (FP64 block only): one block per instance.
 __global__ void k_hc_coefficients_pk(const PkCf* __restrict__ tab, int M) {
     const PkCf a = tab[blockIdx.x];
-    hc_coefficients_block(M, a.npar, a.hob, a.hint, a.cf64, nullptr);
+    hc_coefficients_part(threadIdx.x, blockDim.x, M, a.npar, a.hob, a.hint, a.cf64, nullptr);
 }
 
 int pk_hc_coefficients(const PkCf* tab, int count, int M, hipStream_t st) {
@@ -199,7 +146,7 @@ int pk_hc_coefficients(const PkCf* tab, int count, int M, hipStream_t st) {
 
 int hc_coefficients(const Space* S, const double2* hob, const double2* hint, double2* cf64, float2* cf32,
                     hipStream_t st) {
-    k_hc_coefficients<<<1, 256, 0, st>>>(S->norb, S->npar, hob, hint, cf64, cf32);
+    k_hc_coefficients<<<div_up(cf_size(S->norb), 256), 256, 0, st>>>(S->norb, S->npar, hob, hint, cf64, cf32);
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
 }
@@ -413,6 +360,69 @@ static int check_mode(const Space* S, int prec, int index) {
     return kOk;
 }
 
+// Scratch of the two-stage product: up to kScratchBlocks blocks kept by the
+// space (freed with it), each with an event behind its last use.  A call takes
+// one that is idle, or a new one, or waits on the stream for the last use of
+// one, so calls on several streams and threads never share a block in flight.
+// (A stream-ordered allocation per call from a pool that keeps its memory
+// was tried first; now and then it mapped hundreds of MB anew in every call.)
+constexpr size_t kScratchBlocks = 4;
+
+static SpaceScratch* scratch_take(const Space* S, size_t bytes, hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
+    std::lock_guard<std::mutex> lock(S->scratch_mu);
+    SpaceScratch* pick = nullptr;
+    for (auto& b : S->scratch)
+        if (!b->busy && b->bytes >= bytes && hipEventQuery(b->done) == hipSuccess) {
+            b->busy = true;
+            return b.get();
+        }
+    (void) hipGetLastError();  // hipErrorNotReady of the blocks in flight
+    for (auto& b : S->scratch)
+        if (!b->busy && b->bytes >= bytes && (b->last == st || S->scratch.size() >= kScratchBlocks)) pick = b.get();
+    if (pick) {
+        if (hipStreamWaitEvent(st, pick->done, 0) != hipSuccess) return nullptr;
+        pick->busy = true;
+        return pick;
+    }
+    if (S->scratch.size() >= kScratchBlocks) return nullptr;
+    std::unique_ptr<SpaceScratch> b(new SpaceScratch());
+    if (hipMalloc(&b->p, bytes) != hipSuccess ||
+        hipEventCreateWithFlags(&b->done, hipEventDisableTiming) != hipSuccess) {
+        (void) hipGetLastError();
+        return nullptr;  // ~SpaceScratch frees what there is
+    }
+    b->bytes = bytes;
+    b->busy = true;
+    S->scratch.push_back(std::move(b));
+    return S->scratch.back().get();
+}
+
+static int scratch_give(const Space* S, SpaceScratch* b, hipStream_t st) {
+    const hipError_t e = hipEventRecord(b->done, st);
+    std::lock_guard<std::mutex> lock(S->scratch_mu);
+    b->last = st;
+    b->busy = false;
+    MCTDHB_HIP_CHECK(e);
+    return kOk;
+}
+
+// hc = H coef in two stages, X given or formed from hob and hint.  False
+// (nothing enqueued) when this space or stream takes the one-stage kernels.
+static bool two_stage(const Space* S, const void* coef, const double2* X, const double2* hob, const double2* hint,
+                      void* hc, int prec, hipStream_t st, int& rc) {
+    if (!two_chosen(S, prec)) return false;
+    SpaceScratch* b = scratch_take(S, two_matrix_bytes(S) + two_psi_bytes(S, prec), st);
+    if (!b) return false;
+    char* psi = (char*) b->p + two_matrix_bytes(S);
+    rc = X ? kOk : two_matrix(S, hob, hint, (double2*) b->p, st);
+    if (!rc) rc = two_apply(S, coef, X ? X : (const double2*) b->p, psi, hc, prec, st);
+    const int rg = scratch_give(S, b, st);
+    if (!rc) rc = rg;
+    return true;
+}
+
 int hc_apply(const Space* S, const void* coef, const double2* hob, const double2* hint, void* hc, int prec,
              int index, hipStream_t st) {
     int rc = check_mode(S, prec, index);
@@ -425,6 +435,7 @@ int hc_apply(const Space* S, const void* coef, const double2* hob, const double2
         return kOk;
     }
     if (prec == kPrecMixed && (rc = hc_tune_tiling(S, st))) return rc;
+    if (two_stage(S, coef, nullptr, hob, hint, hc, prec, st, rc)) return rc;
     const int M = S->norb;
     double2* cf64 = nullptr;
     float2* cf32 = nullptr;
@@ -527,12 +538,18 @@ int hc_apply_noalloc(const Space* S, const void* coef, const double2* hob, const
     return dispatch_plain_tiled(S, coef, cf32, hc, 0, st);
 }
 
+// (16-byte aligned: what follows is complex128)
+static size_t hc_one_stage_bytes(int M, int prec) {
+    const size_t b = sizeof(double2) * cf_size(M) + (prec == kPrecMixed ? sizeof(float2) * cf32_size(M) : 0);
+    return (b + 15) & ~(size_t) 15;
+}
+
 size_t hc_coef_bytes(const Space* S, int prec) {
     const int M = S->norb;
     if (use_generic(S)) return sizeof(double2) * ((size_t) M * M + (size_t) M * M * M * M);
-    // FP64 block, followed by the complex64 copy for the mixed form
-    size_t b = sizeof(double2) * cf_size(M);
-    if (prec == kPrecMixed) b += sizeof(float2) * cf32_size(M);
+    // FP64 block, the complex64 copy for the mixed form, the pair matrix
+    size_t b = hc_one_stage_bytes(M, prec);
+    if (S->d_low) b += two_matrix_bytes(S);
     return b;
 }
 
@@ -546,7 +563,9 @@ int hc_build_coef(const Space* S, const double2* hob, const double2* hint, void*
     }
     double2* cf64 = (double2*) cf;
     float2* cf32 = prec == kPrecMixed ? (float2*) (cf64 + cf_size(M)) : nullptr;
-    return hc_coefficients(S, hob, hint, cf64, cf32, st);
+    const int rc = hc_coefficients(S, hob, hint, cf64, cf32, st);
+    if (rc || !S->d_low) return rc;
+    return two_matrix(S, hob, hint, (double2*) ((char*) cf + hc_one_stage_bytes(M, prec)), st);
 }
 
 int hc_apply_cf(const Space* S, const void* coef, const void* cf, void* hc, int prec, int index, hipStream_t st) {
@@ -562,6 +581,8 @@ int hc_apply_cf(const Space* S, const void* coef, const void* cf, void* hc, int 
         return kOk;
     }
     if (prec == kPrecMixed && (rc = hc_tune_tiling(S, st))) return rc;
+    const double2* X = S->d_low ? (const double2*) ((const char*) cf + hc_one_stage_bytes(M, prec)) : nullptr;
+    if (X && two_stage(S, coef, X, nullptr, nullptr, hc, prec, st, rc)) return rc;
     const void* blk = prec == kPrecFP64 ? cf : (const void*) ((const double2*) cf + cf_size(M));
     return dispatch_fused_plain(S, coef, blk, hc, prec, index, st);
 }

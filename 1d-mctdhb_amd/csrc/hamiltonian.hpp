@@ -21,6 +21,7 @@
 // distinct target (130 instead of 230 at N=100, M=5).
 #pragma once
 
+#include "pairs.hpp"
 #include "sil.hpp"
 #include "space.hpp"
 
@@ -110,7 +111,7 @@ unsigned hc_grid_blocks(uint32_t dim);
 // in LDS, one far group of jump types after another (2, 2 <= norb <= 5 and
 // N up to 185; the plain product only: the Lanczos forms keep the one-lane
 // kernel under it).
-constexpr int kTilingLane = 0, kTilingPair = 1, kTilingWindow = 2;
+constexpr int kTilingLane = 0, kTilingPair = 1, kTilingWindow = 2, kTilingTwo = 3;
 inline bool pair_possible(const Space* S) { return S->d_slots && S->dim >= 2 && S->norb >= 2 && S->norb <= 7; }
 inline bool use_pair(const Space* S, int prec) {
     return prec == kPrecMixed && pair_possible(S) && S->hc_tiling == kTilingPair;
@@ -178,6 +179,40 @@ struct SmallSilArgs {
 int hc_sil_small(const Space* S, const double2* cf64, const SmallSilArgs& a, int index, hipStream_t st);
 
 struct PkSil;
+
+// ------------------------------------------------ two stages (hamiltonian_two.hpp)
+// Elements between the arrays of psi of consecutive pairs, and the bytes of
+// all of them.
+inline size_t two_ld(const Space* S) { return ((size_t) S->low_dim + 15) & ~(size_t) 15; }
+inline size_t two_psi_bytes(const Space* S, int prec) {
+    return (size_t) pair_count(S->norb) * two_ld(S) * (prec == kPrecFP64 ? sizeof(double2) : sizeof(float2));
+}
+// The pair matrix X (P x P complex128).
+inline size_t two_matrix_bytes(const Space* S) {
+    return sizeof(double2) * pair_count(S->norb) * pair_count(S->norb);
+}
+// Whether the kernels cover this space (there are pairs, 32-bit byte offsets,
+// tables in LDS), and whether they are the faster form there.
+bool two_possible(const Space* S, int prec);
+bool two_faster(const Space* S, int prec);
+// ... and the form of this space now (the mixed tiling may be set by hand).
+inline bool two_chosen(const Space* S, int prec) {
+    return two_faster(S, prec) && (prec == kPrecFP64 || S->hc_tiling == kTilingTwo);
+}
+int two_matrix(const Space* S, const double2* hob, const double2* hint, double2* X, hipStream_t st);
+int two_apply(const Space* S, const void* c, const double2* X, void* psi, void* out, int prec, hipStream_t st);
+// The Lanczos form (partials as hc_lanczos leaves them).
+int two_lanczos(const Space* S, const double2* X, void* psi, const LanczosHcArgs& a, int prec, hipStream_t st);
+// The last iteration of either form: <w_it, H w_it> of two_rayleigh_blocks
+// blocks in slot 2 it.  The first stage without a store.
+int two_rayleigh(const Space* S, const double2* X, const LanczosHcArgs& a, int prec, hipStream_t st);
+inline unsigned two_rayleigh_blocks(const Space* S) { return div_up(S->low_dim, 256); }
+
+template <int M> struct HcTwo {
+    static int plain(const Space* S, const void* c, const double2* X, void* psi, void* out, int prec, hipStream_t st);
+    static int lanczos(const Space* S, const double2* X, void* psi, const LanczosHcArgs& a, int prec, hipStream_t st);
+    static int rayleigh(const Space* S, const double2* X, const LanczosHcArgs& a, int prec, hipStream_t st);
+};
 
 // Per-orbital-count entry points of the fused kernel (hc_m<M>.hip).  The
 // mixed form always uses on-the-fly indices.

@@ -18,6 +18,7 @@
 // no host synchronisation.
 #include "density.hpp"
 #include "hamiltonian.hpp"
+#include "hc_coef.hpp"
 #include "sil_api.hpp"
 #include "sil_device.hpp"
 
@@ -26,12 +27,31 @@ namespace mctdhb {
 constexpr int kStreamBlock = 256;
 constexpr int kStreamGrid = 1024;
 
-// -------------------------------------------------------------- scalars
+// -------------------------------------------------------------- start
 
-__global__ void k_sil_init(SilState* st, int lm) {
-    if (threadIdx.x == 0) sil_init_state(st, lm);
+// Everything a recursion starts from, in one launch (four before, 3 to 5 us
+// each where the space is small): the scalars (block 0), the coefficients of
+// the H.C form in use and the complex64 copy of C, where wanted.
+struct SilBegin {
+    SilState* st;
+    const double2 *hob, *hint;
+    double2* cf64;  // null: not needed
+    float2* cf32;
+    double2* X;     // null: not needed
+    const double2* C;
+    float2* w0;     // null: not needed
+    uint32_t n;
+    int M, N, lm;
+};
+
+__global__ __launch_bounds__(kStreamBlock) void k_sil_begin(SilBegin a) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    if (blockIdx.x == 0) sil_init_state(a.st, a.lm, threadIdx.x, blockDim.x);
+    if (a.cf64) hc_coefficients_part(t, stride, a.M, a.N, a.hob, a.hint, a.cf64, a.cf32);
+    if (a.X) pair_matrix_part(t, stride, a.M, a.N, a.hob, a.hint, a.X);
+    if (a.w0)
+        for (uint32_t i = t; i < a.n; i += stride) a.w0[i] = from_d2<float2>(a.C[i]);
 }
-
 
 // Sum per-block partials (slot-major): tot[t] = sum_b part[t * nblocks + b],
 // one block per slot.
@@ -125,13 +145,6 @@ __global__ __launch_bounds__(64) void k_sil_ground(SilState* st) {
 }
 
 // ---------------------------------------------------------- streaming
-
-template <typename Zw>
-__global__ __launch_bounds__(kStreamBlock) void k_to_complex64(const double2* __restrict__ a, Zw* __restrict__ b,
-                                                               uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        b[i] = from_d2<Zw>(a[i]);
-}
 
 struct WPtrs {
     const void* w[kMaxKrylov];
@@ -347,6 +360,12 @@ int sil_create(const Space* S, int lm, int prec, int index, Sil** out) {
         *vec = (char*) *base + esz;
         return true;
     };
+    if (!generic && two_possible(S, prec)) ok = ok && hipMalloc((void**) &L->X, two_matrix_bytes(S)) == hipSuccess;
+    // without room for the first stage's values the one-stage kernels run
+    if (ok && L->X && two_chosen(S, prec) && hipMalloc(&L->psi, two_psi_bytes(S, prec)) != hipSuccess) {
+        L->psi = nullptr;
+        (void) hipGetLastError();
+    }
     for (int k = 1; k < lm && ok; k++) ok = padded(&L->wbase[k], &L->w[k], zw);
     if (prec == kPrecMixed) ok = ok && padded(&L->w0fbase, &L->w0f, sizeof(float2));
     if (!ok) {
@@ -363,6 +382,8 @@ void sil_destroy(Sil* L) {
     hipFree(L->d_st);
     hipFree(L->cf64);
     hipFree(L->cf32);
+    hipFree(L->X);
+    hipFree(L->psi);
     hipFree(L->out);
     hipFree(L->part);
     hipFree(L->tot);
@@ -376,6 +397,7 @@ size_t sil_device_bytes(const Space* S, int lm, int prec) {
     const size_t zw = prec == kPrecFP64 ? sizeof(double2) : sizeof(float2);
     size_t b = (size_t) (lm - 1) * zw * n + sizeof(double2) * n;
     if (prec == kPrecMixed) b += sizeof(float2) * n;
+    if (two_faster(S, prec)) b += two_psi_bytes(S, prec);
     return b;
 }
 
@@ -435,23 +457,39 @@ static int sil_run_lanczos(Sil* L, const double2* C, const double2* hob, const d
     const Space* S = L->S;
     const uint32_t n = S->dim;
     int rc;
-    k_sil_init<<<1, 64, 0, st>>>(L->d_st, L->lm);
+    SilBegin bg{};
+    bg.st = L->d_st;
+    bg.hob = hob;
+    bg.hint = hint;
+    bg.M = S->norb;
+    bg.N = S->npar;
+    bg.lm = L->lm;
+    unsigned blocks = 1;
     if (L->generic) {
         const int M = S->norb;
         MCTDHB_HIP_CHECK(hipMemcpyAsync(L->cf64, hob, sizeof(double2) * M * M, hipMemcpyDeviceToDevice, st));
         MCTDHB_HIP_CHECK(hipMemcpyAsync(L->cf64 + M * M, hint, sizeof(double2) * M * M * M * M,
                                         hipMemcpyDeviceToDevice, st));
     } else {
-        rc = hc_coefficients(S, hob, hint, L->cf64, L->cf32, st);
-        if (rc) return rc;
+        bg.X = L->X;
+        if (L->X) blocks = div_up(two_matrix_bytes(S) / sizeof(double2), kStreamBlock);
+        if (!L->psi) {
+            bg.cf64 = L->cf64;
+            bg.cf32 = L->cf32;
+            blocks = std::max(blocks, div_up(cf_size(S->norb), kStreamBlock));
+        }
     }
     if (L->prec == kPrecMixed) {
-        k_to_complex64<float2><<<kStreamGrid, kStreamBlock, 0, st>>>(C, (float2*) L->w0f, n);
+        bg.C = C;
+        bg.w0 = (float2*) L->w0f;
+        bg.n = n;
+        blocks = std::max(blocks, std::min((unsigned) kStreamGrid, div_up(n, kStreamBlock)));
         L->w[0] = L->w0f;
     } else {
         L->w[0] = (void*) C;
     }
-    if (L->prec == kPrecMixed && (rc = hc_tune_tiling(S, st))) return rc;
+    k_sil_begin<<<blocks, kStreamBlock, 0, st>>>(bg);
+    if (L->prec == kPrecMixed && !L->psi && (rc = hc_tune_tiling(S, st))) return rc;
     const unsigned nbh = hc_lanczos_blocks(S, L->prec);
     for (int it = 0; it < L->lm; it++) {
         LanczosHcArgs a{};
@@ -461,9 +499,14 @@ static int sil_run_lanczos(Sil* L, const double2* C, const double2* hob, const d
         a.out = L->out;
         a.part = L->part;
         a.last = it == L->lm - 1;
-        rc = hc_lanczos(S, L->cf64, L->cf32, a, L->prec, L->index, st);
+        if (a.last && L->X) rc = two_rayleigh(S, L->X, a, L->prec, st);
+        else if (L->psi) rc = two_lanczos(S, L->X, L->psi, a, L->prec, st);
+        else rc = hc_lanczos(S, L->cf64, L->cf32, a, L->prec, L->index, st);
         if (rc) return rc;
-        if (a.last)
+        if (a.last && L->X)
+            k_reduce_scalars<0><<<1, kReduceBlock, 0, st>>>(L->part, two_rayleigh_blocks(S), L->tot, L->d_st, it,
+                                                             2 * it, 2);
+        else if (a.last)
             k_reduce_scalars<0><<<2, kReduceBlock, 0, st>>>(L->part, nbh, L->tot, L->d_st, it, 2 * it,
                                                              hc_lanczos_half(S, L->prec) && !L->generic ? 2 : 1);
         else

@@ -21,6 +21,10 @@ struct Sil {
     void* wbase[kMaxKrylov] = {};
     void* w0f = nullptr;
     void* w0fbase = nullptr;
+    // the two-stage H.C (when it is the form of this workspace): pair matrix
+    // and first-stage values
+    double2* X = nullptr;
+    void* psi = nullptr;
     double2* out = nullptr;
     double* part = nullptr;
     size_t part_cap = 0;

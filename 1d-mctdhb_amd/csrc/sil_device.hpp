@@ -12,17 +12,17 @@ namespace mctdhb {
 
 constexpr double kBreakdownTol = 1e-14;  // reference multiconfig_lanczos.c:34
 
-// Fresh scalars for an lm-vector recursion (one thread).
-__device__ inline void sil_init_state(SilState* st, int lm) {
-    for (int k = 0; k <= kMaxKrylov; k++) {
-        st->s[k] = 0;
+// Fresh scalars for an lm-vector recursion, by threads t of T.
+__device__ inline void sil_init_state(SilState* st, int lm, int t, int T) {
+    for (int k = t; k <= kMaxKrylov; k += T) {
+        st->s[k] = k == 0 ? 1.0 : 0.0;
         st->beta[k] = 0;
         st->alpha[k] = make_double2(0, 0);
         st->cre[k] = make_double2(0, 0);
         st->gram[k] = make_double2(0, 0);
         st->y[k] = make_double2(0, 0);
     }
-    st->s[0] = 1.0;
+    if (t != 0) return;
     st->maxbeta = 0;
     st->nrm2 = 0;
     st->eground = 0;

@@ -1,6 +1,8 @@
 // space.hpp - the device-resident configurational space (tables + LUTs).
 #pragma once
 
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "fock.hpp"
@@ -10,6 +12,19 @@ namespace mctdhb {
 constexpr int kMaxOrb = 30;    // reference MAX_ORBITALS (mctdhb_types.h:29)
 constexpr int kMaxPar = 10000; // reference MAX_PARTICLES (mctdhb_types.h:31)
 constexpr int kSpaceTables = 1;  // also build the reference-layout jump tables
+
+// A device block with the event behind its last use.
+struct SpaceScratch {
+    void* p = nullptr;
+    size_t bytes = 0;
+    hipEvent_t done = nullptr;
+    hipStream_t last = nullptr;
+    bool busy = false;
+    ~SpaceScratch() {
+        if (done) hipEventDestroy(done);
+        hipFree(p);  // waits for the device: no use is in flight after it
+    }
+};
 
 struct Space {
     int npar = 0, norb = 0;
@@ -48,6 +63,9 @@ struct Space {
     // tiling of the mixed H.C kernel picked by timing both on this space:
     // -1 not yet timed, 0 one configuration per lane, 1 configuration pairs
     mutable int hc_tiling = -1;
+    // scratch of the two-stage product between calls (hamiltonian.hip)
+    mutable std::vector<std::unique_ptr<SpaceScratch>> scratch;
+    mutable std::mutex scratch_mu;
 };
 
 int space_dimension_exact(int npar, int norb, uint32_t* dim);

@@ -270,9 +270,11 @@ int mctdhb_apply_hamiltonian_dev(const mctdhb_space* space, const void* coef, co
  * norb <= 7; norb 1 and > 7 read hob and hint directly); the space's device
  * must be current.  Every call on one GPU shares that array, so calls that
  * overlap on one GPU (different streams, or threads) race; serialise them.
- * The mixed form runs one configuration per lane unless the paired tiling
- * was already chosen on this space by an allocating call.  Same arguments,
- * results and errors as mctdhb_apply_hamiltonian_dev. */
+ * It never takes the two-stage form (norb 6 and 7), whose scratch does not
+ * fit; the mixed form runs one configuration per lane unless the paired
+ * tiling was already chosen on this space by an allocating call.  Same
+ * arguments and errors as mctdhb_apply_hamiltonian_dev, same results to the
+ * rounding of the form. */
 int mctdhb_apply_hamiltonian_noalloc_dev(const mctdhb_space* space, const void* coef, const void* hob,
                                          const void* hint, void* hc, int prec, int index, void* stream);
 
@@ -290,11 +292,12 @@ int    mctdhb_apply_hamiltonian_cf_dev(const mctdhb_space* space, const void* co
  * both), 2 one configuration per lane with the coefficients each block
  * reaches staged in LDS, one window per far group of jump types
  * (2 <= norb <= 5, N <= 185; the plain product only, the SIL step's
- * Lanczos forms keep tiling 0 under it).  By default the possible ones are
- * timed at the first mixed call on a space of a new (N, M) and the fastest
- * kept for every space of that shape in the process (so a solve runs the
- * same kernels alone and among others).
- * set: -2 query only, -1 time again, 0, 1 or 2 force; *tiling
+ * Lanczos forms keep tiling 0 under it), 3 two stages over the space of
+ * N - 2 particles (norb 6 and 7, N >= 2).  By default norb 6 and 7 take 3;
+ * elsewhere the possible ones are timed at the first mixed call on a space of
+ * a new (N, M) and the fastest kept for every space of that shape in the
+ * process (so a solve runs the same kernels alone and among others).
+ * set: -2 query only, -1 choose again, 0 to 3 force; *tiling
  * (may be NULL) receives the current choice (-1: not yet timed).  Callers
  * that change it must not have a mixed SIL workspace open on the space. */
 int mctdhb_hc_tiling(mctdhb_space* space, int set, int* tiling);

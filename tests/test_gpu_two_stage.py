@@ -1,0 +1,123 @@
+"""The two-stage H.C (M = 6, 7) where it can go wrong: N = 1 (no pairs: the
+one-stage kernel), N = 2 (one configuration of N - 2 particles), sizes around
+its 256-thread blocks, every call that takes it (product, prebuilt
+coefficients, products on two streams at once, under capture), and h and g
+without the usual symmetries, where it must read the same entries as the
+one-stage kernel.  The last Lanczos iteration's pair form of <w, H w> is
+covered for every orbital count.
+
+Bounds: FP64 sums of at most 504 products agree to 1e-12 of the largest
+element.  In the mixed form psi and the result are complex64 (6e-8 each, some
+30 values summed in FP64), below 1e-6 of the largest element."""
+import math
+
+import numpy as np
+import pytest
+
+import gpu_util as gu
+import inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def amd():
+    import mctdhb_amd
+
+    mctdhb_amd.lib()
+    return mctdhb_amd
+
+
+def _problem(npar, norb, symmetric=True):
+    dim = math.comb(npar + norb - 1, norb - 1)
+    if symmetric:
+        return inputs.coefficients(dim, 3), inputs.onebody(norb, 3), inputs.twobody(norb, 3, 0.3)
+    r = np.random.default_rng(8)
+    z = lambda *s: r.standard_normal(s) + 1j * r.standard_normal(s)
+    return inputs.coefficients(dim, 3), z(norb, norb), z(norb ** 4)
+
+
+# NC' = C(N + M - 3, M - 1): 252 and 462 (M = 6), 210 and 462 (M = 7)
+@pytest.mark.parametrize("npar,norb", [(1, 6), (1, 7), (2, 6), (2, 7), (3, 7), (7, 6), (8, 6), (6, 7), (7, 7)])
+def test_product_matches_oracle(amd, orc, npar, norb):
+    print(f"two-stage N={npar} M={norb}", flush=True)
+    c, h, g = _problem(npar, norb)
+    ref = orc.Space(npar, norb).apply_hamiltonian(c, h, g)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    dh, dg = gu.dev(h), gu.dev(g)
+    for prec, dt, tol in ((amd.FP64, np.complex128, 1e-12), (amd.MIXED, np.complex64, 1e-6)):
+        out = gu.empty(D.dim, np.dtype(dt).name)
+        D.apply_hamiltonian(gu.dev(c, dt), dh, dg, out, prec=prec)
+        assert gu.rel_err(gu.host(out), ref) < tol
+        cf = gu.empty(D.coef_bytes(prec) // 8 + 1, "float64")
+        D.hc_coefficients(dh, dg, cf, prec=prec)
+        out2 = gu.empty(D.dim, np.dtype(dt).name)
+        D.apply_hamiltonian_cf(gu.dev(c, dt), cf, out2, prec=prec)
+        assert np.array_equal(gu.host(out2), gu.host(out))
+    D.close()
+
+
+@pytest.mark.parametrize("npar,norb", [(5, 6), (4, 7), (9, 6)])
+def test_same_entries_of_h_and_g_as_the_one_stage_kernel(amd, npar, norb):
+    c, h, g = _problem(npar, norb, symmetric=False)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    a, b = gu.empty(D.dim), gu.empty(D.dim)
+    D.apply_hamiltonian(gu.dev(c), gu.dev(h), gu.dev(g), a)
+    D.apply_hamiltonian_noalloc(gu.dev(c), gu.dev(h), gu.dev(g), b)  # one stage
+    assert not np.array_equal(gu.host(a), gu.host(b))  # two kernels
+    assert gu.rel_err(gu.host(a), gu.host(b)) < 1e-12
+    D.close()
+
+
+def test_products_on_two_streams_do_not_share_scratch(amd, orc):
+    import torch
+
+    npar, norb = 12, 6
+    dim = math.comb(npar + norb - 1, norb - 1)
+    h, g = inputs.onebody(norb, 3), inputs.twobody(norb, 3, 0.3)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    dh, dg = gu.dev(h), gu.dev(g)
+    cs = [gu.dev(inputs.coefficients(dim, 20 + i)) for i in range(6)]
+    ref = []
+    for c in cs:
+        o = gu.empty(dim)
+        D.apply_hamiltonian(c, dh, dg, o)
+        ref.append(gu.host(o))
+    st = [torch.cuda.Stream() for _ in range(6)]  # more than the blocks kept
+    outs = [gu.empty(dim) for _ in cs]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for c, o, s in zip(cs, outs, st):
+            D.apply_hamiltonian(c, dh, dg, o, stream=s)
+    torch.cuda.synchronize()
+    for o, r in zip(outs, ref):
+        assert np.array_equal(gu.host(o), r)
+    D.close()
+
+
+@pytest.mark.parametrize("npar,norb,lm", [(2, 2, 3), (9, 2, 5), (12, 3, 6), (10, 4, 5), (9, 5, 4), (7, 6, 6),
+                                          (5, 7, 5), (1, 6, 4)])
+@pytest.mark.parametrize("imag", [False, True])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_sil_step_matches_oracle(amd, orc, npar, norb, lm, imag, prec):
+    print(f"two-stage sil N={npar} M={norb} lm={lm} imag={imag} prec={prec}", flush=True)
+    c, h, g = _problem(npar, norb)
+    dt = -0.01j if imag else 0.01
+    _, ref = orc.Space(npar, norb).sil_step(c, h, g, lm, dt, imag)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    sil = amd.DeviceSil(D, lm, prec=prec, index=amd.INDEX_FLY)
+    sil.set_small(False)
+    dc = gu.dev(c)
+    sil.step(dc, gu.dev(h), gu.dev(g), dt, imag)
+    assert gu.rel_err(gu.host(dc), ref) < (1e-10 if prec == amd.FP64 else 2e-5)
+    sil.close()
+    D.close()
+
+
+def test_tiling_names_the_form(amd):
+    D6, D5 = amd.DeviceSpace(6, 6, tables=False), amd.DeviceSpace(6, 5, tables=False)
+    assert D6.hc_tiling(3) == 3 and D6.hc_tiling(0) == 0
+    with pytest.raises(amd.MctdhbError):
+        D5.hc_tiling(3)
+    D6.close()
+    D5.close()
