@@ -102,11 +102,11 @@ __global__ __launch_bounds__(kReduceBlock) void k_reduce_scalars(const double* _
         last = atomicAdd(&st->arrive, 1u) == gridDim.x - 1;
     }
     __syncthreads();
-    if (!last || threadIdx.x != 0) return;
+    if (!last || threadIdx.x >= 64) return;
     __threadfence();
-    st->arrive = 0;
-    if (OP == 0) sil_after_hc(st, tot, it, final_it);
-    else sil_after_reorth(st, tot, it);
+    if (threadIdx.x == 0) st->arrive = 0;
+    if (OP == 0) sil_after_hc(st, tot, it, final_it, threadIdx.x);
+    else sil_after_reorth(st, tot, it, threadIdx.x);
 }
 
 

@@ -108,12 +108,15 @@ __device__ __forceinline__ void sil_small_block(unsigned char* smem, const RowCt
             if (it == 0) acc[2] += wit[i].x * wit[i].x + wit[i].y * wit[i].y;
         }
         block_sum_slots(acc, 2 * (it + 1) + 1, L.red, L.tot);
-        if (threadIdx.x == 0) {
-            for (int k = k0; k <= it; k++) {  // d_k = s_k <w_k, out>
+        if (threadIdx.x < 64) {
+            const int k = threadIdx.x;
+            if (k >= k0 && k <= it) {  // d_k = s_k <w_k, out>
                 L.tot[2 * k] *= st->s[k];
                 L.tot[2 * k + 1] *= st->s[k];
             }
-            sil_after_hc(st, L.tot, it, last ? 1 : 0);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            sil_after_hc(st, L.tot, it, last ? 1 : 0, k);
         }
         __syncthreads();
         if (last) break;
@@ -143,7 +146,7 @@ __device__ __forceinline__ void sil_small_block(unsigned char* smem, const RowCt
         for (int t = 0; t < kSmallSlots; t++)  // slot 2 (it + 1), by constant indices
             if (t == 2 * (it + 1)) acc[t] = nrm;
         block_sum_slots(acc, 2 * (it + 1) + 1, L.red, L.tot);
-        if (threadIdx.x == 0) sil_after_reorth(st, L.tot, it);
+        if (threadIdx.x < 64) sil_after_reorth(st, L.tot, it, threadIdx.x);
         __syncthreads();
         if (st->stop) break;
     }
