@@ -701,7 +701,8 @@ struct PackGroup {
     bool stage = false;
     int count = 0;
     void* d_tab = nullptr;  // every stage table, one allocation
-    size_t fft_smem = 0, gs_smem = 0, sil_smem = 0, dm_smem = 0;
+    size_t fft_smem = 0, sil_smem = 0, dm_smem = 0;
+    int gs_threads = 0;
     unsigned fft_n = 0, nl_blocks = 0, dm_grid = 0;
     mctdhb_step_graph graph;
 };
@@ -765,7 +766,7 @@ static int pack_enqueue(const PackGroup& g, PkFft* fft, PkOm* om, PkNlCoef* nlc,
     if (!rc && !g.fold) rc = pk_nl_coef(nlc, g.count, g.M, st);
     if (!rc) rc = pk_nl_rk(nl, g.count, g.M, g.ns, g.nl_blocks, st);
     if (!rc) rc = pk_linear_fft(fft, g.count, g.M, g.fft_smem, st);
-    if (!rc && g.imagtime) rc = pk_gram_schmidt(gs, g.count, g.M, g.gs_smem, st);
+    if (!rc && g.imagtime) rc = pk_gram_schmidt(gs, g.count, g.M, g.gs_threads, st);
     if (!rc) rc = pk_orbital_matrices(om, g.count, g.M, st);
     if (!rc) rc = pk_hc_coefficients(cf, g.count, g.M, st);
     if (!rc) rc = pk_sil_small(sil, g.count, g.M, g.index, g.stage, g.sil_smem, st);
@@ -870,9 +871,8 @@ extern "C" int mctdhb_pack_create(int n, mctdhb_space* const* spaces, mctdhb_sil
             nl[j] = PkNl{o, w->d_pot, w->d_nl, h1, h2, (const double2*) rho2[i], (const double2*) rinv[i],
                          q.tstep, q.g, q.time_fac, q.grid_size};
             g.nl_blocks = std::max(g.nl_blocks, div_up((unsigned) q.grid_size, 64u));
-            const size_t gsm = pk_gs_smem(q.norb, q.grid_size);
-            gs[j] = PkGs{o, q.dx, q.grid_size, q.bounds == kPeriodicBounds ? 1 : 0, gsm ? 1 : 0};
-            g.gs_smem = std::max(g.gs_smem, gsm);
+            gs[j] = PkGs{o, q.dx, q.grid_size, q.bounds == kPeriodicBounds ? 1 : 0};
+            g.gs_threads = std::max(g.gs_threads, pk_gs_threads(q.grid_size));
             cf[j] = PkCf{h1, h2, L->cf64, S->npar};
             SmallSilArgs a{};
             a.st = L->d_st;

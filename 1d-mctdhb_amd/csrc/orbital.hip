@@ -11,6 +11,7 @@
 // The odelib Runge-Kutta the reference links is absent; the nonlinear step
 // uses the classical RK4 tableau.
 #include <cmath>
+#include <complex>
 #include <vector>
 
 #include "mxm_wave.hpp"
@@ -280,109 +281,130 @@ __global__ void k_cn_sequential(double2* __restrict__ orb, int M, int grid, int 
 }
 
 // One block per orbital: the CN right-hand side, then the tridiagonal solve
-// by parallel cyclic reduction (PCR) in place of the two sequential sweeps:
-// log2(m) steps, each eliminating the couplings to the rows s = 1, 2, 4, ...
-// away, every row at once.  Periodic bounds (a cyclic system of size
-// m = grid - 1) go through Sherman-Morrison like the reference
+// with factors made when the workspace is (the matrix never changes): row i
+// of the LU factors without pivoting (the matrix is diagonally dominant) gives
+//   z_i = r_i - L_i z_{i-1},   x_i = IU_i z_i - CU_i x_{i+1},
+// two first-order recurrences, each a prefix scan of affine maps over the
+// threads (PER consecutive rows each).  Periodic bounds (a cyclic system of
+// size m = grid - 1) go through Sherman-Morrison like the reference
 // (tridiagonal_solver.c:161-212), with the textbook split gamma = -b_0
-// (Numerical Recipes' cyclic solver) instead of the reference's
-// gamma = b_0, which leaves a zero first pivot that only a sequential sweep
-// can take; both give the solution of the same system.  The matrix is
-// strictly diagonally dominant (|b_i| > |a_i| + |c_i| for the CN operator),
-// where PCR is stable.  Coefficients (a, b, c, two right-hand sides) live in
-// the workspace scratch, double-buffered: 10 m entries per orbital.
-constexpr int kCnPcrBlock = 1024;
-constexpr int kCnPcrMaxRows = 2 * kCnPcrBlock;  // rows per thread <= 2
-__global__ __launch_bounds__(kCnPcrBlock) void k_cn_pcr(double2* __restrict__ orb, int grid, int bounds,
-                                                         const double2* __restrict__ cn, double2 rhs_up,
-                                                         double2 rhs_lo, double2 rhs_mid, double2* __restrict__ scratch) {
-    const int k = blockIdx.x;
-    double2* f = orb + (size_t) k * grid;
-    const double2 *up = cn, *lo = cn + grid, *mid0 = cn + 2 * grid;
-    const int n = grid;
+// (Numerical Recipes' cyclic solver) instead of the reference's gamma = b_0,
+// which leaves a zero first pivot that only a sequential sweep can take; the
+// correction vector is a factor too.  Bound by the latency of the two scans;
+// cyclic reduction of every row at every step through memory took 35.6 us a
+// half step with 5 orbitals on 801 points, this form 6.5.
+struct CnScanLds {
+    double2 a[16], b[16];  // the waves' maps
+    double2 y0, ym;
+};
+
+// (A, B) of the maps before this thread's own, in the order of the threads
+// (UP) or against it: an inclusive scan over the wave, then over the waves.
+template <bool UP> __device__ __forceinline__ double2 cn_scan(double2 A, double2 B, CnScanLds& L) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    for (int off = 1; off < 64; off <<= 1) {
+        double2 pa, pb;
+        pa.x = UP ? __shfl_up(A.x, off, 64) : __shfl_down(A.x, off, 64);
+        pa.y = UP ? __shfl_up(A.y, off, 64) : __shfl_down(A.y, off, 64);
+        pb.x = UP ? __shfl_up(B.x, off, 64) : __shfl_down(B.x, off, 64);
+        pb.y = UP ? __shfl_up(B.y, off, 64) : __shfl_down(B.y, off, 64);
+        if (UP ? lane >= off : lane + off < 64) {
+            B = cfma(A, pb, B);
+            A = cmul(A, pa);
+        }
+    }
+    if (lane == (UP ? 63 : 0)) {
+        L.a[wave] = A;
+        L.b[wave] = B;
+    }
+    double2 ea, eb;  // the maps before this lane's, within the wave
+    ea.x = UP ? __shfl_up(A.x, 1, 64) : __shfl_down(A.x, 1, 64);
+    ea.y = UP ? __shfl_up(A.y, 1, 64) : __shfl_down(A.y, 1, 64);
+    eb.x = UP ? __shfl_up(B.x, 1, 64) : __shfl_down(B.x, 1, 64);
+    eb.y = UP ? __shfl_up(B.y, 1, 64) : __shfl_down(B.y, 1, 64);
+    if (lane == (UP ? 0 : 63)) {
+        ea = make_double2(1, 0);
+        eb = make_double2(0, 0);
+    }
+    __syncthreads();
+    double2 in = make_double2(0, 0);
+    if (UP)
+        for (int u = 0; u < wave; u++) in = cfma(L.a[u], in, L.b[u]);
+    else
+        for (int u = nw - 1; u > wave; u--) in = cfma(L.a[u], in, L.b[u]);
+    __syncthreads();  // L is used again
+    return cfma(ea, in, eb);
+}
+
+template <int PER>
+__global__ __launch_bounds__(1024) void k_cn_scan(double2* __restrict__ orb, int grid, int bounds,
+                                                  const double2* __restrict__ lu, double2 vm, double2 iv,
+                                                  double2 rhs_up, double2 rhs_lo, double2 rhs_mid) {
+    __shared__ CnScanLds L;
+    double2* f = orb + (size_t) blockIdx.x * grid;
     const bool cyc = bounds != kZeroBounds;
-    const int m = cyc ? n - 1 : n;
-    double2* S = scratch + (size_t) k * 10 * grid;
-    double2* X[5] = {S, S + m, S + 2 * m, S + 3 * m, S + 4 * m};              // a, b, c, d, e
-    double2* Y[5] = {S + 5 * m, S + 6 * m, S + 7 * m, S + 8 * m, S + 9 * m};  // next step
+    const int m = cyc ? grid - 1 : grid, i0 = threadIdx.x * PER;
     const double2 zero = make_double2(0, 0);
-    // Sherman-Morrison split of the corners: beta = up[m-1] couples row 0 to
-    // x_{m-1}, alpha = lo[m-1] row m-1 to x_0
-    const double2 gam = make_double2(-mid0[0].x, -mid0[0].y);
-    const double2 alpha = cyc ? lo[m - 1] : zero, beta = cyc ? up[m - 1] : zero;
-    for (int i = threadIdx.x; i < m; i += blockDim.x) {
-        double2 r;  // right-hand side (split_linear_orbitals.c:288-333)
-        if (i == 0) {
-            r = cmul(rhs_mid, f[0]) + cmul(rhs_up, f[1]);
-            if (cyc) r = r + cmul(rhs_lo, f[n - 2]);
-        } else if (cyc && i == n - 2) {
-            r = cmul(rhs_mid, f[n - 2]) + cmul(rhs_up, f[0]) + cmul(rhs_lo, f[n - 3]);
-        } else if (!cyc && i == n - 1) {
-            r = cmul(rhs_mid, f[n - 1]) + cmul(rhs_lo, f[n - 2]);
-        } else {
-            r = cmul(rhs_mid, f[i]) + cmul(rhs_up, f[i + 1]) + cmul(rhs_lo, f[i - 1]);
-        }
-        double2 b = mid0[i];
-        if (cyc && i == 0) b = b - gam;
-        if (cyc && i == m - 1) b = b - cdiv(cmul(alpha, beta), gam);
-        X[0][i] = i >= 1 ? lo[i - 1] : zero;
-        X[1][i] = b;
-        X[2][i] = i <= m - 2 ? up[i] : zero;
-        X[3][i] = r;
-        X[4][i] = (cyc && i == 0) ? gam : ((cyc && i == m - 1) ? alpha : zero);
-    }
-    __syncthreads();
-    const int nrhs = cyc ? 2 : 1;
-    for (int s = 1; s < m; s *= 2) {
-        for (int i = threadIdx.x; i < m; i += blockDim.x) {
-            const int im = i - s, ip = i + s;
-            const double2 ai = X[0][i], ci = X[2][i];
-            double2 bn = X[1][i], an = zero, cn2 = zero, dn = X[3][i], en = nrhs > 1 ? X[4][i] : zero;
-            if (im >= 0) {
-                const double2 al = cdiv(make_double2(-ai.x, -ai.y), X[1][im]);
-                an = cmul(al, X[0][im]);
-                bn = bn + cmul(al, X[2][im]);
-                dn = dn + cmul(al, X[3][im]);
-                if (nrhs > 1) en = en + cmul(al, X[4][im]);
-            }
-            if (ip < m) {
-                const double2 ga = cdiv(make_double2(-ci.x, -ci.y), X[1][ip]);
-                cn2 = cmul(ga, X[2][ip]);
-                bn = bn + cmul(ga, X[0][ip]);
-                dn = dn + cmul(ga, X[3][ip]);
-                if (nrhs > 1) en = en + cmul(ga, X[4][ip]);
-            }
-            Y[0][i] = an;
-            Y[1][i] = bn;
-            Y[2][i] = cn2;
-            Y[3][i] = dn;
-            Y[4][i] = en;
-        }
-        __syncthreads();
+    auto at = [&](int i) {  // f with the bounds of the operator
+        if (i < 0) return cyc ? f[m - 1] : zero;
+        if (i >= m) return cyc && i == m ? f[0] : zero;
+        return f[i];
+    };
+    double2 v[PER], l[PER], iu[PER], cu[PER];
+    double2 A = make_double2(1, 0), B = zero;
+    double2 fm = at(i0 - 1), fc = at(i0);
 #pragma unroll
-        for (int t = 0; t < 5; t++) {
-            double2* sw = X[t];
-            X[t] = Y[t];
-            Y[t] = sw;
-        }
+    for (int r = 0; r < PER; r++) {
+        const int i = i0 + r;
+        const double2 fp = at(i + 1);
+        const bool in = i < m;
+        v[r] = in ? cmul(rhs_mid, fc) + cmul(rhs_up, fp) + cmul(rhs_lo, fm) : zero;
+        l[r] = in ? lu[i] : zero;
+        iu[r] = in ? lu[grid + i] : zero;
+        cu[r] = in ? lu[2 * grid + i] : zero;
+        B = v[r] - cmul(l[r], B);
+        A = cmul(make_double2(-l[r].x, -l[r].y), A);
+        fm = fc;
+        fc = fp;
     }
-    // every row decoupled: y = d / b, z = e / b
-    for (int i = threadIdx.x; i < m; i += blockDim.x) {
-        const double2 b = X[1][i];
-        Y[3][i] = cdiv(X[3][i], b);
-        if (cyc) Y[4][i] = cdiv(X[4][i], b);
+    double2 prev = cn_scan<true>(A, B, L);
+    A = make_double2(1, 0);
+    B = zero;
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        prev = v[r] - cmul(l[r], prev);
+        v[r] = cmul(iu[r], prev);
     }
-    __syncthreads();
+#pragma unroll
+    for (int r = PER - 1; r >= 0; r--) {
+        B = v[r] - cmul(cu[r], B);
+        A = cmul(make_double2(-cu[r].x, -cu[r].y), A);
+    }
+    double2 next = cn_scan<false>(A, B, L);
+#pragma unroll
+    for (int r = PER - 1; r >= 0; r--) {
+        next = v[r] - cmul(cu[r], next);
+        v[r] = next;
+    }
     double2 fac = zero;
     if (cyc) {
         // x = y - (v.y / (1 + v.z)) z with v = (1, 0, ..., beta / gamma)
-        const double2 vm = cdiv(beta, gam);
-        const double2 vy = Y[3][0] + cmul(vm, Y[3][m - 1]);
-        const double2 vz = Y[4][0] + cmul(vm, Y[4][m - 1]);
-        fac = cdiv(vy, make_double2(1.0 + vz.x, vz.y));
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+            if (i0 + r == 0) L.y0 = v[r];
+            if (i0 + r == m - 1) L.ym = v[r];
+        }
+        __syncthreads();
+        fac = cmul(L.y0 + cmul(vm, L.ym), iv);
     }
-    for (int i = threadIdx.x; i < m; i += blockDim.x) f[i] = cyc ? Y[3][i] - cmul(fac, Y[4][i]) : Y[3][i];
-    if (cyc && threadIdx.x == 0) f[m] = Y[3][0] - cmul(fac, Y[4][0]);
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int i = i0 + r;
+        if (i >= m) continue;
+        const double2 x = cyc ? v[r] - cmul(fac, lu[3 * grid + i]) : v[r];
+        f[i] = x;
+        if (cyc && i == 0) f[m] = x;
+    }
 }
 
 int linear_cn(OrbWork* w, double2* orb, hipStream_t st) {
@@ -394,9 +416,18 @@ int linear_cn(OrbWork* w, double2* orb, hipStream_t st) {
     const double2 a1dt = cscale(cmul(q.d1coef, dt), 1.0 / dx / 4);
     const double2 up = cscale(a2dt, 0.5) + a1dt, lo = cscale(a2dt, 0.5) - a1dt;
     const double2 mid = make_double2(-a2dt.x, 1.0 - a2dt.y);
-    if (w->cn_pcr)
-        k_cn_pcr<<<q.norb, kCnPcrBlock, 0, st>>>(orb, q.grid_size, q.bounds, w->d_cn, up, lo, mid, w->d_cnwork);
-    else
+    if (w->d_cnlu) {
+        // up to four rows per thread
+        const int m = q.bounds != kZeroBounds ? q.grid_size - 1 : q.grid_size;
+        const int t = m <= 1024 ? 256 : (m <= 2048 ? 512 : 1024);
+#define SCAN(per) \
+    k_cn_scan<per><<<q.norb, t, 0, st>>>(orb, q.grid_size, q.bounds, w->d_cnlu, w->cn_vm, w->cn_iv, up, lo, mid)
+        if (m <= t) SCAN(1);
+        else if (m <= 2 * t) SCAN(2);
+        else if (m <= 4 * t) SCAN(4);
+        else SCAN(8);
+#undef SCAN
+    } else
         k_cn_sequential<<<div_up(q.norb, 64), 64, 0, st>>>(orb, q.norb, q.grid_size, q.bounds, w->d_cn, up, lo, mid,
                                                            w->d_cnwork);
     MCTDHB_HIP_CHECK(hipGetLastError());
@@ -1060,16 +1091,171 @@ static int rk_tableau(OrbWork* w, int ns, const double* A, const double* b, doub
 
 // --------------------------------------------------------- Gram-Schmidt
 
-// One block.  The reference (calculus.c:170-191) renormalises F_0, then for
-// i >= 1 projects F_i point by point on each F_j, j < i, and renormalises
-// it.  Its quirk: the coefficient at point p is S_p = <F_j, F_i> evaluated
-// after points < p were updated, and S_{p+1} = S_p (1 - w_p |F_j[p]|^2), so
+// The reference (calculus.c:170-191) renormalises F_0, then for i >= 1
+// projects F_i point by point on each F_j, j < i, and renormalises it.  Its
+// quirk: the coefficient at point p is S_p = <F_j, F_i> evaluated after points
+// < p were updated, and S_{p+1} = S_p (1 - w_p |F_j[p]|^2), so
 // S_p = S_0 prod_{q<p} (1 - w_q |F_j[q]|^2).  The prefix products depend on
-// F_j alone, so the loop runs j-major: finish F_j (renormalise), form its
-// prefix products once, then project every later F_i on it (each F_i still
-// sees its projections in the order j = 0, 1, ..., i - 1).  Thread t owns
-// the points [t per, (t + 1) per): it alone reads and writes them, so the
-// only barriers are those of the block sums (double-buffered, one each).
+// F_j alone.
+//
+// Up to 8 orbitals: one block, every thread holding PER consecutive points of
+// all orbitals in registers.  Step j takes <F_j, F_j> and every <F_j, F_i>,
+// i > j, in one block sum (the normalisation of F_j is applied to the sums),
+// one product scan for the prefix products, and projects all later F_i.  What
+// bounds it is the latency of those M sums and M - 1 scans, two barriers each;
+// one sum per pair (i, j) over orbitals in LDS took 16.0 us at M = 4 on 257
+// points and 36.7 us at M = 5 on 801, this form 7.1 and 11.4 us.
+constexpr int kGsMaxOrb = 8;
+// Threads and points per thread for n grid points: at most 3 points, except
+// on the longest grids.
+struct GsShape {
+    int threads, per;
+};
+__host__ __device__ inline GsShape gs_shape(int n) {
+    const int t = n <= 768 ? 256 : (n <= 1536 ? 512 : 1024);
+    return {t, n <= t ? 1 : (n <= 2 * t ? 2 : (n <= 3 * t ? 3 : 5))};
+}
+inline bool gs_in_registers(int M, int n) { return M <= kGsMaxOrb && n <= 5 * 1024; }
+
+// Inclusive product over the lanes of the wave (fixed order).
+__device__ __forceinline__ double wave_prefix_product(double v) {
+    const int lane = threadIdx.x & 63;
+    for (int off = 1; off < 64; off <<= 1) {
+        const double o = __shfl_up(v, off, 64);
+        if (lane >= off) v *= o;
+    }
+    return v;
+}
+
+struct GsLds {
+    double part[2 * kGsMaxOrb][16];  // sums per wave
+    double tot[2 * kGsMaxOrb];
+    double prod[16];
+};
+
+// Every thread of the block calls it; threads past `threads` only keep the
+// barriers.
+template <int M, int PER>
+__device__ __forceinline__ void gram_schmidt_points(GsLds& L, double2* __restrict__ F, int n, double dx, int tail,
+                                                    int threads) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = threads >> 6;
+    const bool works = t < threads;
+    double2 f[M][PER];
+    double w[PER];
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int p = t * PER + r;
+        const bool in = works && p < n;
+        w[r] = in ? simpson_w(p, n, dx) : 0.0;
+#pragma unroll
+        for (int k = 0; k < M; k++) f[k][r] = in ? F[(size_t) k * n + p] : make_double2(0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        constexpr int NV = 2 * M;
+        double v[NV];
+#pragma unroll
+        for (int i = 0; i < NV; i++) v[i] = 0;
+        double wa[PER];  // w |F_j|^2
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+            wa[r] = w[r] * (f[j][r].x * f[j][r].x + f[j][r].y * f[j][r].y);
+            v[0] += wa[r];
+#pragma unroll
+            for (int i = j + 1; i < M; i++) {
+                const double2 z = cconjmul(f[j][r], f[i][r]);
+                v[2 * (i - j) - 1] += w[r] * z.x;
+                v[2 * (i - j)] += w[r] * z.y;
+            }
+        }
+        if (works) {
+#pragma unroll
+            for (int i = 0; i <= 2 * (M - 1 - j); i++) {
+                const double x = wave_sum(v[i]);
+                if (lane == 0) L.part[i][wave] = x;
+            }
+        }
+        __syncthreads();
+        if (t <= 2 * (M - 1 - j)) {
+            double x = 0;
+            for (int u = 0; u < nw; u++) x += L.part[t][u];
+            L.tot[t] = x;
+        }
+        __syncthreads();
+        const double nr = L.tot[0], sc2 = 1.0 / nr, sc = sqrt(sc2);
+        if (j < M - 1) {
+            // product of (1 - w_q |F_j[q]|^2) over the points before this thread's first
+            double prod = 1.0;
+#pragma unroll
+            for (int r = 0; r < PER; r++) prod *= 1.0 - wa[r] * sc2;
+            const double incl = works ? wave_prefix_product(prod) : 1.0;
+            if (works && lane == 63) L.prod[wave] = incl;
+            double run = __shfl_up(incl, 1, 64);
+            if (lane == 0) run = 1.0;
+            __syncthreads();
+            if (works)
+                for (int u = 0; u < wave; u++) run *= L.prod[u];
+#pragma unroll
+            for (int r = 0; r < PER; r++) {
+                // F_i -= S_0 run F_j / |F_j|, S_0 = <F_j, F_i> / |F_j|
+                const double2 q = cscale(f[j][r], run * sc2);
+#pragma unroll
+                for (int i = j + 1; i < M; i++)
+                    f[i][r] = f[i][r] - cmul(make_double2(L.tot[2 * (i - j) - 1], L.tot[2 * (i - j)]), q);
+                run *= 1.0 - wa[r] * sc2;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+            const int p = t * PER + r;
+            const double2 z = cscale(f[j][r], sc);
+            if (works && p < n && !(tail && p == n - 1)) F[(size_t) j * n + p] = z;
+            if (tail && p == 0) F[(size_t) j * n + n - 1] = z;  // the periodic copy
+        }
+    }
+}
+
+template <int M>
+__device__ __forceinline__ void gram_schmidt_any(GsLds& L, double2* __restrict__ F, int n, double dx, int tail) {
+    const GsShape s = gs_shape(n);
+    switch (s.per) {
+        case 1: gram_schmidt_points<M, 1>(L, F, n, dx, tail, s.threads); break;
+        case 2: gram_schmidt_points<M, 2>(L, F, n, dx, tail, s.threads); break;
+        case 3: gram_schmidt_points<M, 3>(L, F, n, dx, tail, s.threads); break;
+        default: gram_schmidt_points<M, 5>(L, F, n, dx, tail, s.threads); break;
+    }
+}
+
+template <int M>
+__global__ __launch_bounds__(1024) void k_gram_schmidt(double2* __restrict__ F, int n, double dx, int tail) {
+    __shared__ GsLds L;
+    gram_schmidt_any<M>(L, F, n, dx, tail);
+}
+
+// Packed form: one block per instance, as wide as the widest of them needs.
+template <int M> __global__ __launch_bounds__(1024) void k_gram_schmidt_pk(const PkGs* __restrict__ tab) {
+    __shared__ GsLds L;
+    const PkGs a = tab[blockIdx.x];
+    gram_schmidt_any<M>(L, a.F, a.n, a.dx, a.tail);
+}
+
+int pk_gram_schmidt(const PkGs* tab, int count, int M, int threads, hipStream_t st) {
+    switch (M) {
+#define CASE(m) \
+    case m: k_gram_schmidt_pk<m><<<count, threads, 0, st>>>(tab); break;
+        CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
+#undef CASE
+        default: set_error("packed Gram-Schmidt covers 2 <= norb <= 7"); return kInvalidArgument;
+    }
+    MCTDHB_HIP_CHECK(hipGetLastError());
+    return kOk;
+}
+int pk_gs_threads(int n) { return gs_shape(n).threads; }
+
+// More orbitals (or a longer grid): one block, the orbitals in LDS where they
+// fit, j-major with one block sum per pair.  Thread t owns the points
+// [t per, (t + 1) per): it alone reads and writes them, so the only barriers
+// are those of the block sums (double-buffered, one each).
 __device__ __forceinline__ void gram_schmidt_block(double2* __restrict__ F, int M, int n, double dx) {
     __shared__ double red[2][16];
     __shared__ double wave_prod[4];
@@ -1165,35 +1351,28 @@ __device__ __forceinline__ void gram_schmidt_whole(double2* Fs, double2* __restr
     }
 }
 
-__global__ __launch_bounds__(256) void k_gram_schmidt(double2* __restrict__ Fg, int M, int n, double dx, int tail,
-                                                      int staged) {
+__global__ __launch_bounds__(256) void k_gram_schmidt_many(double2* __restrict__ Fg, int M, int n, double dx,
+                                                           int tail, int staged) {
     extern __shared__ double2 Fs[];
     gram_schmidt_whole(Fs, Fg, M, n, dx, tail, staged);
 }
 
-// Packed form: one block per instance.
-__global__ __launch_bounds__(256) void k_gram_schmidt_pk(const PkGs* __restrict__ tab, int M) {
-    extern __shared__ double2 Fs[];
-    const PkGs a = tab[blockIdx.x];
-    gram_schmidt_whole(Fs, a.F, M, a.n, a.dx, a.tail, a.staged);
-}
-
-int pk_gram_schmidt(const PkGs* tab, int count, int M, size_t smem, hipStream_t st) {
-    k_gram_schmidt_pk<<<count, 256, smem, st>>>(tab, M);
-    MCTDHB_HIP_CHECK(hipGetLastError());
-    return kOk;
-}
-
-size_t pk_gs_smem(int M, int n) {
-    const size_t bytes = sizeof(double2) * M * n;
-    return bytes <= kGsStageBytes ? bytes : 0;
-}
-
 int orthonormalize(OrbWork* w, double2* orb, hipStream_t st, bool periodic_tail) {
-    const size_t bytes = sizeof(double2) * w->eq.norb * w->eq.grid_size;
-    const bool staged = bytes <= kGsStageBytes;
-    k_gram_schmidt<<<1, 256, staged ? bytes : 0, st>>>(orb, w->eq.norb, w->eq.grid_size, w->eq.dx,
-                                                       periodic_tail ? 1 : 0, staged ? 1 : 0);
+    const int M = w->eq.norb, n = w->eq.grid_size, tail = periodic_tail ? 1 : 0;
+    if (gs_in_registers(M, n)) {
+        switch (M) {
+#define CASE(m)                                                                                \
+    case m:                                                                                    \
+        k_gram_schmidt<m><<<1, gs_shape(n).threads, 0, st>>>(orb, n, w->eq.dx, tail); \
+        break;
+            CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+#undef CASE
+        }
+    } else {
+        const size_t bytes = sizeof(double2) * M * n;
+        const bool staged = bytes <= kGsStageBytes;
+        k_gram_schmidt_many<<<1, 256, staged ? bytes : 0, st>>>(orb, M, n, w->eq.dx, tail, staged ? 1 : 0);
+    }
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
 }
@@ -1713,6 +1892,42 @@ int density_sync_small(int norb, double2* rho1, double2* rinv, double* eigvals, 
 
 // ------------------------------------------------------------- set-up
 
+// The factors of k_cn_scan from the CN rows (upper | lower | mid), in long
+// double and rounded once: L | IU | CU | correction vector z of the cyclic
+// system, `grid` entries each; vm = beta / gamma, iv = 1 / (1 + v.z).
+static void cn_factor(const std::vector<double2>& cn, int grid, int bounds, std::vector<double2>& lu, double2& vm,
+                      double2& iv) {
+    using C = std::complex<long double>;
+    const bool cyc = bounds != kZeroBounds;
+    const int m = cyc ? grid - 1 : grid;
+    auto get = [&](int part, int i) { return C(cn[(size_t) part * grid + i].x, cn[(size_t) part * grid + i].y); };
+    auto put = [&](int part, int i, C v) { lu[(size_t) part * grid + i] = make_double2((double) v.real(), (double) v.imag()); };
+    lu.assign(4 * (size_t) grid, make_double2(0, 0));
+    const C gam = -get(2, 0), beta = cyc ? get(0, m - 1) : C(0), alpha = cyc ? get(1, m - 1) : C(0);
+    std::vector<C> u(m), cu(m), z(m);
+    for (int i = 0; i < m; i++) {
+        C b = get(2, i);
+        if (cyc && i == 0) b -= gam;
+        if (cyc && i == m - 1) b -= alpha * beta / gam;
+        const C l = i ? get(1, i - 1) / u[i - 1] : C(0);
+        u[i] = i ? b - l * get(0, i - 1) : b;
+        cu[i] = i < m - 1 ? get(0, i) / u[i] : C(0);
+        z[i] = (i == 0 ? gam : (i == m - 1 ? alpha : C(0))) - (i ? l * z[i - 1] : C(0));
+        put(0, i, l);
+        put(1, i, C(1) / u[i]);
+        put(2, i, cu[i]);
+    }
+    vm = iv = make_double2(0, 0);
+    if (!cyc) return;
+    for (int i = m - 1; i >= 0; i--) {
+        z[i] = z[i] / u[i] - (i < m - 1 ? cu[i] * z[i + 1] : C(0));
+        put(3, i, z[i]);
+    }
+    const C v = beta / gam, inv = C(1) / (C(1) + z[0] + v * z[m - 1]);
+    vm = make_double2((double) v.real(), (double) v.imag());
+    iv = make_double2((double) inv.real(), (double) inv.imag());
+}
+
 int orbwork_create(const OrbEq& eq, int imagtime, const double* pot_host, OrbWork** out) {
     *out = nullptr;
     if (eq.norb < 1 || eq.norb > 30 || eq.grid_size < 6) {
@@ -1791,10 +2006,19 @@ int orbwork_create(const OrbEq& eq, int imagtime, const double* pot_host, OrbWor
     MCTDHB_HIP_CHECK(hipMemcpy(w->d_cn, cn.data(), sizeof(double2) * 3 * grid, hipMemcpyHostToDevice));
     // the parallel CN solve needs a nonzero first diagonal (its cyclic split
     // divides by it; the reference's reduced system for mid[0] == 0 stays on
-    // the sequential sweep) and at most two rows per thread
+    // the sequential sweep)
     {
         const double2 m0 = cn[2 * (size_t) grid];
-        w->cn_pcr = (m0.x != 0 || m0.y != 0) && grid >= 4 && grid <= kCnPcrMaxRows + 1 ? 1 : 0;
+        if ((m0.x != 0 || m0.y != 0) && grid >= 4) {
+            std::vector<double2> lu;
+            cn_factor(cn, grid, eq.bounds, lu, w->cn_vm, w->cn_iv);
+            if (hipMalloc((void**) &w->d_cnlu, sizeof(double2) * lu.size()) != hipSuccess) {
+                orbwork_destroy(w);
+                set_error("device allocation failed for the orbital workspace");
+                return kOutOfMemory;
+            }
+            MCTDHB_HIP_CHECK(hipMemcpy(w->d_cnlu, lu.data(), sizeof(double2) * lu.size(), hipMemcpyHostToDevice));
+        }
     }
     // spectral symbol of the linear part: i freq d1 - freq^2 d2 (split_linear_orbitals.c:275-278)
     std::vector<double2> sym(n);
@@ -1826,6 +2050,7 @@ void orbwork_destroy(OrbWork* w) {
     hipFree(w->d_stage);
     hipFree(w->d_red);
     hipFree(w->d_cnwork);
+    hipFree(w->d_cnlu);
     hipFree(w->d_nl);
     hipFree(w->d_fsH);
     hipFree(w->d_fsmat);

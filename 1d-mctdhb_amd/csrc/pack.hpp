@@ -67,7 +67,7 @@ struct PkNl {
 struct PkGs {
     double2* F;
     double dx;
-    int n, tail, staged;
+    int n, tail;
 };
 
 // FP64 coefficient block of the fused H.C row: one block.
@@ -113,12 +113,12 @@ int pk_nl_coef(const PkNlCoef* tab, int count, int M, hipStream_t st);
 int pk_nl_rk(const PkNl* tab, int count, int M, int ns, unsigned max_blocks, hipStream_t st);
 // Whether the RK kernel forms the nonlinear tables itself (no pk_nl_coef).
 bool pk_nl_folds(int M, int ns);
-int pk_gram_schmidt(const PkGs* tab, int count, int M, size_t smem, hipStream_t st);
+// threads: the largest pk_gs_threads of the instances
+int pk_gram_schmidt(const PkGs* tab, int count, int M, int threads, hipStream_t st);
+int pk_gs_threads(int n);
 int pk_hc_coefficients(const PkCf* tab, int count, int M, hipStream_t st);
 int pk_sil_small(const PkSil* tab, int count, int M, int index, bool stage, size_t smem, hipStream_t st);
 int pk_density(const PkDm* tab, int count, int M, unsigned max_nb, size_t smem, hipStream_t st);
-// LDS of the Gram-Schmidt block: the staged orbitals, or 0 (not staged).
-size_t pk_gs_smem(int M, int n);
 int pk_dm_finish(const PkDmFin* tab, int count, int M, hipStream_t st);
 
 }  // namespace mctdhb
