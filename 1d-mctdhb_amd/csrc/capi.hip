@@ -697,8 +697,7 @@ extern "C" int mctdhb_step_graph_destroy(mctdhb_step_graph* g) {
 // launches over its argument tables.
 
 struct PackGroup {
-    int M = 0, ns = 0, imagtime = 0, index = 0, fold = 0;
-    bool stage = false;
+    int M = 0, ns = 0, imagtime = 0, fold = 0, form = 0;
     int count = 0;
     void* d_tab = nullptr;  // every stage table, one allocation
     size_t fft_smem = 0, sil_smem = 0, dm_smem = 0;
@@ -768,8 +767,8 @@ static int pack_enqueue(const PackGroup& g, PkFft* fft, PkOm* om, PkNlCoef* nlc,
     if (!rc) rc = pk_linear_fft(fft, g.count, g.M, g.fft_smem, st);
     if (!rc && g.imagtime) rc = pk_gram_schmidt(gs, g.count, g.M, g.gs_threads, st);
     if (!rc) rc = pk_orbital_matrices(om, g.count, g.M, st);
-    if (!rc) rc = pk_hc_coefficients(cf, g.count, g.M, st);
-    if (!rc) rc = pk_sil_small(sil, g.count, g.M, g.index, g.stage, g.sil_smem, st);
+    if (!rc) rc = pk_pair_matrix(cf, g.count, g.M, st);
+    if (!rc) rc = pk_sil_small(sil, g.count, g.M, g.form, g.sil_smem, st);
     if (!rc) rc = pk_density(dm, g.count, g.M, g.dm_grid, g.dm_smem, st);
     if (!rc) rc = pk_dm_finish(fin, g.count, g.M, st);
     return rc;
@@ -812,21 +811,17 @@ extern "C" int mctdhb_pack_create(int n, mctdhb_space* const* spaces, mctdhb_sil
     std::vector<PackGroup> groups;
     for (int i = 0; i < n; i++) {
         const Space* S = spaces[i]->S;
-        const Sil* L = sils[i]->L;
         const OrbWork* w = orbitals[i]->w;
         PackGroup key;
         key.M = S->norb;
         key.ns = pack_rk_stages(w->rk_order);
         key.imagtime = w->imagtime ? 1 : 0;
-        key.index = L->index;
-        key.stage = sil_small_stage(S);
+        key.form = sil_small_form(S, sils[i]->L->lm);
         key.fold = pk_nl_folds(key.M, key.ns) ? 1 : 0;
         size_t gi = 0;
         for (; gi < groups.size(); gi++) {
             const PackGroup& g = groups[gi];
-            if (g.M == key.M && g.ns == key.ns && g.imagtime == key.imagtime && g.index == key.index &&
-                g.stage == key.stage)
-                break;
+            if (g.M == key.M && g.ns == key.ns && g.imagtime == key.imagtime && g.form == key.form) break;
         }
         if (gi == groups.size()) {
             groups.push_back(key);
@@ -873,20 +868,17 @@ extern "C" int mctdhb_pack_create(int n, mctdhb_space* const* spaces, mctdhb_sil
             g.nl_blocks = std::max(g.nl_blocks, div_up((unsigned) q.grid_size, 64u));
             gs[j] = PkGs{o, q.dx, q.grid_size, q.bounds == kPeriodicBounds ? 1 : 0};
             g.gs_threads = std::max(g.gs_threads, pk_gs_threads(q.grid_size));
-            cf[j] = PkCf{h1, h2, L->cf64, S->npar};
+            cf[j] = PkCf{h1, h2, L->X, S->npar};
             SmallSilArgs a{};
             a.st = L->d_st;
             a.w[0] = c;
             for (int k = 1; k < L->lm; k++) a.w[k] = L->w[k];
-            a.out = L->out;
             a.lm = L->lm;
             a.dt_re = q.prop_dt.x;
             a.dt_im = q.prop_dt.y;
             a.imagtime = w->imagtime;
-            const RowCtx ctx = make_row_ctx(S->dim, S->npar, S->d_ht, S->d_map, S->d_mapot, S->d_maptt,
-                                            S->d_strideot, S->d_stridett, S->d_occ8);
-            sil[j] = PkSil{ctx, L->cf64, S->d_W, S->ldw, a};
-            g.sil_smem = std::max(g.sil_smem, sil_small_smem(S) + (g.stage ? sil_small_stage_bytes(S) : 0));
+            sil[j] = PkSil{small_ctx(S, L->X, L->psi_small), a};
+            g.sil_smem = std::max(g.sil_smem, sil_small_lds(S, a.lm, g.form));
             const unsigned nb = dm_plan(S).nb;
             double2* part = dm_partials(S, sp->dm_work);
             dm[j] = PkDm{low_ctx(S), c, S->d_W, part, S->ldw, dm_root_table(S) ? 1 : 0, nb};

@@ -1,5 +1,5 @@
-// h2_m4.hip - two-stage H.C kernels instantiated for M = 4 orbitals.
-#include "hamiltonian_two.hpp"
+// h2_m4.hip - two-stage H.C and one-workgroup SIL kernels instantiated for M = 4 orbitals.
+#include "sil_small.hpp"
 
 namespace mctdhb {
 template struct HcTwo<4>;

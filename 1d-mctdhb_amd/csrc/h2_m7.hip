@@ -1,5 +1,5 @@
-// h2_m7.hip - two-stage H.C kernels instantiated for M = 7 orbitals.
-#include "hamiltonian_two.hpp"
+// h2_m7.hip - two-stage H.C and one-workgroup SIL kernels instantiated for M = 7 orbitals.
+#include "sil_small.hpp"
 
 namespace mctdhb {
 template struct HcTwo<7>;

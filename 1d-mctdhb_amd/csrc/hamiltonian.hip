@@ -10,7 +10,6 @@
 #include "hamiltonian_impl.hpp"
 #include "hc_coef.hpp"
 #include "hamiltonian_window.hpp"
-#include "pack.hpp"
 #include "rowctx.hpp"
 
 #include <map>
@@ -130,18 +129,6 @@ unsigned hc_lanczos_blocks(const Space* S, int prec) {
 __global__ void k_hc_coefficients(int M, int N, const double2* __restrict__ hob, const double2* __restrict__ hint,
                                   double2* __restrict__ cf64, float2* __restrict__ cf32) {
     hc_coefficients_part(blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, M, N, hob, hint, cf64, cf32);
-}
-
-// Packed form (FP64 block only): one block per instance.
-__global__ void k_hc_coefficients_pk(const PkCf* __restrict__ tab, int M) {
-    const PkCf a = tab[blockIdx.x];
-    hc_coefficients_part(threadIdx.x, blockDim.x, M, a.npar, a.hob, a.hint, a.cf64, nullptr);
-}
-
-int pk_hc_coefficients(const PkCf* tab, int count, int M, hipStream_t st) {
-    k_hc_coefficients_pk<<<count, 256, 0, st>>>(tab, M);
-    MCTDHB_HIP_CHECK(hipGetLastError());
-    return kOk;
 }
 
 int hc_coefficients(const Space* S, const double2* hob, const double2* hint, double2* cf64, float2* cf32,
@@ -585,30 +572,6 @@ int hc_apply_cf(const Space* S, const void* coef, const void* cf, void* hc, int 
     if (X && two_stage(S, coef, X, nullptr, nullptr, hc, prec, st, rc)) return rc;
     const void* blk = prec == kPrecFP64 ? cf : (const void*) ((const double2*) cf + cf_size(M));
     return dispatch_fused_plain(S, coef, blk, hc, prec, index, st);
-}
-
-int pk_sil_small(const PkSil* tab, int count, int M, int index, bool stage, size_t smem, hipStream_t st) {
-    switch (M) {
-        case 2: return HcFused<2>::sil_small_pk(tab, count, index, stage, smem, st);
-        case 3: return HcFused<3>::sil_small_pk(tab, count, index, stage, smem, st);
-        case 4: return HcFused<4>::sil_small_pk(tab, count, index, stage, smem, st);
-        case 5: return HcFused<5>::sil_small_pk(tab, count, index, stage, smem, st);
-        case 6: return HcFused<6>::sil_small_pk(tab, count, index, stage, smem, st);
-        case 7: return HcFused<7>::sil_small_pk(tab, count, index, stage, smem, st);
-        default: set_error("the one-workgroup SIL step covers 2 <= norb <= 7"); return kInvalidArgument;
-    }
-}
-
-int hc_sil_small(const Space* S, const double2* cf64, const SmallSilArgs& a, int index, hipStream_t st) {
-    switch (S->norb) {
-        case 2: return HcFused<2>::sil_small(S, cf64, a, index, st);
-        case 3: return HcFused<3>::sil_small(S, cf64, a, index, st);
-        case 4: return HcFused<4>::sil_small(S, cf64, a, index, st);
-        case 5: return HcFused<5>::sil_small(S, cf64, a, index, st);
-        case 6: return HcFused<6>::sil_small(S, cf64, a, index, st);
-        case 7: return HcFused<7>::sil_small(S, cf64, a, index, st);
-        default: set_error("the one-workgroup SIL step covers 2 <= norb <= 7"); return kInvalidArgument;
-    }
 }
 
 int hc_lanczos(const Space* S, const double2* cf64, const float2* cf32, const LanczosHcArgs& a, int prec,

@@ -22,6 +22,7 @@
 #pragma once
 
 #include "pairs.hpp"
+#include "rowctx.hpp"
 #include "sil.hpp"
 #include "space.hpp"
 
@@ -141,44 +142,36 @@ inline bool hc_lanczos_half(const Space* S, int prec) {
 const float2* hc_padded_copy(const Space* S, const float2* c, hipStream_t st);
 
 // The whole FP64 SIL step in one workgroup (sil_small.hpp): w[0] is C
-// (updated in place), w[1..lm-1] Krylov storage, out one more vector.
+// (updated in place), w[1..lm-1] Krylov storage.  Its size limits: with the W
+// table and the roots bounded, the vector H acts on always fits the LDS.
 constexpr uint32_t kSmallSilMaxDim = 8192;
-constexpr int kSmallSilBlock = 512;
-// LDS of that kernel after the W table and the sqrt LUT.
+constexpr size_t kSmallTableBytes = 48896;
+constexpr int kSmallMaxBlock = 1024;
+// LDS of that kernel after the W table and the roots.
 struct SmallSilLds {
-    double red[(2 * kMaxLanczos + 2) * (kSmallSilBlock / 64)];
+    union {
+        double red[(2 * kMaxLanczos + 2) * (kSmallMaxBlock / 64)];
+        double z[64 * (kMaxLanczos + 2)];  // every lane of wave 0 owns a row (odd stride: no bank conflicts)
+    };
     double tot[2 * kMaxLanczos + 4];
-    double z[64 * (kMaxLanczos + 2)];  // every lane of wave 0 owns a row (odd stride: no bank conflicts)
-    double2 cre[kMaxLanczos];
     double2* w[kMaxLanczos];  // the vectors, indexed at run time
     SilState state;           // the scalars during the step, copied out after the eigensolve
 };
-inline size_t sil_small_smem(const Space* S) {
+inline size_t sil_small_tables(const Space* S) {
     const size_t wsz = (size_t) (S->norb - 1) * S->ldw * 4;
-    return ((wsz + 15) & ~(size_t) 15) + ((sizeof(double) * (S->npar + 3) + 15) & ~(size_t) 15) + sizeof(SmallSilLds);
-}
-// The staged form keeps the current vector and the occupation rows in LDS
-// when everything fits in the 160 KiB one workgroup may allocate on gfx950
-// (NC up to about 6000).
-inline size_t sil_small_stage_bytes(const Space* S) { return (size_t) S->dim * (sizeof(double2) + 8); }
-inline bool sil_small_stage(const Space* S) {
-    return sil_small_smem(S) + sil_small_stage_bytes(S) <= kLdsPerWorkgroup;
+    return ((wsz + 15) & ~(size_t) 15) + ((sizeof(double) * (S->npar + 3) + 15) & ~(size_t) 15);
 }
 inline bool sil_small_fits(const Space* S, int lm) {
     return S->norb >= 2 && S->norb <= 7 && S->dim <= kSmallSilMaxDim && lm <= kMaxLanczos &&
-           sil_small_smem(S) <= 64 * 1024;
+           sil_small_tables(S) <= kSmallTableBytes;
 }
 struct SmallSilArgs {
     SilState* st;
     void* w[kMaxLanczos];
-    double2* out;
     int lm;
     double dt_re, dt_im;
     int imagtime;
 };
-int hc_sil_small(const Space* S, const double2* cf64, const SmallSilArgs& a, int index, hipStream_t st);
-
-struct PkSil;
 
 // ------------------------------------------------ two stages (hamiltonian_two.hpp)
 // Elements between the arrays of psi of consecutive pairs, and the bytes of
@@ -208,10 +201,44 @@ int two_lanczos(const Space* S, const double2* X, void* psi, const LanczosHcArgs
 int two_rayleigh(const Space* S, const double2* X, const LanczosHcArgs& a, int prec, hipStream_t st);
 inline unsigned two_rayleigh_blocks(const Space* S) { return div_up(S->low_dim, 256); }
 
+// Where the one-workgroup step keeps things: in LDS the vector H acts on, psi
+// too, and every Krylov vector too; from the last form down, the first that
+// fits the 160 KiB.
+enum SmallForm : int { kSmallStaged = 0, kSmallPsi = 1, kSmallAll = 2 };
+inline size_t sil_small_lds(const Space* S, int lm, int form) {
+    return sil_small_tables(S) + sizeof(SmallSilLds) +
+           sizeof(double2) * ((size_t) S->dim * (form == kSmallAll ? lm : 1) +
+                              (form >= kSmallPsi ? (size_t) pair_count(S->norb) * S->low_dim : 0));
+}
+inline int sil_small_form(const Space* S, int lm) {
+    int f = kSmallAll;
+    while (f > kSmallStaged && sil_small_lds(S, lm, f) > kLdsPerWorkgroup) f--;
+    return f;
+}
+struct SmallSilCtx {
+    RowCtx row;
+    LowCtx low;
+    const double2* X;
+    double2* psi;  // P arrays of ld entries (kSmallStaged)
+    const uint32_t* W;
+    size_t ld;
+    int ldw;
+};
+inline SmallSilCtx small_ctx(const Space* S, const double2* X, double2* psi) {
+    return SmallSilCtx{make_row_ctx(S->dim, S->npar, S->d_ht, S->d_map, S->d_mapot, S->d_maptt, S->d_strideot,
+                                    S->d_stridett, S->d_occ8),
+                       LowCtx{S->d_low, S->low_dim, S->dim, S->npar}, X, psi, S->d_W, two_ld(S), S->ldw};
+}
+int two_small(const Space* S, const double2* X, double2* psi, const SmallSilArgs& a, hipStream_t st);
+struct PkSil;
+
 template <int M> struct HcTwo {
     static int plain(const Space* S, const void* c, const double2* X, void* psi, void* out, int prec, hipStream_t st);
     static int lanczos(const Space* S, const double2* X, void* psi, const LanczosHcArgs& a, int prec, hipStream_t st);
     static int rayleigh(const Space* S, const double2* X, const LanczosHcArgs& a, int prec, hipStream_t st);
+    // the one-workgroup SIL step (sil_small.hpp), of one solve and of count solves (pack.hpp)
+    static int small(const Space* S, const double2* X, double2* psi, const SmallSilArgs& a, hipStream_t st);
+    static int small_pk(const PkSil* tab, int count, int form, size_t smem, hipStream_t st);
 };
 
 // Per-orbital-count entry points of the fused kernel (hc_m<M>.hip).  The
@@ -221,9 +248,6 @@ template <int M> struct HcFused {
     // mixed form with an explicit tiling (0 per lane, 1 pairs, 2 windows; c padded for 1)
     static int plain_tiled(const Space* S, const void* c, const void* cf, void* out, int tiling, hipStream_t st);
     static int lanczos(const Space* S, const void* cf, const LanczosHcArgs& a, int prec, int index, hipStream_t st);
-    static int sil_small(const Space* S, const void* cf, const SmallSilArgs& a, int index, hipStream_t st);
-    // the same step for count instances, one workgroup each (pack.hpp)
-    static int sil_small_pk(const PkSil* tab, int count, int index, bool stage, size_t smem, hipStream_t st);
 };
 
 }  // namespace mctdhb

@@ -16,7 +16,6 @@
 
 #include "hamiltonian_impl.hpp"
 #include "hamiltonian_window.hpp"
-#include "sil_small.hpp"
 
 namespace mctdhb {
 

@@ -2,6 +2,7 @@
 // choice of form and the dispatch over orbital counts.
 #include "hamiltonian_two.hpp"
 #include "hc_coef.hpp"
+#include "pack.hpp"
 
 namespace mctdhb {
 
@@ -20,6 +21,18 @@ __global__ void k_pair_matrix(int M, int N, const double2* __restrict__ hob, con
 int two_matrix(const Space* S, const double2* hob, const double2* hint, double2* X, hipStream_t st) {
     const int P = pair_count(S->norb);
     k_pair_matrix<<<div_up((uint64_t) P * P, 64), 64, 0, st>>>(S->norb, S->npar, hob, hint, X);
+    MCTDHB_HIP_CHECK(hipGetLastError());
+    return kOk;
+}
+
+// Packed form: one block per instance.
+__global__ void k_pair_matrix_pk(const PkCf* __restrict__ tab, int M) {
+    const PkCf a = tab[blockIdx.x];
+    pair_matrix_part(threadIdx.x, blockDim.x, M, a.npar, a.hob, a.hint, a.X);
+}
+
+int pk_pair_matrix(const PkCf* tab, int count, int M, hipStream_t st) {
+    k_pair_matrix_pk<<<count, 256, 0, st>>>(tab, M);
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
 }
@@ -62,6 +75,22 @@ int two_rayleigh(const Space* S, const double2* X, const LanczosHcArgs& a, int p
     DISPATCH(rayleigh(S, X, a, prec, st))
 }
 
+int two_small(const Space* S, const double2* X, double2* psi, const SmallSilArgs& a, hipStream_t st) {
+    DISPATCH(small(S, X, psi, a, st))
+}
+
 #undef DISPATCH
+
+int pk_sil_small(const PkSil* tab, int count, int M, int form, size_t smem, hipStream_t st) {
+    switch (M) {
+        case 2: return HcTwo<2>::small_pk(tab, count, form, smem, st);
+        case 3: return HcTwo<3>::small_pk(tab, count, form, smem, st);
+        case 4: return HcTwo<4>::small_pk(tab, count, form, smem, st);
+        case 5: return HcTwo<5>::small_pk(tab, count, form, smem, st);
+        case 6: return HcTwo<6>::small_pk(tab, count, form, smem, st);
+        case 7: return HcTwo<7>::small_pk(tab, count, form, smem, st);
+        default: set_error("the one-workgroup SIL step covers 2 <= norb <= 7"); return kInvalidArgument;
+    }
+}
 
 }  // namespace mctdhb

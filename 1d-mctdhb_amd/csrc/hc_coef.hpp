@@ -93,10 +93,14 @@ __device__ __forceinline__ double2 pair_element(int M, int k, int s, int q, int 
     return q == l ? G(k, s, q, q) : cscale(G(k, s, q, l), 2.0);
 }
 
-// X (P x P), entries t, t + stride, ...
+// X (P x P; h alone, M x M, for one particle), entries t, t + stride, ...
 __device__ __forceinline__ void pair_matrix_part(int t, int stride, int M, int N, const double2* __restrict__ hob,
                                                  const double2* __restrict__ hint, double2* __restrict__ X) {
     const int P = M * (M + 1) / 2;
+    if (N == 1) {
+        for (int e = t; e < M * M; e += stride) X[e] = hob[e];
+        return;
+    }
     auto pair = [&](int p, int& a, int& b) {
         a = 0;
         while (p >= M - a) p -= M - a++;

@@ -360,9 +360,12 @@ int sil_create(const Space* S, int lm, int prec, int index, Sil** out) {
         *vec = (char*) *base + esz;
         return true;
     };
-    if (!generic && two_possible(S, prec)) ok = ok && hipMalloc((void**) &L->X, two_matrix_bytes(S)) == hipSuccess;
+    if (!generic) ok = ok && hipMalloc((void**) &L->X, two_matrix_bytes(S)) == hipSuccess;
+    L->pairs = !generic && two_possible(S, prec);
+    if (!generic && prec == kPrecFP64 && sil_small_fits(S, lm) && S->low_dim && sil_small_form(S, lm) == kSmallStaged)
+        ok = ok && hipMalloc((void**) &L->psi_small, two_psi_bytes(S, prec)) == hipSuccess;
     // without room for the first stage's values the one-stage kernels run
-    if (ok && L->X && two_chosen(S, prec) && hipMalloc(&L->psi, two_psi_bytes(S, prec)) != hipSuccess) {
+    if (ok && L->pairs && two_chosen(S, prec) && hipMalloc(&L->psi, two_psi_bytes(S, prec)) != hipSuccess) {
         L->psi = nullptr;
         (void) hipGetLastError();
     }
@@ -384,6 +387,7 @@ void sil_destroy(Sil* L) {
     hipFree(L->cf32);
     hipFree(L->X);
     hipFree(L->psi);
+    hipFree(L->psi_small);
     hipFree(L->out);
     hipFree(L->part);
     hipFree(L->tot);
@@ -471,8 +475,8 @@ static int sil_run_lanczos(Sil* L, const double2* C, const double2* hob, const d
         MCTDHB_HIP_CHECK(hipMemcpyAsync(L->cf64 + M * M, hint, sizeof(double2) * M * M * M * M,
                                         hipMemcpyDeviceToDevice, st));
     } else {
-        bg.X = L->X;
-        if (L->X) blocks = div_up(two_matrix_bytes(S) / sizeof(double2), kStreamBlock);
+        bg.X = L->pairs ? L->X : nullptr;
+        if (L->pairs) blocks = div_up(two_matrix_bytes(S) / sizeof(double2), kStreamBlock);
         if (!L->psi) {
             bg.cf64 = L->cf64;
             bg.cf32 = L->cf32;
@@ -499,11 +503,11 @@ static int sil_run_lanczos(Sil* L, const double2* C, const double2* hob, const d
         a.out = L->out;
         a.part = L->part;
         a.last = it == L->lm - 1;
-        if (a.last && L->X) rc = two_rayleigh(S, L->X, a, L->prec, st);
+        if (a.last && L->pairs) rc = two_rayleigh(S, L->X, a, L->prec, st);
         else if (L->psi) rc = two_lanczos(S, L->X, L->psi, a, L->prec, st);
         else rc = hc_lanczos(S, L->cf64, L->cf32, a, L->prec, L->index, st);
         if (rc) return rc;
-        if (a.last && L->X)
+        if (a.last && L->pairs)
             k_reduce_scalars<0><<<1, kReduceBlock, 0, st>>>(L->part, two_rayleigh_blocks(S), L->tot, L->d_st, it,
                                                              2 * it, 2);
         else if (a.last)
@@ -523,18 +527,17 @@ int sil_step(Sil* L, double2* C, const double2* hob, const double2* hint, double
              hipStream_t st) {
     if (L->prec == kPrecFP64 && !L->generic && sil_small_fits(L->S, L->lm) && L->small) {
         // small spaces: the whole step in one workgroup
-        int rc = hc_coefficients(L->S, hob, hint, L->cf64, L->cf32, st);
+        int rc = two_matrix(L->S, hob, hint, L->X, st);
         if (rc) return rc;
         SmallSilArgs a{};
         a.st = L->d_st;
         a.w[0] = C;
         for (int k = 1; k < L->lm; k++) a.w[k] = L->w[k];
-        a.out = L->out;
         a.lm = L->lm;
         a.dt_re = dt_re;
         a.dt_im = dt_im;
         a.imagtime = imagtime;
-        return hc_sil_small(L->S, L->cf64, a, L->index, st);
+        return two_small(L->S, L->X, L->psi_small, a, st);
     }
     int rc = sil_run_lanczos(L, C, hob, hint, st);
     if (rc) return rc;

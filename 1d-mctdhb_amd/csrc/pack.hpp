@@ -8,7 +8,7 @@
 //
 // A pack holds instances that share the stages' template parameters: the
 // orbital count M, the Runge-Kutta stage count and the SIL kernel variant
-// (index scheme, staged vector).  Grid lengths, particle numbers, pointers
+// (SmallForm).  Grid lengths, particle numbers, pointers
 // and step sizes differ per entry; blocks past an instance's own block count
 // return at once.
 #pragma once
@@ -70,20 +70,17 @@ struct PkGs {
     int n, tail;
 };
 
-// FP64 coefficient block of the fused H.C row: one block.
+// Pair matrix of the two-stage H.C: one block.
 struct PkCf {
     const double2* hob;
     const double2* hint;
-    double2* cf64;
+    double2* X;
     int npar;
 };
 
 // One-workgroup SIL step.
 struct PkSil {
-    RowCtx ctx;
-    const double2* cf;
-    const uint32_t* W;
-    int ldw;
+    SmallSilCtx c;
     SmallSilArgs a;
 };
 
@@ -116,8 +113,8 @@ bool pk_nl_folds(int M, int ns);
 // threads: the largest pk_gs_threads of the instances
 int pk_gram_schmidt(const PkGs* tab, int count, int M, int threads, hipStream_t st);
 int pk_gs_threads(int n);
-int pk_hc_coefficients(const PkCf* tab, int count, int M, hipStream_t st);
-int pk_sil_small(const PkSil* tab, int count, int M, int index, bool stage, size_t smem, hipStream_t st);
+int pk_pair_matrix(const PkCf* tab, int count, int M, hipStream_t st);
+int pk_sil_small(const PkSil* tab, int count, int M, int form, size_t smem, hipStream_t st);
 int pk_density(const PkDm* tab, int count, int M, unsigned max_nb, size_t smem, hipStream_t st);
 int pk_dm_finish(const PkDmFin* tab, int count, int M, hipStream_t st);
 

@@ -21,10 +21,13 @@ struct Sil {
     void* wbase[kMaxKrylov] = {};
     void* w0f = nullptr;
     void* w0fbase = nullptr;
-    // the two-stage H.C (when it is the form of this workspace): pair matrix
-    // and first-stage values
+    // Pair matrix (2 <= norb <= 7), whether the pair kernels cover the space,
+    // first-stage values of the two-stage H.C (null: one stage) and of the
+    // one-workgroup step where they do not fit its LDS.
     double2* X = nullptr;
+    bool pairs = false;
     void* psi = nullptr;
+    double2* psi_small = nullptr;
     double2* out = nullptr;
     double* part = nullptr;
     size_t part_cap = 0;
