@@ -53,24 +53,9 @@ __global__ __launch_bounds__(kStreamBlock) void k_sil_begin(SilBegin a) {
         for (uint32_t i = t; i < a.n; i += stride) a.w0[i] = from_d2<float2>(a.C[i]);
 }
 
-// Sum per-block partials (slot-major): tot[t] = sum_b part[t * nblocks + b],
-// one block per slot.
-__global__ __launch_bounds__(256) void k_reduce_slots(const double* __restrict__ part, int nblocks, int nslot,
-                                                      double* __restrict__ tot, const SilState* st) {
-    __shared__ double red[4];
-    if (st && st->stop) return;
-    const int t = blockIdx.x;
-    double v[1] = {0};
-    const double* p = part + (size_t) t * nblocks;
-    for (int b = threadIdx.x; b < nblocks; b += blockDim.x) v[0] += p[b];
-    block_sum<1>(v, red);
-    if (threadIdx.x == 0) tot[t] = v[0];
-}
-
-
-
-// k_reduce_slots over slots slot0 + blockIdx.x, then (in the last block to
-// finish) the scalar update OP of iteration it: 0 = sil_after_hc, 1 =
+// Sums of the per-block partials (slot-major), one block per slot
+// slot0 + blockIdx.x: tot[t] = sum_b part[t * nblocks + b]; then (in the last
+// block to finish) the scalar update OP of iteration it: 0 = sil_after_hc, 1 =
 // sil_after_reorth.  Blocks count themselves in st->arrive (a vector
 // atomic); the last one resets it.
 constexpr int kReduceBlock = 1024;
@@ -293,9 +278,18 @@ __global__ __launch_bounds__(kStreamBlock) void k_sil_recombine(double2* __restr
     if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
 }
 
+// C / |C| from the sums |C|^2 of nb blocks, which every block adds up itself
+// (one launch less; with streaming grids of a row per thread instead of 1024
+// blocks at any size: FP64 step of NC 23,751 133 -> 128 us).
 __global__ __launch_bounds__(kStreamBlock) void k_scale_by_inv_norm(double2* __restrict__ C, uint32_t n,
-                                                                    const double* __restrict__ nrm2) {
-    const double s = 1.0 / sqrt(nrm2[0]);
+                                                                    const double* __restrict__ part, int nb) {
+    __shared__ double red[kStreamBlock / 64], scale;
+    double v[1] = {0};
+    for (int b = threadIdx.x; b < nb; b += kStreamBlock) v[0] += part[b];
+    block_sum<1>(v, red);
+    if (threadIdx.x == 0) scale = 1.0 / sqrt(v[0]);
+    __syncthreads();
+    const double s = scale;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
         C[i] = cscale(C[i], s);
 }
@@ -405,30 +399,35 @@ size_t sil_device_bytes(const Space* S, int lm, int prec) {
     return b;
 }
 
+// Blocks of a streaming pass: a row per thread, at most kStreamGrid.
+static unsigned stream_grid(uint32_t n) { return std::min((unsigned) kStreamGrid, div_up(n, kStreamBlock)); }
+
 template <typename Zw, int NK>
 static void launch_reorth(Sil* L, int it, hipStream_t st) {
     WPtrs wp{};
     for (int k = 0; k <= it; k++) wp.w[k] = L->w[k];
     const int nslot = 2 * NK + 1;
-    k_sil_reorth<Zw, NK><<<kStreamGrid, kStreamBlock, 0, st>>>(L->out, wp, (Zw*) L->w[it + 1], L->S->dim, L->d_st,
-                                                               L->part, nslot);
-    k_reduce_scalars<1><<<nslot, kReduceBlock, 0, st>>>(L->part, kStreamGrid, L->tot, L->d_st, it, 0, 0);
+    const unsigned grid = stream_grid(L->S->dim);
+    k_sil_reorth<Zw, NK><<<grid, kStreamBlock, 0, st>>>(L->out, wp, (Zw*) L->w[it + 1], L->S->dim, L->d_st, L->part,
+                                                        nslot);
+    k_reduce_scalars<1><<<nslot, kReduceBlock, 0, st>>>(L->part, grid, L->tot, L->d_st, it, 0, 0);
 }
 
 template <typename Zw>
 static void recombine_dispatch(Sil* L, double2* C, hipStream_t st) {
+    const unsigned grid = stream_grid(L->S->dim);
     WPtrs wp{};
     for (int k = 0; k < L->lm; k++) wp.w[k] = L->w[k];
     switch (L->lm) {
 #define CASE(K)                                                                                        \
     case K:                                                                                            \
-        k_sil_recombine<Zw, K><<<kStreamGrid, kStreamBlock, 0, st>>>(C, wp, L->S->dim, L->d_st, L->part); \
+        k_sil_recombine<Zw, K><<<grid, kStreamBlock, 0, st>>>(C, wp, L->S->dim, L->d_st, L->part);        \
         break;
         CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12) CASE(13)
         CASE(14) CASE(15)
 #undef CASE
         default:
-            k_sil_recombine_any<Zw><<<kStreamGrid, kStreamBlock, 0, st>>>(C, wp, L->S->dim, L->d_st, L->part);
+            k_sil_recombine_any<Zw><<<grid, kStreamBlock, 0, st>>>(C, wp, L->S->dim, L->d_st, L->part);
             break;
     }
 }
@@ -545,8 +544,8 @@ int sil_step(Sil* L, double2* C, const double2* hob, const double2* hint, double
     if (L->prec == kPrecFP64) recombine_dispatch<double2>(L, C, st);
     else recombine_dispatch<float2>(L, C, st);
     if (imagtime) {
-        k_reduce_slots<<<1, 256, 0, st>>>(L->part, kStreamGrid, 1, L->tot + 48, nullptr);
-        k_scale_by_inv_norm<<<kStreamGrid, kStreamBlock, 0, st>>>(C, L->S->dim, L->tot + 48);
+        const unsigned grid = stream_grid(L->S->dim);
+        k_scale_by_inv_norm<<<grid, kStreamBlock, 0, st>>>(C, L->S->dim, L->part, grid);
     }
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
