@@ -97,8 +97,20 @@ __global__ __launch_bounds__(kReduceBlock) void k_reduce_scalars(const double* _
 
 
 // exp(-i T prop_dt) e_1 (reference coefficients_integration.c:104-145).  One wave.
-__global__ __launch_bounds__(64) void k_sil_tridiag(SilState* st, double dt_re, double dt_im, int renorm) {
-    __shared__ double z[kMaxKrylov * (kMaxKrylov + 1)];
+// nb: blocks of the last iteration's <w, H w> sums still to be added (slot
+// 2 it of part; 0: alpha_it is there).
+__global__ __launch_bounds__(64) void k_sil_tridiag(SilState* st, double dt_re, double dt_im, int renorm,
+                                                    const double* __restrict__ part, int nb, int it) {
+    __shared__ double z[kMaxKrylov * (kMaxKrylov + 1)], tot[2 * kMaxKrylov + 2];
+    if (nb && !st->stop) {
+        double v = 0;
+        for (int b = threadIdx.x; b < nb; b += 64) v += part[(size_t) (2 * it) * nb + b];
+        v = wave_sum(v);
+        if (threadIdx.x == 0) tot[2 * it] = v;
+        __syncthreads();
+        sil_after_hc(st, tot, it, 2, threadIdx.x);
+        __syncthreads();
+    }
     sil_tridiag_wave(st, dt_re, dt_im, z, kMaxKrylov + 1, renorm);
 }
 
@@ -137,16 +149,39 @@ struct WPtrs {
 
 // w_{it+1} = out - sum_{k<=it} cre_k w_k, with partials of <w_k, w_{it+1}>
 // (slots 2k, 2k+1) and |w_{it+1}|^2 (slot 2(it+1)).
+// nbh: blocks of the H.C kernel whose sums hp are still to be added (0: cre is
+// there); every block then adds them and forms cre itself, block 0 keeps
+// alpha (which no other block of this kernel uses).
 template <typename Zw, int NK>
 __global__ __launch_bounds__(kStreamBlock) void k_sil_reorth(const double2* __restrict__ out, WPtrs wp,
                                                              Zw* __restrict__ wnew, uint32_t n,
-                                                             const SilState* __restrict__ st,
-                                                             double* __restrict__ part, int nslot) {
-    __shared__ double red[2 * NK + 1][kStreamBlock / 64];
+                                                             SilState* st, const double* __restrict__ hp, int nbh,
+                                                             double* __restrict__ part) {
+    __shared__ double red[2 * NK + 1][kStreamBlock / 64], tot[2 * NK + 1];
+    __shared__ double2 crl[NK];
     if (st->stop) return;
+    if (nbh) {
+        constexpr int nslot = 2 * NK + (NK == 1), nw = kStreamBlock / 64, per = (nslot + nw - 1) / nw;
+        const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        double v[per];
+#pragma unroll
+        for (int j = 0; j < per; j++) v[j] = 0;
+        for (int b = lane; b < nbh; b += 64) {
+#pragma unroll
+            for (int j = 0; j < per; j++) v[j] += hp[(size_t) min(wid + j * nw, nslot - 1) * nbh + b];
+        }
+#pragma unroll
+        for (int j = 0; j < per; j++) {
+            const double s = wave_sum(v[j]);
+            if (lane == 0 && wid + j * nw < nslot) tot[wid + j * nw] = s;
+        }
+        __syncthreads();
+        if (wid == 0) sil_after_hc(st, tot, NK - 1, 0, lane, crl, blockIdx.x == 0);
+        __syncthreads();
+    }
     double2 cre[NK];
 #pragma unroll
-    for (int k = 0; k < NK; k++) cre[k] = st->cre[k];
+    for (int k = 0; k < NK; k++) cre[k] = nbh ? crl[k] : st->cre[k];
     double acc[2 * NK + 1];
 #pragma unroll
     for (int t = 0; t < 2 * NK + 1; t++) acc[t] = 0;
@@ -402,15 +437,29 @@ size_t sil_device_bytes(const Space* S, int lm, int prec) {
 // Blocks of a streaming pass: a row per thread, at most kStreamGrid.
 static unsigned stream_grid(uint32_t n) { return std::min((unsigned) kStreamGrid, div_up(n, kStreamBlock)); }
 
+// Up to kFoldBlocks blocks of the H.C kernel its sums are added by the kernel
+// that needs them (each block of the reorthogonalisation, the tridiagonal
+// exponential), which saves the launch of a reduction: 4.2 us and a gap against
+// 1.0 to 1.5 us in the reorthogonalisation (NC 23,751, M = 5, FP64: 128.0 ->
+// 114.8 us a step of five vectors; NC 33,649, M = 6, mixed: 14 us of it).  Every
+// block reads all the sums, so past that they cost what the launch does.  (The
+// last block to finish the H.C kernel adding them instead, behind agent-scope
+// fences, made that kernel 5 us longer.)
+constexpr unsigned kFoldBlocks = 512;
+constexpr int kFoldSlots = 2 * kMaxLanczos + 2;
+static_assert(kFoldBlocks * kFoldSlots + kStreamGrid * (2 * kMaxLanczos + 1) <= kStreamGrid * (2 * kMaxKrylov + 2),
+              "both kernels' sums in part_cap");
+
 template <typename Zw, int NK>
-static void launch_reorth(Sil* L, int it, hipStream_t st) {
+static void launch_reorth(Sil* L, int it, unsigned nbh, hipStream_t st) {
     WPtrs wp{};
     for (int k = 0; k <= it; k++) wp.w[k] = L->w[k];
-    const int nslot = 2 * NK + 1;
     const unsigned grid = stream_grid(L->S->dim);
+    // its own sums beside the ones it still reads
+    double* part = L->part + (nbh ? kFoldBlocks * kFoldSlots : 0);
     k_sil_reorth<Zw, NK><<<grid, kStreamBlock, 0, st>>>(L->out, wp, (Zw*) L->w[it + 1], L->S->dim, L->d_st, L->part,
-                                                        nslot);
-    k_reduce_scalars<1><<<nslot, kReduceBlock, 0, st>>>(L->part, grid, L->tot, L->d_st, it, 0, 0);
+                                                        (int) nbh, part);
+    k_reduce_scalars<1><<<2 * NK + 1, kReduceBlock, 0, st>>>(part, grid, L->tot, L->d_st, it, 0, 0);
 }
 
 template <typename Zw>
@@ -433,10 +482,10 @@ static void recombine_dispatch(Sil* L, double2* C, hipStream_t st) {
 }
 
 template <typename Zw>
-static void reorth_dispatch(Sil* L, int it, hipStream_t st) {
+static void reorth_dispatch(Sil* L, int it, unsigned nbh, hipStream_t st) {
     switch (it + 1) {
 #define CASE(K) \
-    case K: launch_reorth<Zw, K>(L, it, st); break;
+    case K: launch_reorth<Zw, K>(L, it, nbh, st); break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12)
         CASE(13) CASE(14)
 #undef CASE
@@ -456,7 +505,10 @@ static void reorth_dispatch(Sil* L, int it, hipStream_t st) {
 }
 
 // Enqueue the Lanczos recursion (lm H.C applications).  C is w_0 (FP64).
-static int sil_run_lanczos(Sil* L, const double2* C, const double2* hob, const double2* hint, hipStream_t st) {
+// left: blocks whose sums of the last iteration are left to the caller's next
+// kernel (null: none are).
+static int sil_run_lanczos(Sil* L, const double2* C, const double2* hob, const double2* hint, hipStream_t st,
+                           unsigned* left = nullptr) {
     const Space* S = L->S;
     const uint32_t n = S->dim;
     int rc;
@@ -506,17 +558,20 @@ static int sil_run_lanczos(Sil* L, const double2* C, const double2* hob, const d
         else if (L->psi) rc = two_lanczos(S, L->X, L->psi, a, L->prec, st);
         else rc = hc_lanczos(S, L->cf64, L->cf32, a, L->prec, L->index, st);
         if (rc) return rc;
-        if (a.last && L->pairs)
+        const bool fold = nbh <= kFoldBlocks && it + 1 < kMaxLanczos;  // the register kernels of reorth_dispatch
+        if (a.last && L->pairs && left && two_rayleigh_blocks(S) <= kFoldBlocks)
+            *left = two_rayleigh_blocks(S);
+        else if (a.last && L->pairs)
             k_reduce_scalars<0><<<1, kReduceBlock, 0, st>>>(L->part, two_rayleigh_blocks(S), L->tot, L->d_st, it,
                                                              2 * it, 2);
         else if (a.last)
             k_reduce_scalars<0><<<2, kReduceBlock, 0, st>>>(L->part, nbh, L->tot, L->d_st, it, 2 * it,
                                                              hc_lanczos_half(S, L->prec) && !L->generic ? 2 : 1);
-        else
+        else if (!fold)
             k_reduce_scalars<0><<<lanczos_hc_slots(it), kReduceBlock, 0, st>>>(L->part, nbh, L->tot, L->d_st, it, 0, 0);
         if (it == L->lm - 1) break;
-        if (L->prec == kPrecFP64) reorth_dispatch<double2>(L, it, st);
-        else reorth_dispatch<float2>(L, it, st);
+        if (L->prec == kPrecFP64) reorth_dispatch<double2>(L, it, fold ? nbh : 0, st);
+        else reorth_dispatch<float2>(L, it, fold ? nbh : 0, st);
     }
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
@@ -538,9 +593,10 @@ int sil_step(Sil* L, double2* C, const double2* hob, const double2* hint, double
         a.imagtime = imagtime;
         return two_small(L->S, L->X, L->psi_small, a, st);
     }
-    int rc = sil_run_lanczos(L, C, hob, hint, st);
+    unsigned left = 0;
+    int rc = sil_run_lanczos(L, C, hob, hint, st, &left);
     if (rc) return rc;
-    k_sil_tridiag<<<1, 64, 0, st>>>(L->d_st, dt_re, dt_im, imagtime ? 1 : 0);
+    k_sil_tridiag<<<1, 64, 0, st>>>(L->d_st, dt_re, dt_im, imagtime ? 1 : 0, L->part, (int) left, L->lm - 1);
     if (L->prec == kPrecFP64) recombine_dispatch<double2>(L, C, st);
     else recombine_dispatch<float2>(L, C, st);
     if (imagtime) {

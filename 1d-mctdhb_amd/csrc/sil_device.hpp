@@ -42,7 +42,8 @@ __device__ inline void sil_init_state(SilState* st, int lm, int t, int T) {
 // On the last iteration only alpha is formed.  last == 2: the H.C pass
 // summed <w_it, H w_it> (the half-row form), and alpha = <v_it, H v_it -
 // beta v_{it-1}> = s_it^2 <w_it, H w_it> - beta conj(<v_{it-1}, v_it>).
-__device__ __forceinline__ void sil_after_hc(SilState* st, const volatile double* tot, int it, int last, int k) {
+__device__ __forceinline__ void sil_after_hc(SilState* st, const volatile double* tot, int it, int last, int k,
+                                             double2* cre, bool keep) {
     if (k > it) return;
     const double2 t = make_double2(tot[2 * it], tot[2 * it + 1]), d = make_double2(tot[2 * k], tot[2 * k + 1]);
     const double nrm0 = it == 0 && !last ? tot[2] : 0.0;  // <v_0, v_0> = |C|^2
@@ -58,14 +59,18 @@ __device__ __forceinline__ void sil_after_hc(SilState* st, const volatile double
             alpha = alpha - make_double2(st->beta[it - 1] * gp.x, -st->beta[it - 1] * gp.y);
         }
     }
-    if (k == 0) {
+    if (k == 0 && keep) {
         st->alpha[it] = alpha;
         if (it == 0) st->gram[0] = gk;
     }
     if (last) return;
     double2 ortho = d - cmul(alpha, gk);
     if (k == it) ortho = ortho + alpha;
-    st->cre[k] = cscale(ortho, sk);
+    cre[k] = cscale(ortho, sk);
+}
+
+__device__ __forceinline__ void sil_after_hc(SilState* st, const volatile double* tot, int it, int last, int k) {
+    sil_after_hc(st, tot, it, last, k, st->cre, true);
 }
 
 // After the streaming pass that produced w_{it+1}: beta_it, the breakdown
