@@ -340,6 +340,11 @@ __global__ __launch_bounds__(kStreamBlock) void k_export_vector(const Zw* __rest
 
 // ------------------------------------------------------------ the driver
 
+// First-stage values of the one-workgroup step outside LDS.
+static bool small_psi_needed(const Space* S, int lm, int prec) {
+    return prec == kPrecFP64 && sil_small_fits(S, lm) && S->low_dim && sil_small_form(S, lm) == kSmallStaged;
+}
+
 int sil_create(const Space* S, int lm, int prec, int index, Sil** out) {
     *out = nullptr;
     if (lm < 2 || lm > kMaxKrylov) {
@@ -391,7 +396,7 @@ int sil_create(const Space* S, int lm, int prec, int index, Sil** out) {
     };
     if (!generic) ok = ok && hipMalloc((void**) &L->X, two_matrix_bytes(S)) == hipSuccess;
     L->pairs = !generic && two_possible(S, prec);
-    if (!generic && prec == kPrecFP64 && sil_small_fits(S, lm) && S->low_dim && sil_small_form(S, lm) == kSmallStaged)
+    if (small_psi_needed(S, lm, prec))
         ok = ok && hipMalloc((void**) &L->psi_small, two_psi_bytes(S, prec)) == hipSuccess;
     // without room for the first stage's values the one-stage kernels run
     if (ok && L->pairs && two_chosen(S, prec) && hipMalloc(&L->psi, two_psi_bytes(S, prec)) != hipSuccess) {
@@ -431,6 +436,7 @@ size_t sil_device_bytes(const Space* S, int lm, int prec) {
     size_t b = (size_t) (lm - 1) * zw * n + sizeof(double2) * n;
     if (prec == kPrecMixed) b += sizeof(float2) * n;
     if (two_faster(S, prec)) b += two_psi_bytes(S, prec);
+    if (small_psi_needed(S, lm, prec)) b += two_psi_bytes(S, prec);
     return b;
 }
 

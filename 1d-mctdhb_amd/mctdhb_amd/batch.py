@@ -74,12 +74,12 @@ DEVICE_DRAW_DIM = 1 << 16
 
 def footprint_bytes(dim: int, norb: int, grid: int, lanczos: int = 5) -> int:
     """Device memory of one instance, upper estimate: coefficients and the
-    Krylov vectors (complex128), the H.C output and, from six orbitals on,
-    its first-stage values (complex128, one per pair of orbitals), occupation
+    Krylov vectors (complex128), the H.C output and, from six orbitals on
+    and for the one-workgroup step, its first-stage values (complex128, one per pair of orbitals), occupation
     rows of N and N - 2 particles, the density partial sums, orbitals with
     their stage and FFT buffers, and a fixed allowance for the small tables
     and matrices."""
-    pairs = norb * (norb + 1) // 2 if norb >= 6 else 0
+    pairs = norb * (norb + 1) // 2 if norb >= 6 or dim <= 8192 else 0
     return dim * (16 * (lanczos + 3 + pairs) + 16) + (dim // 4096 + 2) * 16 * norb ** 4 + 16 * norb * grid * 24 + (1 << 20)
 
 
