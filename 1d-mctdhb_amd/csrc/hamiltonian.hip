@@ -436,6 +436,14 @@ int hc_apply(const Space* S, const void* coef, const double2* hob, const double2
     return rc;
 }
 
+// Prebuilt block: FP64 coefficients | pair matrix | (mixed) complex64 copy.
+// Where the first two stand does not depend on the precision, so a block
+// built for the mixed form serves FP64 products too.
+static size_t block_cf32_off(const Space* S) {
+    return sizeof(double2) * cf_size(S->norb) + (S->d_low ? two_matrix_bytes(S) : 0);
+}
+static const void* block_cf32(const Space* S, const void* cf) { return (const char*) cf + block_cf32_off(S); }
+
 // ------------------------------------------- H.C without device allocation
 // The coefficient block of hc_apply_noalloc lives in this array.  Host code
 // never passes its name to a kernel or a copy: each device's copy of it is
@@ -513,7 +521,7 @@ int hc_apply_noalloc(const Space* S, const void* coef, const double2* hob, const
     // every entry of the block is written here, so nothing needs clearing
     if ((rc = hc_build_coef(S, hob, hint, blk, prec, st))) return rc;
     if (prec == kPrecFP64) return dispatch_fused_plain(S, coef, blk, hc, prec, index, st);
-    const void* cf32 = (const double2*) blk + cf_size(S->norb);
+    const void* cf32 = block_cf32(S, blk);
     if (S->hc_tiling == 1 && S->d_pad) {  // staging already allocated: a device copy only
         const float2* cp = hc_padded_copy(S, (const float2*) coef, st);
         if (!cp) {
@@ -525,19 +533,10 @@ int hc_apply_noalloc(const Space* S, const void* coef, const double2* hob, const
     return dispatch_plain_tiled(S, coef, cf32, hc, 0, st);
 }
 
-// (16-byte aligned: what follows is complex128)
-static size_t hc_one_stage_bytes(int M, int prec) {
-    const size_t b = sizeof(double2) * cf_size(M) + (prec == kPrecMixed ? sizeof(float2) * cf32_size(M) : 0);
-    return (b + 15) & ~(size_t) 15;
-}
-
 size_t hc_coef_bytes(const Space* S, int prec) {
     const int M = S->norb;
     if (use_generic(S)) return sizeof(double2) * ((size_t) M * M + (size_t) M * M * M * M);
-    // FP64 block, the complex64 copy for the mixed form, the pair matrix
-    size_t b = hc_one_stage_bytes(M, prec);
-    if (S->d_low) b += two_matrix_bytes(S);
-    return b;
+    return block_cf32_off(S) + (prec == kPrecMixed ? sizeof(float2) * cf32_size(M) : 0);
 }
 
 int hc_build_coef(const Space* S, const double2* hob, const double2* hint, void* cf, int prec, hipStream_t st) {
@@ -548,11 +547,10 @@ int hc_build_coef(const Space* S, const double2* hob, const double2* hint, void*
                                         hipMemcpyDeviceToDevice, st));
         return kOk;
     }
-    double2* cf64 = (double2*) cf;
-    float2* cf32 = prec == kPrecMixed ? (float2*) (cf64 + cf_size(M)) : nullptr;
-    const int rc = hc_coefficients(S, hob, hint, cf64, cf32, st);
+    float2* cf32 = prec == kPrecMixed ? (float2*) block_cf32(S, cf) : nullptr;
+    const int rc = hc_coefficients(S, hob, hint, (double2*) cf, cf32, st);
     if (rc || !S->d_low) return rc;
-    return two_matrix(S, hob, hint, (double2*) ((char*) cf + hc_one_stage_bytes(M, prec)), st);
+    return two_matrix(S, hob, hint, (double2*) cf + cf_size(M), st);
 }
 
 int hc_apply_cf(const Space* S, const void* coef, const void* cf, void* hc, int prec, int index, hipStream_t st) {
@@ -568,9 +566,9 @@ int hc_apply_cf(const Space* S, const void* coef, const void* cf, void* hc, int 
         return kOk;
     }
     if (prec == kPrecMixed && (rc = hc_tune_tiling(S, st))) return rc;
-    const double2* X = S->d_low ? (const double2*) ((const char*) cf + hc_one_stage_bytes(M, prec)) : nullptr;
+    const double2* X = S->d_low ? (const double2*) cf + cf_size(M) : nullptr;
     if (X && two_stage(S, coef, X, nullptr, nullptr, hc, prec, st, rc)) return rc;
-    const void* blk = prec == kPrecFP64 ? cf : (const void*) ((const double2*) cf + cf_size(M));
+    const void* blk = prec == kPrecFP64 ? cf : block_cf32(S, cf);
     return dispatch_fused_plain(S, coef, blk, hc, prec, index, st);
 }
 

@@ -280,7 +280,8 @@ int mctdhb_apply_hamiltonian_noalloc_dev(const mctdhb_space* space, const void* 
 
 /* The (hob, hint)-derived coefficient block of the H.C kernels, built once
  * and reused across applications with the same one- and two-body matrices.
- * cf must hold mctdhb_hc_coef_bytes(space, prec) bytes of device memory. */
+ * cf must hold mctdhb_hc_coef_bytes(space, prec) bytes of device memory.  A
+ * block built for MIXED serves FP64 products too. */
 size_t mctdhb_hc_coef_bytes(const mctdhb_space* space, int prec);
 int    mctdhb_hc_coefficients_dev(const mctdhb_space* space, const void* hob, const void* hint, void* cf,
                                   int prec, void* stream);

@@ -57,6 +57,21 @@ def test_product_matches_oracle(amd, orc, npar, norb):
     D.close()
 
 
+@pytest.mark.parametrize("npar,norb", [(1, 6), (5, 6), (4, 7), (8, 5)])
+def test_mixed_block_serves_fp64_products(amd, npar, norb):
+    c, h, g = _problem(npar, norb)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    dc, dh, dg = gu.dev(c), gu.dev(h), gu.dev(g)
+    outs = []
+    for built in (amd.FP64, amd.MIXED):
+        cf = gu.empty(D.coef_bytes(built) // 8 + 1, "float64")
+        D.hc_coefficients(dh, dg, cf, prec=built)
+        outs.append(gu.empty(D.dim))
+        D.apply_hamiltonian_cf(dc, cf, outs[-1], prec=amd.FP64)
+    assert np.array_equal(gu.host(outs[0]), gu.host(outs[1]))
+    D.close()
+
+
 @pytest.mark.parametrize("npar,norb", [(5, 6), (4, 7), (9, 6)])
 def test_same_entries_of_h_and_g_as_the_one_stage_kernel(amd, npar, norb):
     c, h, g = _problem(npar, norb, symmetric=False)
