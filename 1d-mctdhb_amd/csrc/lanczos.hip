@@ -551,7 +551,8 @@ static int sil_run_lanczos(Sil* L, const double2* C, const double2* hob, const d
     }
     k_sil_begin<<<blocks, kStreamBlock, 0, st>>>(bg);
     if (L->prec == kPrecMixed && !L->psi && (rc = hc_tune_tiling(S, st))) return rc;
-    const unsigned nbh = hc_lanczos_blocks(S, L->prec);
+    // the blocks of the form that runs: with psi the two-stage one, whatever the space's tiling is by now
+    const unsigned nbh = L->psi ? hc_grid_blocks(S->dim) : hc_lanczos_blocks(S, L->prec);
     for (int it = 0; it < L->lm; it++) {
         LanczosHcArgs a{};
         for (int k = 0; k <= it; k++) a.w[k] = L->w[k];

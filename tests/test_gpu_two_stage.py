@@ -136,3 +136,19 @@ def test_tiling_names_the_form(amd):
         D5.hc_tiling(3)
     D6.close()
     D5.close()
+
+
+def test_open_workspace_keeps_its_form_when_the_tiling_changes(amd, orc):
+    npar, norb, lm = 9, 6, 5
+    c, h, g = _problem(npar, norb)
+    _, ref = orc.Space(npar, norb).sil_step(c, h, g, lm, 0.01, False)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    for made, later in ((3, 1), (3, 0), (1, 3), (0, 1)):
+        D.hc_tiling(made)
+        sil = amd.DeviceSil(D, lm, prec=amd.MIXED, index=amd.INDEX_FLY)
+        D.hc_tiling(later)
+        dc = gu.dev(c)
+        sil.step(dc, gu.dev(h), gu.dev(g), 0.01, False)
+        assert gu.rel_err(gu.host(dc), ref) < 2e-5, (made, later)
+        sil.close()
+    D.close()
