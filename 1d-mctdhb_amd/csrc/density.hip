@@ -308,9 +308,10 @@ __global__ __launch_bounds__(kDmFinishThreads) void k_dm_finish_pk(const PkDmFin
 }
 
 // More partials: one block per element sums them, and the last block to
-// arrive fills.  Blocks count themselves in *arrive (a vector atomic); the
-// last one resets it.  Each block writes one element before it counts, so
-// the release it makes is cheap.
+// arrive fills.  Blocks count themselves in *arrive (a vector atomic), which
+// k_gram has cleared: a count left over from calls that overlapped on one
+// workspace spoils those calls only.  Each block writes one element before it
+// counts, so the release it makes is cheap.
 template <typename Z>
 __global__ __launch_bounds__(256) void k_dm_reduce(int M, int npar, const double2* __restrict__ part, int nb,
                                                    double2* tot, unsigned* arrive, DmOut out) {
@@ -333,7 +334,6 @@ __global__ __launch_bounds__(256) void k_dm_reduce(int M, int npar, const double
     __syncthreads();
     if (!last) return;
     __threadfence();
-    if (threadIdx.x == 0) *arrive = 0;
     for (int t = threadIdx.x; t < (int) gridDim.x; t += blockDim.x) lds[t] = tot[t];
     __syncthreads();
     dm_fill_block<Z>(M, npar, lds, out, lds + gridDim.x);
@@ -362,19 +362,6 @@ int pk_density(const PkDm* tab, int count, int M, unsigned max_nb, size_t smem, 
         case 6: return DmPairs<6>::run_pk(tab, count, max_nb, smem, st);
         case 7: return DmPairs<7>::run_pk(tab, count, max_nb, smem, st);
         default: set_error("packed density kernels cover 2 <= norb <= 7"); return kInvalidArgument;
-    }
-}
-
-static int dispatch_dm(const Space* S, const void* c, int prec, double2* part, const DmPlan& plan, const DmOut& out,
-                       hipStream_t st) {
-    switch (S->norb) {
-        case 2: return DmPairs<2>::run(S, c, prec, part, plan, out, st);
-        case 3: return DmPairs<3>::run(S, c, prec, part, plan, out, st);
-        case 4: return DmPairs<4>::run(S, c, prec, part, plan, out, st);
-        case 5: return DmPairs<5>::run(S, c, prec, part, plan, out, st);
-        case 6: return DmPairs<6>::run(S, c, prec, part, plan, out, st);
-        case 7: return DmPairs<7>::run(S, c, prec, part, plan, out, st);
-        default: set_error("pair density kernels cover 2 <= norb <= 7"); return kInvalidArgument;
     }
 }
 
@@ -438,12 +425,22 @@ static DmWork dm_work(const Space* S, void* base) {
     return w;
 }
 
+static int dispatch_dm(const Space* S, const void* c, int prec, const DmWork& w, const DmPlan& plan, const DmOut& out,
+                       hipStream_t st) {
+    unsigned* arrive = plan.nb > kDmFinishBlocks ? w.arrive : nullptr;
+    switch (S->norb) {
+        case 2: return DmPairs<2>::run(S, c, prec, w.part, arrive, plan, out, st);
+        case 3: return DmPairs<3>::run(S, c, prec, w.part, arrive, plan, out, st);
+        case 4: return DmPairs<4>::run(S, c, prec, w.part, arrive, plan, out, st);
+        case 5: return DmPairs<5>::run(S, c, prec, w.part, arrive, plan, out, st);
+        case 6: return DmPairs<6>::run(S, c, prec, w.part, arrive, plan, out, st);
+        case 7: return DmPairs<7>::run(S, c, prec, w.part, arrive, plan, out, st);
+        default: set_error("pair density kernels cover 2 <= norb <= 7"); return kInvalidArgument;
+    }
+}
+
 int dm_workspace_create(const Space* S, void** work) {
-    const size_t bytes = dm_work(S, nullptr).bytes;
-    MCTDHB_HIP_CHECK(hipMalloc(work, bytes));
-    if (dm_generic(S->norb) || dm_plan(S).nb <= kDmFinishBlocks) return kOk;  // nothing counts
-    MCTDHB_HIP_CHECK(hipMemset(*work, 0, 256));
-    MCTDHB_HIP_CHECK(hipStreamSynchronize(nullptr));  // cleared before any stream counts
+    MCTDHB_HIP_CHECK(hipMalloc(work, dm_work(S, nullptr).bytes));
     return kOk;
 }
 
@@ -488,7 +485,7 @@ int density_matrices(const Space* S, const void* coef, double2* rho1, double2* r
     if (generic) return density_generic(S, coef, rho1, rho2, w, sy, st);
     const DmPlan plan = dm_plan(S);
     const DmOut out{coef, rho1, rho2, sy};
-    const int rc = dispatch_dm(S, coef, prec, w.part, plan, out, st);
+    const int rc = dispatch_dm(S, coef, prec, w, plan, out, st);
     if (rc || plan.nb == 1) return rc;
     const int nb = (int) plan.nb, E = gram_elements(M);
     const size_t smem = dm_finish_lds(M);

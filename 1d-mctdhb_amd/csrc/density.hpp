@@ -17,7 +17,7 @@ constexpr int kDmThreads = 64 * kDmWaves;
 DmPlan dm_plan(const Space* S);
 
 // Scratch of density_matrices (per-block partials, totals and the arrival
-// counter of the last stage): allocated and cleared by dm_workspace_create.
+// counter of the last stage, which the first one clears): one call at a time.
 int dm_workspace_create(const Space* S, void** work);
 // the partial sums in it
 double2* dm_partials(const Space* S, void* work);
@@ -48,8 +48,9 @@ struct DmOut {
 // sums, or with one block everything.
 struct PkDm;
 template <int M> struct DmPairs {
-    static int run(const Space* S, const void* c, int prec, double2* part, const DmPlan& plan, const DmOut& out,
-                   hipStream_t st);
+    // arrive: the counter to clear, where the last stage counts
+    static int run(const Space* S, const void* c, int prec, double2* part, unsigned* arrive, const DmPlan& plan,
+                   const DmOut& out, hipStream_t st);
     // FP64 partials of count instances (pack.hpp); max_nb: their largest plan
     static int run_pk(const PkDm* tab, int count, unsigned max_nb, size_t smem, hipStream_t st);
 };

@@ -268,14 +268,16 @@ __device__ __forceinline__ void gram_block(unsigned char* smem, uint32_t bid, ui
 }
 
 // One block (nb = 1) also fills rho1 and rho2 and synchronises rho1: its sums
-// go to LDS behind those of the waves.
+// go to LDS behind those of the waves.  arrive (may be null): cleared for the
+// last stage.
 template <int M, typename Z>
 __global__ __launch_bounds__(kDmThreads) void k_gram(LowCtx low, const Z* __restrict__ c,
                                                      const uint32_t* __restrict__ Wg, int ldw, int use_sq,
-                                                     double2* part, DmOut out) {
+                                                     double2* part, unsigned* arrive, DmOut out) {
     extern __shared__ __align__(16) unsigned char smem[];
     double2* tot = (double2*) (smem + gram_sum_lds<M>());
     const bool one = gridDim.x == 1;
+    if (arrive && blockIdx.x == 0 && threadIdx.x == 0) *arrive = 0;
     gram_block<M, Z>(smem, xcd_block(blockIdx.x, gridDim.x), gridDim.x, low, c, Wg, ldw, use_sq, one ? tot : part);
     if (one) {
         __syncthreads();
@@ -299,8 +301,8 @@ int DmPairs<M>::run_pk(const PkDm* tab, int count, unsigned max_nb, size_t smem,
 }
 
 template <int M>
-int DmPairs<M>::run(const Space* S, const void* c, int prec, double2* part, const DmPlan& plan, const DmOut& out,
-                    hipStream_t st) {
+int DmPairs<M>::run(const Space* S, const void* c, int prec, double2* part, unsigned* arrive, const DmPlan& plan,
+                    const DmOut& out, hipStream_t st) {
     const size_t smem = dm_pair_smem(S);
     if (!smem) {
         set_error("density kernel LDS budget exceeded for this (N, M)");
@@ -309,10 +311,10 @@ int DmPairs<M>::run(const Space* S, const void* c, int prec, double2* part, cons
     const int use_sq = dm_root_table(S) ? 1 : 0;
     if (prec == kDmMixed)
         k_gram<M, float2><<<plan.nb, kDmThreads, smem, st>>>(low_ctx(S), (const float2*) c, S->d_W, S->ldw, use_sq,
-                                                             part, out);
+                                                             part, arrive, out);
     else
         k_gram<M, double2><<<plan.nb, kDmThreads, smem, st>>>(low_ctx(S), (const double2*) c, S->d_W, S->ldw, use_sq,
-                                                              part, out);
+                                                              part, arrive, out);
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
 }

@@ -304,7 +304,10 @@ int    mctdhb_apply_hamiltonian_cf_dev(const mctdhb_space* space, const void* co
 int mctdhb_hc_tiling(mctdhb_space* space, int set, int* tiling);
 
 /* rho1 (M x M, <a+_k a_l>) and rho2 (M^4, <a+_k a+_s a_q a_l>), complex128;
- * rho2 may be NULL.  coef complex128 (FP64) or complex64 (MIXED). */
+ * rho2 may be NULL.  coef complex128 (FP64) or complex64 (MIXED).  The sums
+ * of a space's density calls (this one, mctdhb_density_sync_dev and the steps)
+ * share one workspace: serialise those that would overlap on one space (other
+ * streams, threads).  Calls on different spaces are independent. */
 int mctdhb_density_dev(mctdhb_space* space, const void* coef, void* rho1, void* rho2, int prec,
                        int index, void* stream);
 
