@@ -348,32 +348,19 @@ static int check_mode(const Space* S, int prec, int index) {
 }
 
 // Scratch of the two-stage product: up to kScratchBlocks blocks kept by the
-// space (freed with it), each with an event behind its last use.  A call takes
-// one that is idle, or a new one, or waits on the stream for the last use of
-// one, so calls on several streams and threads never share a block in flight.
+// space (freed with it), each with an event behind its last use, so calls on
+// several streams and threads never share a block in flight.  A call takes
+// the block its stream used last, one that is idle, a new one, or the one
+// given back longest ago behind an event wait; a block too small for it (of
+// the mixed form) it replaces; and with all of them in other threads' hands,
+// which is while those enqueue, it waits.  So the form of a product does not
+// depend on what else runs: only a capturing stream, whose graph must not
+// keep a block, and a failed allocation take the one-stage kernels.
 // (A stream-ordered allocation per call from a pool that keeps its memory
 // was tried first; now and then it mapped hundreds of MB anew in every call.)
 constexpr size_t kScratchBlocks = 4;
 
-static SpaceScratch* scratch_take(const Space* S, size_t bytes, hipStream_t st) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
-    std::lock_guard<std::mutex> lock(S->scratch_mu);
-    SpaceScratch* pick = nullptr;
-    for (auto& b : S->scratch)
-        if (!b->busy && b->bytes >= bytes && hipEventQuery(b->done) == hipSuccess) {
-            b->busy = true;
-            return b.get();
-        }
-    (void) hipGetLastError();  // hipErrorNotReady of the blocks in flight
-    for (auto& b : S->scratch)
-        if (!b->busy && b->bytes >= bytes && (b->last == st || S->scratch.size() >= kScratchBlocks)) pick = b.get();
-    if (pick) {
-        if (hipStreamWaitEvent(st, pick->done, 0) != hipSuccess) return nullptr;
-        pick->busy = true;
-        return pick;
-    }
-    if (S->scratch.size() >= kScratchBlocks) return nullptr;
+static std::unique_ptr<SpaceScratch> scratch_new(size_t bytes) {
     std::unique_ptr<SpaceScratch> b(new SpaceScratch());
     if (hipMalloc(&b->p, bytes) != hipSuccess ||
         hipEventCreateWithFlags(&b->done, hipEventDisableTiming) != hipSuccess) {
@@ -381,16 +368,68 @@ static SpaceScratch* scratch_take(const Space* S, size_t bytes, hipStream_t st) 
         return nullptr;  // ~SpaceScratch frees what there is
     }
     b->bytes = bytes;
-    b->busy = true;
-    S->scratch.push_back(std::move(b));
-    return S->scratch.back().get();
+    return b;
+}
+
+static SpaceScratch* scratch_take(const Space* S, size_t bytes, hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+        (void) hipGetLastError();
+        return nullptr;
+    }
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    std::unique_lock<std::mutex> lock(S->scratch_mu);
+    SpaceScratch *pick = nullptr, *oldest = nullptr;
+    for (;;) {
+        size_t low = S->scratch.size();  // a block too small
+        SpaceScratch* idle = nullptr;
+        pick = oldest = nullptr;
+        for (size_t i = 0; i < S->scratch.size(); i++) {
+            SpaceScratch* b = S->scratch[i].get();
+            if (b->busy) continue;
+            if (b->bytes < bytes) {
+                low = i;
+                continue;
+            }
+            if (b->last == st) pick = b;
+            else if (!idle && hipEventQuery(b->done) == hipSuccess) idle = b;
+            if (!oldest || b->turn < oldest->turn) oldest = b;
+        }
+        (void) hipGetLastError();  // hipErrorNotReady of the blocks in flight
+        if (!pick) pick = idle;
+        if (pick) break;
+        if (S->scratch.size() < kScratchBlocks) {
+            if (auto b = scratch_new(bytes)) {
+                S->scratch.push_back(std::move(b));
+                pick = S->scratch.back().get();
+                break;
+            }
+            if (!oldest) return nullptr;
+        }
+        if ((pick = oldest)) break;
+        if (low < S->scratch.size()) {
+            S->scratch.erase(S->scratch.begin() + low);
+            continue;
+        }
+        S->scratch_given.wait(lock);
+    }
+    // nothing to wait for where the last use is over or was on this stream
+    if (hipStreamWaitEvent(st, pick->done, 0) != hipSuccess) {
+        (void) hipGetLastError();
+        return nullptr;
+    }
+    pick->busy = true;
+    return pick;
 }
 
 static int scratch_give(const Space* S, SpaceScratch* b, hipStream_t st) {
     const hipError_t e = hipEventRecord(b->done, st);
+    if (e != hipSuccess) (void) hipStreamSynchronize(st);  // no event: idle from here on
     std::lock_guard<std::mutex> lock(S->scratch_mu);
     b->last = st;
+    b->turn = ++S->scratch_turn;
     b->busy = false;
+    S->scratch_given.notify_one();
     MCTDHB_HIP_CHECK(e);
     return kOk;
 }

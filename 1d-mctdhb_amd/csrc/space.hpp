@@ -1,6 +1,7 @@
 // space.hpp - the device-resident configurational space (tables + LUTs).
 #pragma once
 
+#include <condition_variable>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -19,7 +20,8 @@ struct SpaceScratch {
     size_t bytes = 0;
     hipEvent_t done = nullptr;
     hipStream_t last = nullptr;
-    bool busy = false;
+    uint64_t turn = 0;  // when it was given back
+    bool busy = false;  // between take and give of one call
     ~SpaceScratch() {
         if (done) hipEventDestroy(done);
         hipFree(p);  // waits for the device: no use is in flight after it
@@ -65,7 +67,9 @@ struct Space {
     mutable int hc_tiling = -1;
     // scratch of the two-stage product between calls (hamiltonian.hip)
     mutable std::vector<std::unique_ptr<SpaceScratch>> scratch;
+    mutable uint64_t scratch_turn = 0;
     mutable std::mutex scratch_mu;
+    mutable std::condition_variable scratch_given;
 };
 
 int space_dimension_exact(int npar, int norb, uint32_t* dim);

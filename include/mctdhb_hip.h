@@ -258,7 +258,13 @@ int mctdhb_space_tables(const mctdhb_space* space, const uint16_t** hash_table,
                         const uint32_t** maptt, const uint32_t** strideot, const uint32_t** stridett);
 
 /* hc = H coef.  hob: M x M row-major complex128; hint: M^4 complex128 with
- * hint[k + sM + qM^2 + lM^3].  coef/hc complex128 (FP64) or complex64 (MIXED). */
+ * hint[k + sM + qM^2 + lM^3].  coef/hc complex128 (FP64) or complex64 (MIXED).
+ * norb 6 and 7 take two stages over the space of N - 2 particles, with scratch
+ * of norb (norb + 1) / 2 values of C(N + norb - 3, norb - 1) configurations
+ * each: the space allocates it in the first such call and keeps it, up to four
+ * blocks where calls on several streams overlap.  Equal inputs give equal bits
+ * whatever else runs; only on a capturing stream, or when that memory cannot
+ * be had, do these calls run the one-stage kernels (equal to rounding). */
 int mctdhb_apply_hamiltonian_dev(const mctdhb_space* space, const void* coef, const void* hob,
                                  const void* hint, void* hc, int prec, int index, void* stream);
 

@@ -1,7 +1,9 @@
 """The two-stage H.C (M = 6, 7) where it can go wrong: N = 1 (no pairs: the
 one-stage kernel), N = 2 (one configuration of N - 2 particles), sizes around
 its 256-thread blocks, every call that takes it (product, prebuilt
-coefficients, products on two streams at once, under capture), and h and g
+coefficients), products on several streams and threads at once, which share
+the space's scratch and keep their form, the one-stage form of a capturing
+stream, and h and g
 without the usual symmetries, where it must read the same entries as the
 one-stage kernel.  The last Lanczos iteration's pair form of <w, H w> is
 covered for every orbital count.
@@ -107,6 +109,117 @@ def test_products_on_two_streams_do_not_share_scratch(amd, orc):
     torch.cuda.synchronize()
     for o, r in zip(outs, ref):
         assert np.array_equal(gu.host(o), r)
+    D.close()
+
+
+def _reference_bits(amd, npar, norb, cs, dh, dg, prec):
+    """Products one at a time on a space of their own, and one-stage ones,
+    whose bits differ."""
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    out = []
+    for c in cs:
+        a, b = gu.empty(D.dim, str(c.dtype)[6:]), gu.empty(D.dim, str(c.dtype)[6:])
+        D.apply_hamiltonian(c, dh, dg, a, prec=prec)
+        D.apply_hamiltonian_noalloc(c, dh, dg, b, prec=prec)
+        assert not np.array_equal(gu.host(a), gu.host(b))
+        out.append(gu.host(a))
+    D.close()
+    return out
+
+
+def test_form_does_not_depend_on_the_scratch_in_use(amd):
+    """Blocks of the mixed form, as many as a space keeps and all in flight,
+    do not keep FP64 products (larger blocks) off the two-stage form."""
+    import torch
+
+    npar, norb = 12, 6
+    h, g = inputs.onebody(norb, 3), inputs.twobody(norb, 3, 0.3)
+    dh, dg = gu.dev(h), gu.dev(g)
+    c = gu.dev(inputs.coefficients(math.comb(npar + norb - 1, norb - 1), 20))
+    c32 = c.to(torch.complex64)
+    ref, = _reference_bits(amd, npar, norb, [c], dh, dg, amd.FP64)
+    ref32, = _reference_bits(amd, npar, norb, [c32], dh, dg, amd.MIXED)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    st = [torch.cuda.Stream() for _ in range(6)]
+    small, full = [torch.zeros_like(c32) for _ in st], [torch.zeros_like(c) for _ in st]
+    torch.cuda.synchronize()
+    for prec, src, outs in ((amd.MIXED, c32, small), (amd.FP64, c, full), (amd.MIXED, c32, small)):
+        for s, o in zip(st, outs):
+            with torch.cuda.stream(s):
+                torch.cuda._sleep(50_000_000)  # some 20 ms: the block stays in flight
+            D.apply_hamiltonian(src, dh, dg, o, prec=prec, stream=s)
+    torch.cuda.synchronize()
+    for o in full:
+        assert np.array_equal(gu.host(o), ref)
+    for o in small:
+        assert np.array_equal(gu.host(o), ref32)
+    D.close()
+
+
+def test_form_does_not_depend_on_other_threads(amd):
+    import threading
+
+    import torch
+
+    npar, norb, threads, rounds = 9, 7, 8, 40
+    h, g = inputs.onebody(norb, 3), inputs.twobody(norb, 3, 0.3)
+    dh, dg = gu.dev(h), gu.dev(g)
+    dim = math.comb(npar + norb - 1, norb - 1)
+    cs = [gu.dev(inputs.coefficients(dim, 40 + i)) for i in range(threads)]
+    ref = _reference_bits(amd, npar, norb, cs, dh, dg, amd.FP64)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    st = [torch.cuda.Stream() for _ in range(threads)]
+    outs = [[torch.zeros_like(cs[0]) for _ in range(rounds)] for _ in range(threads)]
+    torch.cuda.synchronize()
+    go, failed = threading.Barrier(threads), []
+
+    def work(i):
+        try:
+            for r in range(rounds):
+                go.wait(60)
+                D.apply_hamiltonian(cs[i], dh, dg, outs[i][r], stream=st[i])
+        except Exception as e:  # noqa: BLE001
+            failed.append(e)
+            go.abort()
+
+    pool = [threading.Thread(target=work, args=(i,)) for i in range(threads)]
+    for t in pool:
+        t.start()
+    for t in pool:
+        t.join()
+    assert not failed
+    torch.cuda.synchronize()
+    for i in range(threads):
+        for o in outs[i]:
+            assert np.array_equal(gu.host(o), ref[i])
+    D.close()
+
+
+def test_captured_product_matches_oracle(amd, orc):
+    """A capturing stream takes the one-stage kernels: its graph keeps no
+    scratch of the space."""
+    import torch
+
+    npar, norb = 8, 6
+    c, h, g = _problem(npar, norb)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    dc, dh, dg, out, cf = gu.dev(c), gu.dev(h), gu.dev(g), gu.empty(D.dim), gu.empty(D.coef_bytes(amd.FP64) // 8, "float64")
+    D.hc_coefficients(dh, dg, cf)
+    D.apply_hamiltonian_cf(dc, cf, out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        D.apply_hamiltonian_cf(dc, cf, out, stream=torch.cuda.current_stream())
+    S = orc.Space(npar, norb)
+    for seed in (3, 4, 5):
+        dc.copy_(gu.dev(inputs.coefficients(D.dim, seed)))
+        eager = gu.empty(D.dim)
+        D.apply_hamiltonian_cf(dc, cf, eager)  # eager work between the replays
+        out.zero_()
+        graph.replay()
+        ref = S.apply_hamiltonian(inputs.coefficients(D.dim, seed), h, g)
+        assert gu.rel_err(gu.host(out), ref) < 1e-12 and gu.rel_err(gu.host(eager), ref) < 1e-12
+    del graph
     D.close()
 
 
