@@ -437,8 +437,8 @@ static int scratch_give(const Space* S, SpaceScratch* b, hipStream_t st) {
 // hc = H coef in two stages, X given or formed from hob and hint.  False
 // (nothing enqueued) when this space or stream takes the one-stage kernels.
 static bool two_stage(const Space* S, const void* coef, const double2* X, const double2* hob, const double2* hint,
-                      void* hc, int prec, int index, hipStream_t st, int& rc) {
-    if (!two_chosen(S, prec, index)) return false;
+                      void* hc, int prec, hipStream_t st, int& rc) {
+    if (!two_chosen(S, prec)) return false;
     SpaceScratch* b = scratch_take(S, two_matrix_bytes(S) + two_psi_bytes(S, prec), st);
     if (!b) return false;
     char* psi = (char*) b->p + two_matrix_bytes(S);
@@ -461,7 +461,7 @@ int hc_apply(const Space* S, const void* coef, const double2* hob, const double2
         return kOk;
     }
     if (prec == kPrecMixed && (rc = hc_tune_tiling(S, st))) return rc;
-    if (two_stage(S, coef, nullptr, hob, hint, hc, prec, index, st, rc)) return rc;
+    if (two_stage(S, coef, nullptr, hob, hint, hc, prec, st, rc)) return rc;
     const int M = S->norb;
     double2* cf64 = nullptr;
     float2* cf32 = nullptr;
@@ -606,7 +606,7 @@ int hc_apply_cf(const Space* S, const void* coef, const void* cf, void* hc, int 
     }
     if (prec == kPrecMixed && (rc = hc_tune_tiling(S, st))) return rc;
     const double2* X = S->d_low ? (const double2*) cf + cf_size(M) : nullptr;
-    if (X && two_stage(S, coef, X, nullptr, nullptr, hc, prec, index, st, rc)) return rc;
+    if (X && two_stage(S, coef, X, nullptr, nullptr, hc, prec, st, rc)) return rc;
     const void* blk = prec == kPrecFP64 ? cf : block_cf32(S, cf);
     return dispatch_fused_plain(S, coef, blk, hc, prec, index, st);
 }

@@ -188,12 +188,9 @@ inline size_t two_matrix_bytes(const Space* S) {
 // tables in LDS), and whether they are the faster form there.
 bool two_possible(const Space* S, int prec);
 bool two_faster(const Space* S, int prec);
-// Whether a caller of this index mode asked for the jump tables to be read
-// (the mixed form never does): the one-stage rows read them.
-inline bool wants_tables(int prec, int index) { return prec == kPrecFP64 && index == kIndexTables; }
-// The form of this space now (the mixed tiling may be set by hand).
-inline bool two_chosen(const Space* S, int prec, int index) {
-    return !wants_tables(prec, index) && two_faster(S, prec) && (prec == kPrecFP64 || S->hc_tiling == kTilingTwo);
+// ... and the form of this space now (the mixed tiling may be set by hand).
+inline bool two_chosen(const Space* S, int prec) {
+    return two_faster(S, prec) && (prec == kPrecFP64 || S->hc_tiling == kTilingTwo);
 }
 int two_matrix(const Space* S, const double2* hob, const double2* hint, double2* X, hipStream_t st);
 int two_apply(const Space* S, const void* c, const double2* X, void* psi, void* out, int prec, hipStream_t st);

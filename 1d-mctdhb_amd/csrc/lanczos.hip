@@ -395,11 +395,11 @@ int sil_create(const Space* S, int lm, int prec, int index, Sil** out) {
         return true;
     };
     if (!generic) ok = ok && hipMalloc((void**) &L->X, two_matrix_bytes(S)) == hipSuccess;
-    L->pairs = !generic && !wants_tables(prec, index) && two_possible(S, prec);
+    L->pairs = !generic && two_possible(S, prec);
     if (small_psi_needed(S, lm, prec))
         ok = ok && hipMalloc((void**) &L->psi_small, two_psi_bytes(S, prec)) == hipSuccess;
     // without room for the first stage's values the one-stage kernels run
-    if (ok && L->pairs && two_chosen(S, prec, index) && hipMalloc(&L->psi, two_psi_bytes(S, prec)) != hipSuccess) {
+    if (ok && L->pairs && two_chosen(S, prec) && hipMalloc(&L->psi, two_psi_bytes(S, prec)) != hipSuccess) {
         L->psi = nullptr;
         (void) hipGetLastError();
     }

@@ -21,8 +21,7 @@ struct Sil {
     void* wbase[kMaxKrylov] = {};
     void* w0f = nullptr;
     void* w0fbase = nullptr;
-    // Pair matrix (2 <= norb <= 7), whether the multi-kernel step may use the
-    // pair kernels (they cover the space and no tables were asked for),
+    // Pair matrix (2 <= norb <= 7), whether the pair kernels cover the space,
     // first-stage values of the two-stage H.C (null: one stage) and of the
     // one-workgroup step where they do not fit its LDS.
     double2* X = nullptr;

@@ -239,11 +239,7 @@ typedef struct mctdhb_sil   mctdhb_sil;   /* Krylov workspace of the SIL step */
 #define MCTDHB_FP64 0  /* complex128 throughout (the parity form) */
 #define MCTDHB_MIXED 1 /* complex64 coefficients and H.C, FP64 density sums and Lanczos scalars */
 
-/* Index schemes: where the jumps of H.C come from.  TABLES asks for a space
- * with tables in every call.  FP64 products and the steps of several kernels
- * read them; what has no jumps gives the same numbers under either scheme: the
- * density matrices of 2 <= norb <= 7 and the one-workgroup step.  MIXED always
- * takes FLY. */
+/* index schemes */
 #define MCTDHB_INDEX_TABLES 0 /* read the reference jump tables */
 #define MCTDHB_INDEX_FLY 1    /* closed-form rank deltas, no table traffic */
 

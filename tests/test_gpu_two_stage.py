@@ -112,38 +112,6 @@ def test_products_on_two_streams_do_not_share_scratch(amd, orc):
     D.close()
 
 
-@pytest.mark.parametrize("npar,norb", [(8, 6), (6, 7), (9, 5)])
-def test_table_indices_read_the_tables(amd, orc, npar, norb):
-    """FP64 with INDEX_TABLES: the one-stage rows over the tables in products
-    and in every iteration of a multi-kernel step, so the bits are not those of
-    the pair forms."""
-    c, h, g = _problem(npar, norb)
-    S = orc.Space(npar, norb)
-    D = amd.DeviceSpace(npar, norb, tables=True)
-    dc, dh, dg = gu.dev(c), gu.dev(h), gu.dev(g)
-    out, one = gu.empty(D.dim), gu.empty(D.dim)
-    D.apply_hamiltonian(dc, dh, dg, out, index=amd.INDEX_TABLES)
-    D.apply_hamiltonian_noalloc(dc, dh, dg, one, index=amd.INDEX_TABLES)
-    assert np.array_equal(gu.host(out), gu.host(one))
-    assert gu.rel_err(gu.host(out), S.apply_hamiltonian(c, h, g)) < 1e-12
-    cf = gu.empty(D.coef_bytes() // 8, "float64")
-    D.hc_coefficients(dh, dg, cf)
-    D.apply_hamiltonian_cf(dc, cf, out, index=amd.INDEX_TABLES)
-    assert np.array_equal(gu.host(out), gu.host(one))
-    _, ref = S.sil_step(c, h, g, 5, 0.01, False)
-    steps = []
-    for index in (amd.INDEX_TABLES, amd.INDEX_FLY):
-        sil = amd.DeviceSil(D, 5, index=index)
-        sil.set_small(False)
-        v = gu.dev(c)
-        sil.step(v, dh, dg, 0.01, False)
-        steps.append(gu.host(v))
-        assert gu.rel_err(steps[-1], ref) < 1e-10
-        sil.close()
-    assert not np.array_equal(*steps)
-    D.close()
-
-
 def _reference_bits(amd, npar, norb, cs, dh, dg, prec):
     """Products one at a time on a space of their own, and one-stage ones,
     whose bits differ."""
