@@ -473,7 +473,7 @@ int density_matrices(const Space* S, const void* coef, double2* rho1, double2* r
     const int M = S->norb;
     const bool generic = dm_generic(M);
     if (prec == kDmMixed && generic) {
-        set_error("mixed precision density matrices cover 2 <= norb <= 8");
+        set_error("mixed precision density matrices cover 2 <= norb <= 7");
         return kInvalidArgument;
     }
     if ((generic || index == kIdxTables) && !S->tables) {

@@ -239,7 +239,12 @@ typedef struct mctdhb_sil   mctdhb_sil;   /* Krylov workspace of the SIL step */
 #define MCTDHB_FP64 0  /* complex128 throughout (the parity form) */
 #define MCTDHB_MIXED 1 /* complex64 coefficients and H.C, FP64 density sums and Lanczos scalars */
 
-/* index schemes */
+/* Index schemes: where the kernels that go from jump to jump (the one-stage
+ * H.C) find their targets.  Both give the same bits.  TABLES asks for a space
+ * with tables in every call; what has no jumps ignores the scheme beyond that:
+ * the two-stage H.C (norb 6 and 7), the density matrices of 2 <= norb <= 7,
+ * the last iteration of a Lanczos recursion and the one-workgroup step.  MIXED
+ * always takes FLY. */
 #define MCTDHB_INDEX_TABLES 0 /* read the reference jump tables */
 #define MCTDHB_INDEX_FLY 1    /* closed-form rank deltas, no table traffic */
 
