@@ -126,14 +126,19 @@ unsigned hc_lanczos_blocks(const Space* S, int prec) {
 
 // ------------------------------------------------------- coefficient block
 
+// The coefficient block from hob (M x M row-major) and hint (M^4), with its
+// mixed copy cf32 (cf32_size(M) elements) and the pair matrix X where they are
+// not null.
 __global__ void k_hc_coefficients(int M, int N, const double2* __restrict__ hob, const double2* __restrict__ hint,
-                                  double2* __restrict__ cf64, float2* __restrict__ cf32) {
-    hc_coefficients_part(blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, M, N, hob, hint, cf64, cf32);
+                                  double2* __restrict__ cf64, float2* __restrict__ cf32, double2* __restrict__ X) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    hc_coefficients_part(t, stride, M, N, hob, hint, cf64, cf32);
+    if (X) pair_matrix_part(t, stride, M, N, hob, hint, X);
 }
 
-int hc_coefficients(const Space* S, const double2* hob, const double2* hint, double2* cf64, float2* cf32,
-                    hipStream_t st) {
-    k_hc_coefficients<<<div_up(cf_size(S->norb), 256), 256, 0, st>>>(S->norb, S->npar, hob, hint, cf64, cf32);
+static int hc_coefficients(const Space* S, const double2* hob, const double2* hint, double2* cf64, float2* cf32,
+                           double2* X, hipStream_t st) {
+    k_hc_coefficients<<<div_up(cf_size(S->norb), 256), 256, 0, st>>>(S->norb, S->npar, hob, hint, cf64, cf32, X);
     MCTDHB_HIP_CHECK(hipGetLastError());
     return kOk;
 }
@@ -467,7 +472,7 @@ int hc_apply(const Space* S, const void* coef, const double2* hob, const double2
     float2* cf32 = nullptr;
     MCTDHB_HIP_CHECK(hipMallocAsync((void**) &cf64, sizeof(double2) * cf_size(M), st));
     if (prec == kPrecMixed) MCTDHB_HIP_CHECK(hipMallocAsync((void**) &cf32, sizeof(float2) * cf32_size(M), st));
-    rc = hc_coefficients(S, hob, hint, cf64, cf32, st);
+    rc = hc_coefficients(S, hob, hint, cf64, cf32, nullptr, st);
     if (!rc) rc = dispatch_fused_plain(S, coef, prec == kPrecFP64 ? (const void*) cf64 : (const void*) cf32, hc,
                                        prec, index, st);
     hipFreeAsync(cf64, st);
@@ -475,13 +480,22 @@ int hc_apply(const Space* S, const void* coef, const double2* hob, const double2
     return rc;
 }
 
-// Prebuilt block: FP64 coefficients | pair matrix | (mixed) complex64 copy.
-// Where the first two stand does not depend on the precision, so a block
-// built for the mixed form serves FP64 products too.
+// Prebuilt block: FP64 coefficients | pair matrix, where the space may take two
+// stages | (mixed) complex64 copy.  Where the first two stand does not depend
+// on the precision, so a block built for the mixed form serves FP64 products
+// too.
+static bool block_pairs(const Space* S) { return two_faster(S, kPrecMixed); }
 static size_t block_cf32_off(const Space* S) {
-    return sizeof(double2) * cf_size(S->norb) + (S->d_low ? two_matrix_bytes(S) : 0);
+    return sizeof(double2) * cf_size(S->norb) + (block_pairs(S) ? two_matrix_bytes(S) : 0);
 }
 static const void* block_cf32(const Space* S, const void* cf) { return (const char*) cf + block_cf32_off(S); }
+// One launch; the one-stage kernels alone need no pair matrix.
+static int block_build(const Space* S, const double2* hob, const double2* hint, void* cf, int prec, bool one_stage,
+                       hipStream_t st) {
+    double2* X = one_stage || !block_pairs(S) ? nullptr : (double2*) cf + cf_size(S->norb);
+    return hc_coefficients(S, hob, hint, (double2*) cf, prec == kPrecMixed ? (float2*) block_cf32(S, cf) : nullptr, X,
+                           st);
+}
 
 // ------------------------------------------- H.C without device allocation
 // The coefficient block of hc_apply_noalloc lives in this array.  Host code
@@ -557,8 +571,8 @@ int hc_apply_noalloc(const Space* S, const void* coef, const double2* hob, const
     }
     void* blk = nullptr;
     if ((rc = scratch_address(&blk))) return rc;
-    // every entry of the block is written here, so nothing needs clearing
-    if ((rc = hc_build_coef(S, hob, hint, blk, prec, st))) return rc;
+    // every entry that is read is written here, so nothing needs clearing
+    if ((rc = block_build(S, hob, hint, blk, prec, true, st))) return rc;
     if (prec == kPrecFP64) return dispatch_fused_plain(S, coef, blk, hc, prec, index, st);
     const void* cf32 = block_cf32(S, blk);
     if (S->hc_tiling == 1 && S->d_pad) {  // staging already allocated: a device copy only
@@ -586,10 +600,7 @@ int hc_build_coef(const Space* S, const double2* hob, const double2* hint, void*
                                         hipMemcpyDeviceToDevice, st));
         return kOk;
     }
-    float2* cf32 = prec == kPrecMixed ? (float2*) block_cf32(S, cf) : nullptr;
-    const int rc = hc_coefficients(S, hob, hint, (double2*) cf, cf32, st);
-    if (rc || !S->d_low) return rc;
-    return two_matrix(S, hob, hint, (double2*) cf + cf_size(M), st);
+    return block_build(S, hob, hint, cf, prec, false, st);
 }
 
 int hc_apply_cf(const Space* S, const void* coef, const void* cf, void* hc, int prec, int index, hipStream_t st) {
@@ -605,7 +616,7 @@ int hc_apply_cf(const Space* S, const void* coef, const void* cf, void* hc, int 
         return kOk;
     }
     if (prec == kPrecMixed && (rc = hc_tune_tiling(S, st))) return rc;
-    const double2* X = S->d_low ? (const double2*) cf + cf_size(M) : nullptr;
+    const double2* X = block_pairs(S) ? (const double2*) cf + cf_size(M) : nullptr;
     if (X && two_stage(S, coef, X, nullptr, nullptr, hc, prec, st, rc)) return rc;
     const void* blk = prec == kPrecFP64 ? cf : block_cf32(S, cf);
     return dispatch_fused_plain(S, coef, blk, hc, prec, index, st);

@@ -58,12 +58,6 @@ __host__ __device__ constexpr int cf32_size(int M) { return cf_f64_off(M) + 2 * 
 
 constexpr int kFusedMaxOrb = 7;  // fused kernels instantiated for 2 <= M <= 7
 
-// Build the coefficient block from hob (M x M row-major) and hint (M^4),
-// both complex128 device arrays, into cf64 (and the mixed block cf32, of
-// cf32_size(M) complex64 elements, if non-null).
-int hc_coefficients(const Space* S, const double2* hob, const double2* hint, double2* cf64, float2* cf32,
-                    hipStream_t st);
-
 // hc = H coef.  prec / index select the kernel; coef/hc are complex128 for
 // FP64 and complex64 for mixed.  Uses the reference-order generic kernel for
 // M > 8 (tables required) and M == 1.

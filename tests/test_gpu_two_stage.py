@@ -112,6 +112,36 @@ def test_products_on_two_streams_do_not_share_scratch(amd, orc):
     D.close()
 
 
+@pytest.mark.parametrize("npar,norb", [(9, 2), (6, 5), (5, 6), (4, 7)])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_coefficient_blocks_take_one_launch(amd, npar, norb, prec):
+    """Kernels counted as the nodes of a captured graph: a block is built by
+    one, a product on the fixed scratch is two (block and rows)."""
+    import ctypes
+
+    import torch
+
+    c, h, g = _problem(npar, norb)
+    D = amd.DeviceSpace(npar, norb, tables=False)
+    src = gu.dev(c, np.complex128 if prec == amd.FP64 else np.complex64)
+    dh, dg, out = gu.dev(h), gu.dev(g), torch.zeros_like(src)
+    cf = gu.empty(D.coef_bytes(prec) // 8 + 1, "float64")
+
+    def kernels(call):
+        call(torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph):
+            call(torch.cuda.current_stream())
+        n = ctypes.c_size_t()
+        assert gu.hip().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+        return n.value
+
+    assert kernels(lambda st: D.hc_coefficients(dh, dg, cf, prec=prec, stream=st)) == 1
+    assert kernels(lambda st: D.apply_hamiltonian_noalloc(src, dh, dg, out, prec=prec, stream=st)) == 2
+    D.close()
+
+
 def _reference_bits(amd, npar, norb, cs, dh, dg, prec):
     """Products one at a time on a space of their own, and one-stage ones,
     whose bits differ."""
