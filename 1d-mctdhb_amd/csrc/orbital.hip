@@ -10,8 +10,8 @@
 //   lapack_interface.c:10-163, synchronize.c:41-56 (M x M eigen/regularise/invert)
 // The odelib Runge-Kutta the reference links is absent; the nonlinear step
 // uses the classical RK4 tableau.
+#include <algorithm>
 #include <cmath>
-#include <complex>
 #include <vector>
 
 #include "mxm_wave.hpp"
@@ -1892,40 +1892,82 @@ int density_sync_small(int norb, double2* rho1, double2* rinv, double* eigvals, 
 
 // ------------------------------------------------------------- set-up
 
-// The factors of k_cn_scan from the CN rows (upper | lower | mid), in long
-// double and rounded once: L | IU | CU | correction vector z of the cyclic
-// system, `grid` entries each; vm = beta / gamma, iv = 1 / (1 + v.z).
-static void cn_factor(const std::vector<double2>& cn, int grid, int bounds, std::vector<double2>& lu, double2& vm,
-                      double2& iv) {
-    using C = std::complex<long double>;
+// Complex long double, for the factors below (std::complex's division scales
+// and checks its operands, which costs ten times the rest).
+struct CnLong {
+    long double x, y;
+};
+static inline CnLong operator+(CnLong a, CnLong b) { return {a.x + b.x, a.y + b.y}; }
+static inline CnLong operator-(CnLong a, CnLong b) { return {a.x - b.x, a.y - b.y}; }
+static inline CnLong operator*(CnLong a, CnLong b) { return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
+static inline CnLong inverse(CnLong a) {
+    const long double s = 1 / (a.x * a.x + a.y * a.y);
+    return {a.x * s, -a.y * s};
+}
+
+// The factors of k_cn_scan from the CN rows cn (upper | lower | mid), in long
+// double and rounded once: lu = L | IU | CU | correction vector z of the cyclic
+// system, `grid` entries each, the unused ones zero; vm = beta / gamma, iv =
+// 1 / (1 + v.z).  Every workspace pays for it, also those that never take a
+// Crank-Nicolson step, hence one reciprocal per row, and none from the row on
+// that repeats the pivot before it: rows 1 .. m - 2 are alike, so the factors
+// stay what they are there (after about a hundred rows at usual steps).
+static void cn_factor(const double2* cn, int grid, int bounds, double2* lu, double2& vm, double2& iv) {
+    using C = CnLong;
     const bool cyc = bounds != kZeroBounds;
     const int m = cyc ? grid - 1 : grid;
-    auto get = [&](int part, int i) { return C(cn[(size_t) part * grid + i].x, cn[(size_t) part * grid + i].y); };
-    auto put = [&](int part, int i, C v) { lu[(size_t) part * grid + i] = make_double2((double) v.real(), (double) v.imag()); };
-    lu.assign(4 * (size_t) grid, make_double2(0, 0));
-    const C gam = -get(2, 0), beta = cyc ? get(0, m - 1) : C(0), alpha = cyc ? get(1, m - 1) : C(0);
-    std::vector<C> u(m), cu(m), z(m);
-    for (int i = 0; i < m; i++) {
+    auto get = [&](int part, int i) { return C{cn[part * grid + i].x, cn[part * grid + i].y}; };
+    auto put = [&](int part, int i, C v) { lu[part * grid + i] = make_double2((double) v.x, (double) v.y); };
+    const C zero{0, 0};
+    const C gam = zero - get(2, 0), inv_gam = inverse(gam);
+    const C beta = cyc ? get(0, m - 1) : zero, alpha = cyc ? get(1, m - 1) : zero;
+    struct Row {
+        C l, iu, c;
+    };
+    std::vector<Row> head;  // rows until they repeat; `tail` is row m - 1
+    head.reserve(256);
+    auto row = [&](int i, C above) {
         C b = get(2, i);
-        if (cyc && i == 0) b -= gam;
-        if (cyc && i == m - 1) b -= alpha * beta / gam;
-        const C l = i ? get(1, i - 1) / u[i - 1] : C(0);
-        u[i] = i ? b - l * get(0, i - 1) : b;
-        cu[i] = i < m - 1 ? get(0, i) / u[i] : C(0);
-        z[i] = (i == 0 ? gam : (i == m - 1 ? alpha : C(0))) - (i ? l * z[i - 1] : C(0));
-        put(0, i, l);
-        put(1, i, C(1) / u[i]);
-        put(2, i, cu[i]);
+        if (cyc && i == 0) b = b - gam;
+        if (cyc && i == m - 1) b = b - alpha * beta * inv_gam;
+        Row r{zero, zero, zero};
+        if (i) r.l = get(1, i - 1) * above;
+        r.iu = inverse(i ? b - r.l * get(0, i - 1) : b);
+        if (i < m - 1) r.c = get(0, i) * r.iu;
+        put(0, i, r.l);
+        put(1, i, r.iu);
+        put(2, i, r.c);
+        return r;
+    };
+    C iu = zero;
+    for (int i = 0; i < m - 1; i++) {
+        head.push_back(row(i, iu));
+        const bool repeats = i && head[i].iu.x == iu.x && head[i].iu.y == iu.y;
+        iu = head[i].iu;
+        if (!repeats) continue;
+        for (int part = 0; part < 3; part++) std::fill_n(lu + part * grid + i + 1, m - 2 - i, lu[part * grid + i]);
+        break;
     }
+    const Row tail = row(m - 1, iu);
     vm = iv = make_double2(0, 0);
     if (!cyc) return;
-    for (int i = m - 1; i >= 0; i--) {
-        z[i] = z[i] / u[i] - (i < m - 1 ? cu[i] * z[i + 1] : C(0));
+    const int known = (int) head.size() - 1;
+    auto at = [&](int i) -> const Row& { return i == m - 1 ? tail : head[std::min(i, known)]; };
+    std::vector<C> z(m);
+    C t = gam;
+    for (int i = 0; i < m; i++) {
+        const Row& r = at(i);
+        if (i) t = (i == m - 1 ? alpha : zero) - r.l * t;
+        z[i] = t * r.iu;
+    }
+    put(3, m - 1, z[m - 1]);
+    for (int i = m - 2; i >= 0; i--) {
+        z[i] = z[i] - at(i).c * z[i + 1];
         put(3, i, z[i]);
     }
-    const C v = beta / gam, inv = C(1) / (C(1) + z[0] + v * z[m - 1]);
-    vm = make_double2((double) v.real(), (double) v.imag());
-    iv = make_double2((double) inv.real(), (double) inv.imag());
+    const C v = beta * inv_gam, inv = inverse(C{1, 0} + z[0] + v * z[m - 1]);
+    vm = make_double2((double) v.x, (double) v.y);
+    iv = make_double2((double) inv.x, (double) inv.y);
 }
 
 int orbwork_create(const OrbEq& eq, int imagtime, const double* pot_host, OrbWork** out) {
@@ -1946,8 +1988,13 @@ int orbwork_create(const OrbEq& eq, int imagtime, const double* pot_host, OrbWor
         delete w;
         return kInvalidArgument;
     }
-    // FFT exponential (split_linear_orbitals.c:56-80) and twiddles on the host
-    std::vector<double2> fexp(n), tw(n);
+    // Everything that never changes is made on the host and kept in one
+    // allocation, filled by one copy: CN rows, their factors (7 grid), FFT
+    // exponential, twiddles, symbol (n each).
+    std::vector<double2> fixed(7 * (size_t) grid + 3 * (size_t) n, make_double2(0, 0));
+    double2 *cn = fixed.data(), *lu = cn + 3 * (size_t) grid, *fexp = lu + 4 * (size_t) grid, *tw = fexp + n,
+            *sym = tw + n;
+    // FFT exponential (split_linear_orbitals.c:56-80) and twiddles
     const double2 dt = make_double2(0.5 * eq.prop_dt.x, 0.5 * eq.prop_dt.y);
     for (int i = 0; i < n; i++) {
         const double freq = (i <= (n - 1) / 2) ? (2 * M_PI * i) / (n * eq.dx) : (2 * M_PI * (i - n)) / (n * eq.dx);
@@ -1962,9 +2009,10 @@ int orbwork_create(const OrbEq& eq, int imagtime, const double* pot_host, OrbWor
         const long long r = i % n;
         const double ang = 2 * M_PI * (double) r / (double) n;
         tw[i] = make_double2(cos(ang), -sin(ang));
+        // spectral symbol of the linear part: i freq d1 - freq^2 d2 (split_linear_orbitals.c:275-278)
+        sym[i] = make_double2(-freq * eq.d1coef.y - freq * freq * eq.d2coef, freq * eq.d1coef.x);
     }
     // CN tridiagonal (split_linear_orbitals.c:22-54)
-    std::vector<double2> cn(3 * (size_t) grid, make_double2(0, 0));
     {
         const double a2 = eq.d2coef, dx = eq.dx;
         const double2 a2dt = make_double2(dt.x * a2 / dx / dx, dt.y * a2 / dx / dx);
@@ -1984,10 +2032,13 @@ int orbwork_create(const OrbEq& eq, int imagtime, const double* pot_host, OrbWor
             cn[grid + grid - 2] = make_double2(minus_half.x - a1dt.x, minus_half.y - a1dt.y);
         }
     }
+    // the parallel CN solve needs a nonzero first diagonal (its cyclic split
+    // divides by it; the reference's reduced system for mid[0] == 0 stays on
+    // the sequential sweep)
+    const bool factored = cn[2 * grid].x != 0 || cn[2 * grid].y != 0;
+    if (factored) cn_factor(cn, grid, eq.bounds, lu, w->cn_vm, w->cn_iv);
     bool ok = hipMalloc((void**) &w->d_pot, sizeof(double) * grid) == hipSuccess;
-    ok = ok && hipMalloc((void**) &w->d_fexp, sizeof(double2) * n) == hipSuccess;
-    ok = ok && hipMalloc((void**) &w->d_tw, sizeof(double2) * n) == hipSuccess;
-    ok = ok && hipMalloc((void**) &w->d_cn, sizeof(double2) * 3 * grid) == hipSuccess;
+    ok = ok && hipMalloc((void**) &w->d_cn, sizeof(double2) * fixed.size()) == hipSuccess;
     ok = ok && hipMalloc((void**) &w->d_stage, sizeof(double2) * 7 * (size_t) M * grid) == hipSuccess;
     ok = ok && hipMalloc((void**) &w->d_red, sizeof(double) * 1024) == hipSuccess;
     ok = ok && hipMalloc((void**) &w->d_cnwork, sizeof(double2) * 10 * (size_t) M * grid) == hipSuccess;
@@ -1995,38 +2046,16 @@ int orbwork_create(const OrbEq& eq, int imagtime, const double* pot_host, OrbWor
                    hipSuccess;
     ok = ok && hipMalloc((void**) &w->d_fsH, sizeof(double2) * (size_t) M * grid) == hipSuccess;
     ok = ok && hipMalloc((void**) &w->d_fsmat, sizeof(double2) * 3 * M * M) == hipSuccess;
-    ok = ok && hipMalloc((void**) &w->d_hsym, sizeof(double2) * n) == hipSuccess;
     if (!ok) {
         orbwork_destroy(w);
         set_error("device allocation failed for the orbital workspace");
         return kOutOfMemory;
     }
-    MCTDHB_HIP_CHECK(hipMemcpy(w->d_fexp, fexp.data(), sizeof(double2) * n, hipMemcpyHostToDevice));
-    MCTDHB_HIP_CHECK(hipMemcpy(w->d_tw, tw.data(), sizeof(double2) * n, hipMemcpyHostToDevice));
-    MCTDHB_HIP_CHECK(hipMemcpy(w->d_cn, cn.data(), sizeof(double2) * 3 * grid, hipMemcpyHostToDevice));
-    // the parallel CN solve needs a nonzero first diagonal (its cyclic split
-    // divides by it; the reference's reduced system for mid[0] == 0 stays on
-    // the sequential sweep)
-    {
-        const double2 m0 = cn[2 * (size_t) grid];
-        if ((m0.x != 0 || m0.y != 0) && grid >= 4) {
-            std::vector<double2> lu;
-            cn_factor(cn, grid, eq.bounds, lu, w->cn_vm, w->cn_iv);
-            if (hipMalloc((void**) &w->d_cnlu, sizeof(double2) * lu.size()) != hipSuccess) {
-                orbwork_destroy(w);
-                set_error("device allocation failed for the orbital workspace");
-                return kOutOfMemory;
-            }
-            MCTDHB_HIP_CHECK(hipMemcpy(w->d_cnlu, lu.data(), sizeof(double2) * lu.size(), hipMemcpyHostToDevice));
-        }
-    }
-    // spectral symbol of the linear part: i freq d1 - freq^2 d2 (split_linear_orbitals.c:275-278)
-    std::vector<double2> sym(n);
-    for (int i = 0; i < n; i++) {
-        const double freq = (i <= (n - 1) / 2) ? (2 * M_PI * i) / (n * eq.dx) : (2 * M_PI * (i - n)) / (n * eq.dx);
-        sym[i] = make_double2(-freq * eq.d1coef.y - freq * freq * eq.d2coef, freq * eq.d1coef.x);
-    }
-    MCTDHB_HIP_CHECK(hipMemcpy(w->d_hsym, sym.data(), sizeof(double2) * n, hipMemcpyHostToDevice));
+    if (factored) w->d_cnlu = w->d_cn + (lu - cn);
+    w->d_fexp = w->d_cn + (fexp - cn);
+    w->d_tw = w->d_cn + (tw - cn);
+    w->d_hsym = w->d_cn + (sym - cn);
+    MCTDHB_HIP_CHECK(hipMemcpy(w->d_cn, cn, sizeof(double2) * fixed.size(), hipMemcpyHostToDevice));
     int rc = orbwork_set_potential(w, pot_host);
     if (rc) {
         orbwork_destroy(w);
@@ -2044,17 +2073,13 @@ int orbwork_set_potential(OrbWork* w, const double* pot_host) {
 void orbwork_destroy(OrbWork* w) {
     if (!w) return;
     hipFree(w->d_pot);
-    hipFree(w->d_fexp);
-    hipFree(w->d_tw);
     hipFree(w->d_cn);
     hipFree(w->d_stage);
     hipFree(w->d_red);
     hipFree(w->d_cnwork);
-    hipFree(w->d_cnlu);
     hipFree(w->d_nl);
     hipFree(w->d_fsH);
     hipFree(w->d_fsmat);
-    hipFree(w->d_hsym);
     hipFree(w->d_dvrT);
     delete w;
 }

@@ -26,18 +26,18 @@ struct OrbWork {
     int dvr = 0;       // full-equation RK: linear part by the exponential DVR
     int nfft = 0, log2n = -1;  // FFT length grid_size - 1 (log2n < 0: not a power of two)
     double* d_pot = nullptr;     // grid_size
+    double2* d_cn = nullptr;     // 3 * grid_size: upper | lower | mid; the allocation holds the next four too
+    double2* d_cnlu = nullptr;   // 4 * grid_size: factors of the parallel CN solve (null: sequential)
     double2* d_fexp = nullptr;   // nfft: exp(-i dt/2 (i a1 k - a2 k^2))
-    double2* d_tw = nullptr;     // nfft / 2 twiddles exp(-2 pi i t / nfft)
-    double2* d_cn = nullptr;     // 3 * grid_size: upper | lower | mid
+    double2* d_tw = nullptr;     // nfft twiddles exp(-2 pi i t / nfft)
+    double2* d_hsym = nullptr;   // nfft: spectral symbol of the linear part
     double2* d_stage = nullptr;  // 7 * norb * grid_size: up to six stages and y
     double* d_red = nullptr;     // reduction scratch
     double2* d_cnwork = nullptr; // 10 * norb * grid_size: Crank-Nicolson solve scratch
-    double2* d_cnlu = nullptr;   // 4 * grid_size: factors of the parallel CN solve (null: sequential)
     double2 cn_vm{0, 0}, cn_iv{0, 0};  // its cyclic correction
     double2* d_nl = nullptr;     // grid-independent factors of the nonlinear term
     double2* d_fsH = nullptr;    // norb * grid_size: H y of the full-equation step
     double2* d_fsmat = nullptr;  // 3 norb^2: projections, Gram matrix, projector coefficients
-    double2* d_hsym = nullptr;   // nfft: spectral symbol of the linear part
     double2* d_dvrT = nullptr;   // nfft^2: exponential-DVR matrix, transposed (built on first use)
 };
 
