@@ -3,4 +3,5 @@
 
 namespace mctdhb {
 template struct HcTwo<6>;
+template struct HcTwoRows<6>;
 }  // namespace mctdhb

@@ -3,4 +3,5 @@
 
 namespace mctdhb {
 template struct HcTwo<7>;
+template struct HcTwoRows<7>;
 }  // namespace mctdhb

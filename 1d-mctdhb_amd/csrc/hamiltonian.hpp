@@ -137,7 +137,14 @@ const float2* hc_padded_copy(const Space* S, const float2* c, hipStream_t st);
 
 // The whole FP64 SIL step in one workgroup (sil_small.hpp): w[0] is C
 // (updated in place), w[1..lm-1] Krylov storage.  Its size limits: with the W
-// table and the roots bounded, the vector H acts on always fits the LDS.
+// table and the roots bounded, the vector H acts on always fits the LDS.  They
+// say what the kernel holds, and packs take all of it.  Alone on the card a
+// step is faster there only up to NC of about 1000 at every orbital count (5
+// vectors, one workgroup and several kernels, us: M = 3 NC 861 60 and 86, 1891
+// 102 and 87; M = 4 969 95 and 97, 7770 492 and 97; M = 5 495 72 and 109, 1001
+// 124 and 113, 7315 723 and 116; M = 6 792 111 and 128, 2002 278 and 130;
+// M = 7 924 165 and 169, 3003 528 and 174); callers choose with
+// mctdhb_sil_set_small.
 constexpr uint32_t kSmallSilMaxDim = 8192;
 constexpr size_t kSmallTableBytes = 48896;
 constexpr int kSmallMaxBlock = 1024;
@@ -226,9 +233,13 @@ inline SmallSilCtx small_ctx(const Space* S, const double2* X, double2* psi) {
 int two_small(const Space* S, const double2* X, double2* psi, const SmallSilArgs& a, hipStream_t st);
 struct PkSil;
 
-template <int M> struct HcTwo {
+// The two-stage product, for the orbital counts that take it (two_faster).
+template <int M> struct HcTwoRows {
     static int plain(const Space* S, const void* c, const double2* X, void* psi, void* out, int prec, hipStream_t st);
     static int lanczos(const Space* S, const double2* X, void* psi, const LanczosHcArgs& a, int prec, hipStream_t st);
+};
+// The pair forms of every orbital count.
+template <int M> struct HcTwo {
     static int rayleigh(const Space* S, const double2* X, const LanczosHcArgs& a, int prec, hipStream_t st);
     // the one-workgroup SIL step (sil_small.hpp), of one solve and of count solves (pack.hpp)
     static int small(const Space* S, const double2* X, double2* psi, const SmallSilArgs& a, hipStream_t st);

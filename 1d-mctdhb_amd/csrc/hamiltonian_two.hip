@@ -12,6 +12,8 @@ extern template struct HcTwo<4>;
 extern template struct HcTwo<5>;
 extern template struct HcTwo<6>;
 extern template struct HcTwo<7>;
+extern template struct HcTwoRows<6>;
+extern template struct HcTwoRows<7>;
 
 __global__ void k_pair_matrix(int M, int N, const double2* __restrict__ hob, const double2* __restrict__ hint,
                               double2* __restrict__ X) {
@@ -46,11 +48,31 @@ bool two_possible(const Space* S, int prec) {
 // particles replace 256 (M = 6) and 504 (M = 7) gathers and products per
 // configuration: FP64 product at N=37, M=6 147 -> 116 us; mixed Lanczos
 // iteration at N=30, M=7 485 -> 279 us, SIL step 3.93 -> 2.21 ms; N=18, M=6
-// (NC 33,649) whole step 290 -> 263 us.  At M = 5 the 15 arrays of psi go to
+// (NC 33,649) whole step 290 -> 263 us.  No lower bound on NC: a product of the
+// smallest spaces takes no longer in two launches than one-stage rows do with
+// a prebuilt block (mixed, M = 6: NC 21 12.7 and 12.5 us, NC 252 12.3 and 12.0;
+// M = 7: NC 28 19.7 and 26.1; FP64 is faster at every size).  At M = 5 the 15 arrays of psi go to
 // memory and back (1 GB complex64 at N=100), which costs more than the 131
 // gathers they replace: SIL step 1.93 -> 2.23 ms mixed, 2.82 -> 3.68 ms FP64;
 // at N=200, M=4 0.67 -> 0.76 ms.
 bool two_faster(const Space* S, int prec) { return S->norb >= 6 && two_possible(S, prec); }
+
+#define ROWS(call)                                                                                          \
+    switch (S->norb) {                                                                                      \
+        case 6: return HcTwoRows<6>::call;                                                                   \
+        case 7: return HcTwoRows<7>::call;                                                                   \
+        default: set_error("the two-stage H.C covers norb 6 and 7"); return kInvalidArgument;                \
+    }
+
+int two_apply(const Space* S, const void* c, const double2* X, void* psi, void* out, int prec, hipStream_t st) {
+    ROWS(plain(S, c, X, psi, out, prec, st))
+}
+
+int two_lanczos(const Space* S, const double2* X, void* psi, const LanczosHcArgs& a, int prec, hipStream_t st) {
+    ROWS(lanczos(S, X, psi, a, prec, st))
+}
+
+#undef ROWS
 
 #define DISPATCH(call)                                                                                      \
     switch (S->norb) {                                                                                      \
@@ -60,16 +82,8 @@ bool two_faster(const Space* S, int prec) { return S->norb >= 6 && two_possible(
         case 5: return HcTwo<5>::call;                                                                       \
         case 6: return HcTwo<6>::call;                                                                       \
         case 7: return HcTwo<7>::call;                                                                       \
-        default: set_error("two-stage H.C kernels cover 2 <= norb <= 7"); return kInvalidArgument;           \
+        default: set_error("the pair forms of H.C cover 2 <= norb <= 7"); return kInvalidArgument;           \
     }
-
-int two_apply(const Space* S, const void* c, const double2* X, void* psi, void* out, int prec, hipStream_t st) {
-    DISPATCH(plain(S, c, X, psi, out, prec, st))
-}
-
-int two_lanczos(const Space* S, const double2* X, void* psi, const LanczosHcArgs& a, int prec, hipStream_t st) {
-    DISPATCH(lanczos(S, X, psi, a, prec, st))
-}
 
 int two_rayleigh(const Space* S, const double2* X, const LanczosHcArgs& a, int prec, hipStream_t st) {
     DISPATCH(rayleigh(S, X, a, prec, st))

@@ -240,7 +240,7 @@ static int two_collect(const Space* S, const Z* c, const Z* psi, int stop_check,
 }
 
 template <int M>
-int HcTwo<M>::plain(const Space* S, const void* c, const double2* X, void* psi, void* out, int prec, hipStream_t st) {
+int HcTwoRows<M>::plain(const Space* S, const void* c, const double2* X, void* psi, void* out, int prec, hipStream_t st) {
     int rc;
     if (prec == kPrecFP64) {
         if ((rc = two_product<M>(S, (const double2*) c, X, (double2*) psi, 0, nullptr, st))) return rc;
@@ -266,7 +266,7 @@ int HcTwo<M>::rayleigh(const Space* S, const double2* X, const LanczosHcArgs& a,
 }
 
 template <int M>
-int HcTwo<M>::lanczos(const Space* S, const double2* X, void* psi, const LanczosHcArgs& a, int prec, hipStream_t st) {
+int HcTwoRows<M>::lanczos(const Space* S, const double2* X, void* psi, const LanczosHcArgs& a, int prec, hipStream_t st) {
     int rc;
     if (prec == kPrecFP64) {
         const double2* w = (const double2*) a.w[a.it];
