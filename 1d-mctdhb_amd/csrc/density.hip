@@ -369,10 +369,12 @@ static bool dm_generic(int M) { return M == 1 || M > 7; }
 
 // Runs of configurations go to waves.  Up to 1024 configurations of N - 2
 // particles one block of 8 waves does it all and the separate finish (a
-// launch) is saved; then 64 per wave, so a middling space still reaches many
-// CUs; from 256 blocks on, one per CU (the LDS buffers of M >= 4 hold a CU
-// each), the runs get longer: 512 blocks took 0.169 ms against 0.161 at N=100,
-// M=5 and 0.187 against 0.176 at N=30, M=7.
+// launch) is saved (1001 at M = 5: 13.2 us, two blocks 15.3; 1225 at M = 3:
+// 13.8 in one block, 10.3 in several; at M = 6 several win earlier, 792: 29.0
+// and 26.8).  Then 64 per wave, so a middling space still reaches many CUs.
+// From 256 blocks on, one per CU (the LDS buffers of M >= 4 hold a CU each),
+// the runs get longer: 128, 256 and 512 blocks take 272, 149 and 155 us at
+// N=100, M=5, 282, 153 and 165 us at N=30, M=7 (complex64).
 DmPlan dm_plan(const Space* S) {
     if (dm_generic(S->norb)) return {div_up(S->dim, kDmTile)};
     return {S->low_dim <= 1024 ? 1u : std::min(256u, div_up(S->low_dim, 64 * kDmWaves))};

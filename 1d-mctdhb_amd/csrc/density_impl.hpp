@@ -12,7 +12,7 @@
 // product per jump (about 80 per configuration at M = 5, one sum per element
 // on the vector ALU); here it is P = 15 gathers, and the sums are matrix
 // work.  Measured on MI355X, whole call: N=100, M=5 in FP64 0.495 ms before,
-// 0.149 ms now; N=30, M=7 from complex64 coefficients 1.81 ms before, 0.155 ms
+// 0.149 ms now; N=30, M=7 from complex64 coefficients 1.81 ms before, 0.153 ms
 // now.  What bounds it is the FP64 unit, which matrix and vector instructions
 // share (run together they add up, they do not overlap): 3 products of
 // 16 x 16 x 4 per four configurations (10 at M >= 6) are 0.083 and 0.087 ms at

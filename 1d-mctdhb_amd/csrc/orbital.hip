@@ -417,7 +417,10 @@ int linear_cn(OrbWork* w, double2* orb, hipStream_t st) {
     const double2 up = cscale(a2dt, 0.5) + a1dt, lo = cscale(a2dt, 0.5) - a1dt;
     const double2 mid = make_double2(-a2dt.x, 1.0 - a2dt.y);
     if (w->d_cnlu) {
-        // up to four rows per thread
+        // the fewest waves at up to four rows per thread (M = 5, us: 257 points
+        // 4.6 at 256 threads, 6.3 at 512; 1025 points 7.0 at 256, 7.1 at 512,
+        // 10.2 at 1024; 2049 points 15.5 at 256 (8 rows), 10.5 at 512, 11.5 at
+        // 1024; 4097 points 27.6 at 512 (8 rows), 17.9 at 1024)
         const int m = q.bounds != kZeroBounds ? q.grid_size - 1 : q.grid_size;
         const int t = m <= 1024 ? 256 : (m <= 2048 ? 512 : 1024);
 #define SCAN(per) \
@@ -1106,8 +1109,12 @@ static int rk_tableau(OrbWork* w, int ns, const double* A, const double* b, doub
 // one sum per pair (i, j) over orbitals in LDS took 16.0 us at M = 4 on 257
 // points and 36.7 us at M = 5 on 801, this form 7.1 and 11.4 us.
 constexpr int kGsMaxOrb = 8;
-// Threads and points per thread for n grid points: at most 3 points, except
-// on the longest grids.
+// Threads and points per thread for n grid points: as few waves as hold them
+// at up to 3 points a thread (from 3073 points on 5, the widest block has no
+// more threads).  M = 5, us: 513 points 9.6 at 256 threads, 10.4 at 512; 1025
+// points 18.7 at 256 (5 points), 11.9 at 512, 16.1 at 1024; 2049 points 28.8 at
+// 512 (5 points), 18.0 at 1024.  Two and eight orbitals order them alike but
+// for M = 8 at 513 points (29.1 at 256, 22.1 at 512).
 struct GsShape {
     int threads, per;
 };
@@ -1115,7 +1122,7 @@ __host__ __device__ inline GsShape gs_shape(int n) {
     const int t = n <= 768 ? 256 : (n <= 1536 ? 512 : 1024);
     return {t, n <= t ? 1 : (n <= 2 * t ? 2 : (n <= 3 * t ? 3 : 5))};
 }
-inline bool gs_in_registers(int M, int n) { return M <= kGsMaxOrb && n <= 5 * 1024; }
+inline bool gs_in_registers(int M) { return M <= kGsMaxOrb; }  // workspaces have at most 4097 points
 
 // Inclusive product over the lanes of the wave (fixed order).
 __device__ __forceinline__ double wave_prefix_product(double v) {
@@ -1252,7 +1259,7 @@ int pk_gram_schmidt(const PkGs* tab, int count, int M, int threads, hipStream_t 
 }
 int pk_gs_threads(int n) { return gs_shape(n).threads; }
 
-// More orbitals (or a longer grid): one block, the orbitals in LDS where they
+// More orbitals: one block, the orbitals in LDS where they
 // fit, j-major with one block sum per pair.  Thread t owns the points
 // [t per, (t + 1) per): it alone reads and writes them, so the only barriers
 // are those of the block sums (double-buffered, one each).
@@ -1359,7 +1366,7 @@ __global__ __launch_bounds__(256) void k_gram_schmidt_many(double2* __restrict__
 
 int orthonormalize(OrbWork* w, double2* orb, hipStream_t st, bool periodic_tail) {
     const int M = w->eq.norb, n = w->eq.grid_size, tail = periodic_tail ? 1 : 0;
-    if (gs_in_registers(M, n)) {
+    if (gs_in_registers(M)) {
         switch (M) {
 #define CASE(m)                                                                                \
     case m:                                                                                    \

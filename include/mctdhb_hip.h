@@ -329,7 +329,9 @@ int mctdhb_sil_create(const mctdhb_space* space, int lanczos_iter, int prec, int
 int mctdhb_sil_destroy(mctdhb_sil* sil);
 /* FP64 steps of spaces up to 8192 configurations, 2 <= norb <= 7 and at most
  * 15 Krylov vectors run as one workgroup (the whole recursion in one
- * kernel); on = 0 keeps them on the multi-kernel path.  Default on. */
+ * kernel); on = 0 keeps them on the multi-kernel path.  Default on.  Alone on
+ * the card, spaces of more than about 1000 configurations step faster with it
+ * off (7315 configurations, norb 5, 5 vectors: 723 and 116 us); packs need it. */
 int mctdhb_sil_set_small(mctdhb_sil* sil, int on);
 size_t mctdhb_sil_device_bytes(const mctdhb_space* space, int lanczos_iter, int prec);
 /* coef (complex128, device) <- exp(-i H prop_dt) coef; renormalised when

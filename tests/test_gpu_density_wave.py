@@ -1,11 +1,11 @@
-"""The density kernels of large spaces, against the FP64 oracle (reference
-density_matrices.c:9-443) for every orbital count of the fused forms, each
-shape above 65536 configurations: the element-family passes (one family per
-block) for M <= 5 and the one-pass wave-sum kernel for M >= 6.  FP64 with
-on-the-fly and table indices within 1e-10 relative, complex64 products
-within 2e-6, and the trace identities tr rho1 = N and
-sum_s rho2[k,s,s,l] = (N - 1) rho1[k,l]; the wave form is also deterministic
-from call to call."""
+"""The density matrices of large spaces, against the FP64 oracle (reference
+density_matrices.c:9-443) for every orbital count from three on, each shape
+above 65536 configurations: many blocks and the grid-wide finish.  FP64 within
+1e-10 relative, from complex64 coefficients within 2e-6, and the trace
+identities tr rho1 = N and sum_s rho2[k,s,s,l] = (N - 1) rho1[k,l]; the sums are
+also the same from call to call.  The pair sums have no jumps, so table and
+on-the-fly indices name the same kernels: with tables it is the call that is
+covered."""
 import math
 
 import numpy as np
